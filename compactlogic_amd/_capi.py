@@ -120,6 +120,7 @@ SIGNATURES: dict[str, list] = {
     "cl_group_sum_cross_entropy_forward_noalloc": [_int, _p, _i64, _i64, _i64, _i64, _i64, _f64,
                                                    _p, _i64, _p, _p, _p, _p, _p],
     "cl_pack_bits": [_p, _i64, _i64, _i32, _p, ctypes.POINTER(_i64), _p],
+    "cl_pack_bits_batch": [_p, _i64, _i64, _i32, _p, ctypes.POINTER(_i64), _p],
     "cl_dense_eval_packed": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p],
     "cl_group_bit_sum": [_p, _i64, _i64, _i64, _i64, _p, _p],
     "cl_fill_splitmix64": [_p, _i64, _u64, _p],

@@ -149,34 +149,6 @@ __global__ __launch_bounds__(kNetThreads) void k_packed_net(const uint32_t* __re
 // range of columns, loading the next column's input words while it evaluates the current one.
 constexpr int kSlotCap = 72;  // gate slots per thread (registers)
 
-// Exchange with lane l ^ K inside each 32-lane half of the wave.
-template <int K>
-__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
-    if constexpr (K == 1) return dpp_move<0xB1>(v);         // quad_perm [1,0,3,2]
-    else if constexpr (K == 2) return dpp_move<0x4E>(v);    // quad_perm [2,3,0,1]
-    else if constexpr (K == 8) return dpp_move<0x128>(v);   // row_ror:8
-    else return uint32_t(__builtin_amdgcn_ds_swizzle(int(v), (K << 10) | 0x1F));  // xor mode
-}
-
-// One stage of the 32 x 32 bit transpose across a half-wave (row = lane, column = bit): lanes
-// l and l ^ K swap the off-diagonal K x K blocks of every 2K x 2K block.  The lane with bit K
-// clear keeps its columns c with c & K == 0 and takes the partner's same columns shifted up by
-// K; the other keeps c & K != 0 and takes the partner's shifted down.  A rotation by K or
-// 32 - K moves the wanted bits into place for either lane (the bits it wraps round are masked).
-template <int K>
-__device__ __forceinline__ uint32_t transpose_stage(uint32_t t, int lane) {
-    constexpr uint32_t m = K == 16 ? 0x0000FFFFu
-                           : K == 8 ? 0x00FF00FFu
-                           : K == 4 ? 0x0F0F0F0Fu
-                           : K == 2 ? 0x33333333u
-                                    : 0x55555555u;  // columns c with c & K == 0
-    const bool low = (lane & K) == 0;
-    const uint32_t p = xor_lane<K>(t);
-    const uint32_t sh = __builtin_amdgcn_alignbit(p, p, low ? 32 - K : K);  // rotate right
-    const uint32_t keep = low ? m : ~m;
-    return (t & keep) | (sh & ~keep);
-}
-
 // Adds the 1-bit numbers of x into the bit planes a[I..B) (a ripple of half adders).
 template <int I, int B>
 __device__ __forceinline__ void add_planes(uint32_t (&a)[B], uint32_t x) {

@@ -185,22 +185,36 @@ def eval(x, a, b, w, gate_seq):  # noqa: A001 - mirrors difflogic_cuda.eval
 _PACK_DTYPES = {8: torch.int8, 16: torch.int16, 32: torch.int32, 64: torch.int64}
 
 
-def tensor_packbits_cuda(t, bit_count):
-    """bool [rows, n] -> (packed [rows, ceil(n / bit_count)], pad_len)
-    (compactlogic/cuda/difflogic_kernel.cu:453-494)."""
-    _check(t, "t")
+def _packbits(entry, t, rows, n, bit_count):
     if t.dtype != torch.bool:
         raise RuntimeError("t must be a bool tensor")
     if bit_count not in _PACK_DTYPES:
         raise ValueError("`bit_count` has to be in { 8, 16, 32, 64 }")
-    rows, n = t.shape
     words = -(-n // bit_count)
     packed = torch.empty((rows, words), dtype=_PACK_DTYPES[bit_count], device=t.device)
     pad = ctypes.c_int64(0)
     with torch.cuda.device(t.device):
-        _capi.call("cl_pack_bits", ptr(t), rows, n, bit_count, ptr(packed), ctypes.byref(pad),
+        _capi.call(entry, ptr(t), *t.shape, bit_count, ptr(packed), ctypes.byref(pad),
                    stream_of(t))
     return packed, int(pad.value)
+
+
+def tensor_packbits_cuda(t, bit_count):
+    """bool [rows, n] -> (packed [rows, ceil(n / bit_count)], pad_len)
+    (compactlogic/cuda/difflogic_kernel.cu:453-494)."""
+    _check(t, "t")
+    rows, n = t.shape
+    return _packbits("cl_pack_bits", t, rows, n, bit_count)
+
+
+def packbits_batch(t, bit_count):
+    """tensor_packbits_cuda(t.T.contiguous(), bit_count) of a bool batch t [n, features],
+    reading the batch as it lies (a contiguous batch is not transposed first)."""
+    if t.t().is_contiguous() or not t.is_contiguous():
+        return tensor_packbits_cuda(t.t().contiguous(), bit_count)
+    _check(t, "t")
+    n, features = t.shape
+    return _packbits("cl_pack_bits_batch", t, features, n, bit_count)
 
 
 def groupbitsum(b, pad_len, k):

@@ -37,8 +37,7 @@ class PackBitsTensor:
         if t.device.type != "cuda":
             raise NotImplementedError(
                 f"PackBitsTensor only supports device tensors, but got {t.device}.")
-        t = t.T.contiguous()
-        self.t, self.pad_len = _dl.tensor_packbits_cuda(t, self.bit_count)
+        self.t, self.pad_len = _dl.packbits_batch(t, self.bit_count)
 
     @classmethod
     def from_packed(cls, words: torch.Tensor, pad_len: int = 0, bit_count: int | None = None):

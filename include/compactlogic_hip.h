@@ -519,6 +519,12 @@ int cl_transpose(int dtype, const void* src, void* dst, int64_t rows, int64_t co
 int cl_pack_bits(const uint8_t* t, int64_t rows, int64_t n, int32_t bit_count, void* packed,
                  int64_t* pad_len, void* stream);
 
+/* cl_pack_bits of the transposed batch without transposing it: t is [n, features] (a sample's
+ * features contiguous), packed [features, ceil(n / bit_count)].  What PackBitsTensor does with a
+ * batch (third_party/convlogic_source_code/src/difflogic/packbitstensor.py:11-21) in one pass. */
+int cl_pack_bits_batch(const uint8_t* t, int64_t n, int64_t features, int32_t bit_count,
+                       void* packed, int64_t* pad_len, void* stream);
+
 /* Integer difflogic_cuda.eval on packed words
  * (third_party/convlogic_source_code/src/difflogic/cuda/difflogic_kernel.cu:271-330) with
  * compactlogic's slot semantics (compactlogic/compactlogic.py:120-130):

@@ -114,3 +114,25 @@ def test_cfg4_network_slice_bit_exact(device):
     assert np.array_equal(xw.cpu().numpy().view(np.uint64), ref_x)
     ref = P.network_counts(ref_x, layers, cfg.k)
     assert np.array_equal(counts.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("bits", [8, 16, 32, 64])
+@pytest.mark.parametrize("n,feats,skew", [(1, 1, 0), (63, 5, 1), (64, 16, 0), (65, 17, 3),
+                                          (1023, 63, 0), (1024, 64, 2), (1025, 65, 0),
+                                          (8193, 130, 5), (3000, 784, 0)])
+def test_pack_bits_batch(device, bits, n, feats, skew):
+    """A sample-major batch packed as it lies: sample counts around the 64-sample blocks and
+    the 1024-sample tiles, feature counts around the 16-byte pieces and the 64-feature tiles, a
+    base address off every alignment, the batch's last byte the allocation's last."""
+    rng = np.random.default_rng(n + feats)
+    t = rng.integers(0, 2, (n, feats)).astype(bool)
+    flat = torch.zeros(skew + n * feats, dtype=torch.bool, device=device)
+    x = flat[skew:].view(n, feats)
+    x.copy_(torch.as_tensor(t))
+    packed, pad = dl.packbits_batch(x, bits)
+    ref, ref_pad = P.pack_bits(t.T.copy(), bits)
+    assert pad == ref_pad
+    assert np.array_equal(packed.cpu().numpy().view(np.uint8), ref)
+    for other in (x.t().contiguous().t(), torch.cat((x, x), 1)[:, :feats]):  # other layouts
+        again, pad = dl.packbits_batch(other, bits)
+        assert pad == ref_pad and torch.equal(again, packed)
