@@ -43,6 +43,8 @@ SIGNATURES: dict[str, list] = {
                                _i64, _i64, _i64, _i64, _i64, _p],
     "cl_dense_backward_rows": [_int, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64,
                                _i64, _i64, _p],
+    "cl_dense_backward_rows_any": [_int, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64,
+                               _i64, _i64, _p],
     "cl_transpose": [_int, _p, _p, _i64, _i64, _p],
     "cl_tree_conv_forward": [_int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _int, _int,
                              _int, _int, _int, _int, _p, _p, _p, _p, _p],
@@ -108,6 +110,8 @@ SIGNATURES: dict[str, list] = {
                                                   _i64, _i64, _i64, _p, _i64, _p],
     "cl_dense_backward_rows_first": [_int, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64,
                                      _i64, _i64, _p, _i64, _p, _i64, _p, _p, _p, _i64, _p],
+    "cl_dense_backward_rows_first_any": [_int, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64,
+                               _i64, _i64, _p, _i64, _p, _i64, _p, _p, _p, _i64, _p],
     "cl_plan_locality_order": [ctypes.POINTER(_i32), ctypes.POINTER(_i32), _i64, _i64,
                                ctypes.POINTER(_i32)],
     "cl_packed_bank_layout": [ctypes.POINTER(_i32), ctypes.POINTER(_i32),

@@ -44,6 +44,55 @@ __device__ __forceinline__ V vld(const void* p) {
     return *reinterpret_cast<const V*>(p);
 }
 
+// Rows of a batch that is no multiple of the 16-byte vector (TAIL): the rows then start at any
+// element, which the hardware's 16-byte accesses allow, and the row's last vector is moved back
+// to end with the row (tail_off), overlapping the one before it.  Two lanes then hold, compute
+// and store the same values for the overlapped samples, and sums over the batch leave them out
+// of the later lane (tail_keep).  Scalar accesses for such batches took 2.8 times as long (12011
+// neurons on 10007 inputs, batch 1999: forward 102 -> 55 us, backward 252 -> 72 us); only
+// batches shorter than one vector still use them.
+template <bool TAIL, typename T, typename V>
+__device__ __forceinline__ V vldr(const T* p) {
+    if constexpr (TAIL) {
+        typedef V Any __attribute__((aligned(sizeof(T))));
+        return *reinterpret_cast<const Any*>(p);
+    } else {
+        return *reinterpret_cast<const V*>(p);
+    }
+}
+
+template <bool TAIL, typename T, typename V>
+__device__ __forceinline__ void vstr(T* p, V v) {
+    if constexpr (TAIL) {
+        typedef V Any __attribute__((aligned(sizeof(T))));
+        *reinterpret_cast<Any*>(p) = v;
+    } else {
+        *reinterpret_cast<V*>(p) = v;
+    }
+}
+
+// Where the lane whose vector starts at sample idx < B reads and writes its row.
+template <bool TAIL, int VEC>
+__device__ __forceinline__ int64_t tail_off(int64_t idx, int64_t B) {
+    return TAIL && idx + VEC > B ? B - VEC : idx;
+}
+
+// v without the samples of another lane: its first `over` elements zero (all for over >= VEC).
+template <bool TAIL, typename T, int VEC>
+__device__ __forceinline__ typename VT<T, VEC>::type tail_keep(typename VT<T, VEC>::type v,
+                                                               int over) {
+    using V = typename VT<T, VEC>::type;
+    if constexpr (VEC == 1) {
+        return over > 0 ? V(T(0)) : v;
+    } else if constexpr (TAIL) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) v[i] = i < over ? T(0) : v[i];
+        return v;
+    } else {
+        return over > 0 ? V(T(0)) : v;
+    }
+}
+
 // One 16-byte load of an int4 record (the HIP struct type may be split into narrower loads).
 __device__ __forceinline__ int4 ld_rec(const int4* p) {
     typedef int I4 __attribute__((ext_vector_type(4)));
@@ -51,26 +100,16 @@ __device__ __forceinline__ int4 ld_rec(const int4* p) {
     return make_int4(v[0], v[1], v[2], v[3]);
 }
 
-// Lane accesses of the forward / backward tiled kernels are this many 16-byte vectors wide.
-// One for both: with connections='random' (16 runs per neuron) two-vector backward lanes
-// measured 0.346 ms per 12000 -> 12000 layer against 0.335 ms with one (2.78 -> 2.69 ms per
-// step); 8-lane chunks were far slower (0.58 ms: the per-chunk run work doubles).
+// Lane accesses of the forward / backward tiled kernels are one 16-byte vector wide: with
+// connections='random' (16 runs per neuron) two-vector backward lanes measured 0.346 ms per
+// 12000 -> 12000 layer against 0.335 ms with one (2.78 -> 2.69 ms per step); 8-lane chunks were
+// far slower (0.58 ms: the per-chunk run work doubles).
 // Runs of a neuron the tiled forward gathers together (connections='random': 0.134 -> 0.111 ms
 // per 12000 -> 12000 layer against one at a time; eight measured 0.124 ms).
 constexpr int kFwdRunBatch = 4;
 // Inverse-index entries the tiled backward gathers together (connections='random': 0.367 ->
 // 0.314 ms per 12000 -> 12000 layer against one at a time; two 0.342, eight 0.339 ms).
 constexpr int kBwdEntryBatch = 4;
-#ifndef CL_FWD_VEC_MULT
-#define CL_FWD_VEC_MULT 1
-#endif
-#ifndef CL_BWD_VEC_MULT
-#define CL_BWD_VEC_MULT 1
-#endif
-#ifndef CL_FUSED_VEC_MULT
-#define CL_FUSED_VEC_MULT 1
-#endif
-
 // Store of an output row segment.  Regular (write-back) stores measure faster inside a
 // training step than non-temporal ones: the next kernel reads these rows right away and then
 // finds them in the Infinity Cache.
@@ -293,7 +332,7 @@ __global__ __launch_bounds__(256) void k_prep(const T* __restrict__ w, int softm
 // neurons per tile).  nab[o] = (a, b of the first run, first run, end run) is one load, after
 // which the coefficients and both gathers of every neuron of the group are issued together.
 // Neurons with several runs continue through run_ab for the others.
-template <typename T, int VEC, int LPN, int NPG>
+template <typename T, int VEC, int LPN, int NPG, bool TAIL>
 __device__ __forceinline__ void fwd_tile(const T* __restrict__ x, const T* __restrict__ kc,
                                          const int4* __restrict__ nab,
                                          const int2* __restrict__ run_ab, T* __restrict__ y,
@@ -303,8 +342,9 @@ __device__ __forceinline__ void fwd_tile(const T* __restrict__ x, const T* __res
     using V4 = typename VT<T, 4>::type;
     constexpr int GROUPS = 256 / LPN;
     const int64_t obase = (t * GROUPS + threadIdx.x / LPN) * NPG;
-    const int64_t idx = c * (LPN * VEC) + int64_t(threadIdx.x % LPN) * VEC;
-    if (obase >= out_dim || idx >= B) return;
+    const int64_t at = c * (LPN * VEC) + int64_t(threadIdx.x % LPN) * VEC;
+    if (obase >= out_dim || at >= B) return;
+    const int64_t idx = tail_off<TAIL, VEC>(at, B);
     int4 rec[NPG];
 #pragma unroll
     for (int j = 0; j < NPG; ++j)
@@ -319,8 +359,8 @@ __device__ __forceinline__ void fwd_tile(const T* __restrict__ x, const T* __res
                 uint32_t(rec[j].y) < uint64_t(in_dim);
         if (ok[j]) {
             k[j] = vld<V4>(kc + 4 * int64_t(rec[j].z));
-            va[j] = vld<V>(x + int64_t(rec[j].x) * B + idx);
-            vb[j] = vld<V>(x + int64_t(rec[j].y) * B + idx);
+            va[j] = vldr<TAIL, T, V>(x + int64_t(rec[j].x) * B + idx);
+            vb[j] = vldr<TAIL, T, V>(x + int64_t(rec[j].y) * B + idx);
         }
     }
 #pragma unroll
@@ -348,8 +388,8 @@ __device__ __forceinline__ void fwd_tile(const T* __restrict__ x, const T* __res
                     const bool v = uint32_t(ab[q].x) < uint64_t(in_dim) &&
                                    uint32_t(ab[q].y) < uint64_t(in_dim);
                     badr = badr || !v;
-                    a[q] = vld<V>(x + int64_t(v ? ab[q].x : 0) * B + idx);
-                    b[q] = vld<V>(x + int64_t(v ? ab[q].y : 0) * B + idx);
+                    a[q] = vldr<TAIL, T, V>(x + int64_t(v ? ab[q].x : 0) * B + idx);
+                    b[q] = vldr<TAIL, T, V>(x + int64_t(v ? ab[q].y : 0) * B + idx);
                 }
                 if (badr) break;
 #pragma unroll
@@ -367,16 +407,16 @@ __device__ __forceinline__ void fwd_tile(const T* __restrict__ x, const T* __res
                     break;
                 }
                 const V4 kr = vld<V4>(kc + 4 * r);
-                const V a = vld<V>(x + int64_t(ab.x) * B + idx);
-                const V b = vld<V>(x + int64_t(ab.y) * B + idx);
+                const V a = vldr<TAIL, T, V>(x + int64_t(ab.x) * B + idx);
+                const V b = vldr<TAIL, T, V>(x + int64_t(ab.y) * B + idx);
                 acc += kr[3] * (a * b) + kr[2] * b + kr[1] * a + kr[0];
             }
         }
-        vst_stream<V>(y + o * B + idx, acc);
+        vstr<TAIL, T, V>(y + o * B + idx, acc);
     }
 }
 
-template <typename T, int VEC, int LPN, int NPG>
+template <typename T, int VEC, int LPN, int NPG, bool TAIL>
 __global__ __launch_bounds__(256) void k_fwd_tiled(const T* __restrict__ x,
                                                    const T* __restrict__ kc,
                                                    const int4* __restrict__ nab,
@@ -386,7 +426,7 @@ __global__ __launch_bounds__(256) void k_fwd_tiled(const T* __restrict__ x,
                                                    TileMap tm) {
     int64_t c, t;
     if (map_tile(tm, blockIdx.x, c, t))
-        fwd_tile<T, VEC, LPN, NPG>(x, kc, nab, run_ab, y, in_dim, out_dim, num_runs, B, c, t);
+        fwd_tile<T, VEC, LPN, NPG, TAIL>(x, kc, nab, run_ab, y, in_dim, out_dim, num_runs, B, c, t);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -448,7 +488,7 @@ __device__ __forceinline__ T fused_rcp(T v) {
 // the tile's first row, and the next class), the tile's lane groups add theirs in LDS in row
 // order, and the tile writes part[(t * 2 + slot) * B + n]; a tile spans at most two classes
 // (gsz >= 256 / LPN * NPG rows, checked by the host).
-template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD>
+template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD, bool TAIL>
 __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T* __restrict__ w,
                                                int softmax, const uint8_t* __restrict__ gs,
                                                const int4* __restrict__ nab,
@@ -469,7 +509,7 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
     const int l = threadIdx.x % LPN;
     const int64_t idx = c * (LPN * VEC) + int64_t(l) * VEC;
     const bool col = idx < B;
-    const int64_t off = col ? idx : 0;
+    const int64_t off = col ? tail_off<TAIL, VEC>(idx, B) : 0;
     const bool writer = uint32_t(c) == uint32_t(t) % uint32_t(tm.nchunks);
     // Every load is unconditional (a clamped address, the value masked after it arrives): a
     // load under a branch makes the compiler wait there for all loads in flight, which would
@@ -499,8 +539,8 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
     for (int j = 0; j < NPG; ++j) {
         ok[j] = live[j] && rec[j].z >= 0 && rec[j].w == rec[j].z + 1 && rec[j].w <= num_runs &&
                 uint32_t(rec[j].x) < uint64_t(in_dim) && uint32_t(rec[j].y) < uint64_t(in_dim);
-        va[j] = vld<V>(x + int64_t(ok[j] ? rec[j].x : 0) * B + off);
-        vb[j] = vld<V>(x + int64_t(ok[j] ? rec[j].y : 0) * B + off);
+        va[j] = vldr<TAIL, T, V>(x + int64_t(ok[j] ? rec[j].x : 0) * B + off);
+        vb[j] = vldr<TAIL, T, V>(x + int64_t(ok[j] ? rec[j].y : 0) * B + off);
         // entry positions of the run's two sides, for the tile's writer chunk
         if constexpr (COEF) {
             const int64_t rz = ok[j] ? rec[j].z : 0;
@@ -582,7 +622,7 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
                 if (o < bound) h0 += acc;
                 else h1 += acc;
             } else {
-                vst_stream<V>(y + o * B + idx, acc);
+                vstr<TAIL, T, V>(y + o * B + off, acc);
             }
         }
     }
@@ -611,7 +651,7 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
     }
 }
 
-template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD>
+template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD, bool TAIL>
 __global__ __launch_bounds__(256) void k_fwd_fused(const T* __restrict__ x, const T* __restrict__ w,
                                                    int softmax, const uint8_t* __restrict__ gs,
                                                    const int4* __restrict__ nab,
@@ -624,7 +664,7 @@ __global__ __launch_bounds__(256) void k_fwd_fused(const T* __restrict__ x, cons
     __shared__ T red[HEAD ? 2 * 256 * VEC : 1];
     int64_t c, t;
     if (map_tile(tm, blockIdx.x, c, t))  // uniform per workgroup
-        fwd_fused_tile<T, VEC, LPN, NPG, COEF, HEAD>(x, w, softmax, gs, nab, inv_pos, probs,
+        fwd_fused_tile<T, VEC, LPN, NPG, COEF, HEAD, TAIL>(x, w, softmax, gs, nab, inv_pos, probs,
                                                      inv_coef, y, in_dim, out_dim, num_runs, B,
                                                      G, tm, c, t, part, gsz, red);
 }
@@ -698,7 +738,7 @@ __device__ __forceinline__ Coef4<T> row_run_coef(const SlotProbs<T, NG>& sp,
 // k_wgrad_full: weight gradient per neuron over the whole batch (16 lanes per neuron), with
 // the softmax backward when `probs` is given.  Used when no input gradient is needed, so no
 // per-chunk moments or finalize pass are required.
-template <typename T, int VEC>
+template <typename T, int VEC, bool TAIL>
 __global__ __launch_bounds__(256) void k_wgrad_full(const T* __restrict__ x, const T* __restrict__ gy,
                                                     const uint8_t* __restrict__ gs,
                                                     const T* __restrict__ probs,
@@ -734,9 +774,10 @@ __global__ __launch_bounds__(256) void k_wgrad_full(const T* __restrict__ x, con
             const T* xa = x + int64_t(ab.x) * B;
             const T* xb = x + int64_t(ab.y) * B;
             for (int64_t idx = int64_t(l) * VEC; idx < B; idx += 16 * VEC) {
-                const V vg = vld<V>(gyr + idx);
-                const V va = vld<V>(xa + idx);
-                const V vb = vld<V>(xb + idx);
+                const int64_t off = tail_off<TAIL, VEC>(idx, B);
+                const V vg = tail_keep<TAIL, T, VEC>(vldr<TAIL, T, V>(gyr + off), int(idx - off));
+                const V va = vldr<TAIL, T, V>(xa + off);
+                const V vb = vldr<TAIL, T, V>(xb + off);
                 const V ga = vg * va;
                 s1 += hsum<T, VEC>(vg);
                 sa += hsum<T, VEC>(ga);
@@ -784,7 +825,7 @@ __global__ __launch_bounds__(256) void k_wgrad_full(const T* __restrict__ x, con
 // unconditional (clamped, masked afterwards) so they are in flight together, and run o's
 // pair is fetched with run_ptr[o]: in a layer of single-run neurons run o is neuron o's
 // only run, and its row gathers need no second round trip.
-template <typename T, int VEC, int U, bool HAS_P>
+template <typename T, int VEC, int U, bool HAS_P, bool TAIL>
 __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
                                                     const T* __restrict__ gy,
                                                     const uint8_t* __restrict__ gs,
@@ -800,14 +841,13 @@ __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
     const int64_t o = int64_t(blockIdx.x) * 4 + wave_id();
     if (o >= out_dim) return;  // uniform per wave
     int64_t off[U];
-    bool in[U];
+    const int over0 = (lane + 1) * VEC - int(B);  // as in k_bwd_rows
     V vg[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int64_t idx = int64_t(u * 64 + lane) * VEC;
-        in[u] = idx < B;
-        off[u] = in[u] ? idx : 0;
-        vg[u] = vld<V>(gy + o * B + off[u]);
+        off[u] = idx < B ? tail_off<TAIL, VEC>(idx, B) : 0;
+        vg[u] = vldr<TAIL, T, V>(gy + o * B + off[u]);
     }
     const int gl = lane < G ? lane : 0;
     const int code = gs[o * G + gl];
@@ -824,7 +864,7 @@ __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
     T s1 = 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        vg[u] = in[u] ? vg[u] : V(T(0));
+        vg[u] = tail_keep<TAIL, T, VEC>(vg[u], over0 + 64 * VEC * u);
         s1 += hsum<T, VEC>(vg[u]);
     }
     const T m0 = wave_total(s1);
@@ -845,8 +885,8 @@ __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
         V va[U], vb[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            va[u] = vld<V>(x + int64_t(ab.x) * B + off[u]);
-            vb[u] = vld<V>(x + int64_t(ab.y) * B + off[u]);
+            va[u] = vldr<TAIL, T, V>(x + int64_t(ab.x) * B + off[u]);
+            vb[u] = vldr<TAIL, T, V>(x + int64_t(ab.y) * B + off[u]);
         }
         T m1, m2, m3;
         run_moments<T, VEC, U>(vg, va, vb, m1, m2, m3);
@@ -867,7 +907,7 @@ __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
 // kBwdEntryBatch at a time, their records and row gathers in flight together.
 // part[(r * nchunks + c) * 4 + j] receives the chunk-c moments of run r (WANT_GW) at the
 // run's operand-a entry.
-template <typename T, int VEC, int LPN, int NPG, bool WANT_GX, bool WANT_GW>
+template <typename T, int VEC, int LPN, int NPG, bool WANT_GX, bool WANT_GW, bool TAIL>
 __device__ __forceinline__ void bwd_tile(
     const T* __restrict__ x, const T* __restrict__ gy, const int4* __restrict__ slot_rec,
     const int4* __restrict__ inv_rec, const T* __restrict__ inv_coef, T* __restrict__ gx,
@@ -882,6 +922,8 @@ __device__ __forceinline__ void bwd_tile(
     if (slot0 >= in_dim) return;  // uniform per lane group
     const int64_t idx = c * (LPN * VEC) + int64_t(threadIdx.x % LPN) * VEC;
     const bool col = idx < B;
+    const int64_t off = col ? tail_off<TAIL, VEC>(idx, B) : 0;
+    const int over = col ? int(idx - off) : VEC;
     const bool leader = (threadIdx.x % LPN) == 0;
 
     int64_t row[NPG], e0[NPG], deg[NPG];
@@ -908,14 +950,13 @@ __device__ __forceinline__ void bwd_tile(
     for (int j = 0; j < NPG; ++j) {
         acc[j] = V(T(0));
         xi[j] = V(T(0));
-        if (WANT_GW && live[j] && col) xi[j] = vld<V>(x + row[j] * B + idx);
+        if (WANT_GW && live[j] && col) xi[j] = vldr<TAIL, T, V>(x + row[j] * B + off);
     }
     // Entries are taken kBwdEntryBatch at a time: the batch's records and coefficients, then
     // all of its row gathers, are in flight together (every load unconditional: an unused
     // entry reads entry e0 and row 0, lanes past the batch read sample 0, and both are masked
     // afterwards); the accumulation order is the entry order.
     constexpr int EB = kBwdEntryBatch;
-    const int64_t off = col ? idx : 0;
 #pragma unroll
     for (int j = 0; j < NPG; ++j)
         if (!live[j]) e0[j] = 0;  // a dead or corrupt slot's unused loads read entry 0
@@ -944,8 +985,8 @@ __device__ __forceinline__ void bwd_tile(
                     use[j][q] = false;
                 }
                 const bool u = use[j][q];
-                vo[j][q] = vld<V>(x + int64_t(u ? cur[j][q].y : 0) * B + off);
-                vg[j][q] = vld<V>(gy + int64_t(u ? cur[j][q].x : 0) * B + off);
+                vo[j][q] = vldr<TAIL, T, V>(x + int64_t(u ? cur[j][q].y : 0) * B + off);
+                vg[j][q] = vldr<TAIL, T, V>(gy + int64_t(u ? cur[j][q].x : 0) * B + off);
             }
 #pragma unroll
         for (int j = 0; j < NPG; ++j)
@@ -953,9 +994,10 @@ __device__ __forceinline__ void bwd_tile(
             for (int q = 0; q < EB; ++q) {
                 if (!use[j][q]) continue;
                 const V o = col ? vo[j][q] : V(T(0));
-                const V g = col ? vg[j][q] : V(T(0));
+                V g = col ? vg[j][q] : V(T(0));
                 if (WANT_GX) acc[j] += (ck[j][q][0] + ck[j][q][1] * o) * g;
                 if (WANT_GW && cur[j][q].w == 0) {
+                    if constexpr (TAIL) g = tail_keep<TAIL, T, VEC>(g, over);
                     const V ga = g * xi[j];
                     T s1 = hsum<T, VEC>(g), sa = hsum<T, VEC>(ga);
                     T sb = hsum<T, VEC>(g * o), sab = hsum<T, VEC>(ga * o);
@@ -980,12 +1022,12 @@ __device__ __forceinline__ void bwd_tile(
             if (!live[j]) continue;
             V r = acc[j];
             if (bad[j]) r = V(nan_of<T>());
-            vst_stream<V>(gx + row[j] * B + idx, r);
+            vstr<TAIL, T, V>(gx + row[j] * B + off, r);
         }
     }
 }
 
-template <typename T, int VEC, int LPN, int NPG, bool WANT_GX, bool WANT_GW>
+template <typename T, int VEC, int LPN, int NPG, bool WANT_GX, bool WANT_GW, bool TAIL>
 __global__ __launch_bounds__(256) void k_bwd_tiled(
     const T* __restrict__ x, const T* __restrict__ gy, const int4* __restrict__ slot_rec,
     const int4* __restrict__ inv_rec, const T* __restrict__ inv_coef, T* __restrict__ gx,
@@ -993,7 +1035,7 @@ __global__ __launch_bounds__(256) void k_bwd_tiled(
     int64_t in_dim, int64_t out_dim, int64_t num_runs, int64_t B, TileMap tm) {
     int64_t c, t;
     if (map_tile(tm, blockIdx.x, c, t))
-        bwd_tile<T, VEC, LPN, NPG, WANT_GX, WANT_GW>(x, gy, slot_rec, inv_rec, inv_coef, gx, part,
+        bwd_tile<T, VEC, LPN, NPG, WANT_GX, WANT_GW, TAIL>(x, gy, slot_rec, inv_rec, inv_coef, gx, part,
                                                      in_dim, out_dim, num_runs, B, tm, c, t);
 }
 
@@ -1013,7 +1055,7 @@ __global__ __launch_bounds__(256) void k_bwd_tiled(
 constexpr int kPartRows = 16;
 constexpr int kPartMaxSlots = 64;
 
-template <typename T, int VEC, int LPN, bool WANT_GX, bool WANT_GW>
+template <typename T, int VEC, int LPN, bool WANT_GX, bool WANT_GW, bool TAIL>
 __global__ __launch_bounds__(256) void k_bwd_part(
     const T* __restrict__ x, const T* __restrict__ gy, const int4* __restrict__ slot_rec,
     const int4* __restrict__ inv_rec, const T* __restrict__ inv_coef,
@@ -1035,8 +1077,10 @@ __global__ __launch_bounds__(256) void k_bwd_part(
     const int tl = g / kPartRows, rg = g % kPartRows;
     const int64_t tile = t * TPW + tl;
     const int64_t slot = tile * kPartRows + rg;
-    const int64_t idx = c * CH + int64_t(l) * VEC;
-    const bool col = idx < B;
+    const int64_t at = c * CH + int64_t(l) * VEC;
+    const bool col = at < B;
+    const int64_t idx = col ? tail_off<TAIL, VEC>(at, B) : 0;
+    const int over = col ? int(at - idx) : VEC;
     const bool leader = l == 0;
     T* xs_t = xs + tl * kPartRows * CH;
     T* cs_t = cs + int64_t(tl) * slots * CH;
@@ -1050,7 +1094,7 @@ __global__ __launch_bounds__(256) void k_bwd_part(
         live = false;  // corrupt slot record: nothing is read or written for it
     if (!live) deg = 0;
     V xi = V(T(0));
-    if (live && col) xi = vld<V>(x + row * B + idx);
+    if (live && col) xi = vldr<TAIL, T, V>(x + row * B + idx);
     *reinterpret_cast<V*>(xs_t + rg * CH + l * VEC) = xi;
     __syncthreads();
 
@@ -1071,7 +1115,7 @@ __global__ __launch_bounds__(256) void k_bwd_part(
                 sa >= slots || sb >= slots)
                 continue;  // corrupt record: skipped, nothing is read or written for it
             V vg = V(T(0));
-            if (col) vg = vld<V>(gy + int64_t(tr.x) * B + idx);
+            if (col) vg = vldr<TAIL, T, V>(gy + int64_t(tr.x) * B + idx);
             const V2 ka = vld<V2>(inv_coef + 2 * int64_t(tr.z));
             const V2 kb = vld<V2>(inv_coef + 2 * int64_t(tr.w));
             const V va = *reinterpret_cast<const V*>(xs_t + al * CH + l * VEC);
@@ -1081,6 +1125,7 @@ __global__ __launch_bounds__(256) void k_bwd_part(
                 *reinterpret_cast<V*>(cs_t + sb * CH + l * VEC) = (kb[0] + kb[1] * va) * vg;
             }
             if (WANT_GW) {
+                if constexpr (TAIL) vg = tail_keep<TAIL, T, VEC>(vg, over);
                 const V ga = vg * va;
                 T s1 = hsum<T, VEC>(vg), s2 = hsum<T, VEC>(ga);
                 T s3 = hsum<T, VEC>(vg * vb), s4 = hsum<T, VEC>(ga * vb);
@@ -1136,11 +1181,12 @@ __global__ __launch_bounds__(256) void k_bwd_part(
         }
         V vo = V(T(0)), vg = V(T(0));
         if (col) {
-            vo = vld<V>(x + int64_t(cur.y) * B + idx);
-            vg = vld<V>(gy + int64_t(cur.x) * B + idx);
+            vo = vldr<TAIL, T, V>(x + int64_t(cur.y) * B + idx);
+            vg = vldr<TAIL, T, V>(gy + int64_t(cur.x) * B + idx);
         }
         if (WANT_GX) acc += (ck[0] + ck[1] * vo) * vg;
         if (WANT_GW && cur.w == 0) {
+            if constexpr (TAIL) vg = tail_keep<TAIL, T, VEC>(vg, over);
             const V ga = vg * xi;
             T s1 = hsum<T, VEC>(vg), s2 = hsum<T, VEC>(ga);
             T s3 = hsum<T, VEC>(vg * vo), s4 = hsum<T, VEC>(ga * vo);
@@ -1161,7 +1207,7 @@ __global__ __launch_bounds__(256) void k_bwd_part(
     if (WANT_GX && live && col) {
         V r = acc;
         if (bad) r = V(nan_of<T>());
-        vst_stream<V>(gx + row * B + idx, r);
+        vstr<TAIL, T, V>(gx + row * B + idx, r);
     }
 }
 
@@ -1227,7 +1273,8 @@ struct FirstLayer {
 // workgroup share a row, wave `part` taking the contiguous part of its entries
 // [deg * part / S, deg * (part + 1) / S); the parts' input-gradient sums meet in LDS and are
 // added in part order (deterministic; the association differs from S = 1 by rounding).
-template <typename T, int VEC, int U, bool WANT_GW, bool HAS_P, bool FIRST = false, int S = 1>
+template <typename T, int VEC, int U, bool WANT_GW, bool HAS_P, bool TAIL, bool FIRST = false,
+          int S = 1>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_rows_waves<T, U, FIRST>())))
 void k_bwd_rows(
     const T* __restrict__ x, const T* __restrict__ gy, const int4* __restrict__ slot_rec,
@@ -1240,7 +1287,7 @@ void k_bwd_rows(
     static_assert(S == 1 || !FIRST, "the first-layer mode takes one wave per row");
     using V = typename VT<T, VEC>::type;
     using V2 = typename VT<T, 2>::type;
-    constexpr int EPI = U <= 2 ? 2 : U <= 4 ? (FIRST ? CL_FIRST_EPI4 : CL_BWD_ROWS_EPI4) : 1;
+    constexpr int EPI = U <= 2 ? 2 : U <= 4 ? (FIRST || TAIL ? CL_FIRST_EPI4 : CL_BWD_ROWS_EPI4) : 1;
     const int lane = threadIdx.x & 63;
     const int64_t w = blockIdx.x;
     const int wv = wave_id();
@@ -1266,14 +1313,17 @@ void k_bwd_rows(
     for (int u = 0; u < U; ++u) {
         const int64_t idx = int64_t(u * 64 + lane) * VEC;
         in[u] = idx < B;
-        off[u] = in[u] ? idx : 0;
+        off[u] = in[u] ? int32_t(tail_off<TAIL, VEC>(idx, B)) : 0;
     }
+    // leading samples of vector u that another lane holds (or that lie past the batch): those
+    // before element over0 + 64 * VEC * u
+    const int over0 = (lane + 1) * VEC - int(B);
     V xi[U], acc[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         acc[u] = V(T(0));
         xi[u] = V(T(0));
-        if constexpr (WANT_GW) xi[u] = vld<V>(x + row * B + off[u]);
+        if constexpr (WANT_GW) xi[u] = vldr<TAIL, T, V>(x + row * B + off[u]);
     }
     const int gl = lane < G ? lane : 0;  // slot of this lane in the finalize (clamped)
     bool bad = false;
@@ -1312,8 +1362,8 @@ void k_bwd_rows(
                                          : int64_t(cur[q].x);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                vo[q][u] = vld<V>(x + int64_t(cur[q].y) * B + off[u]);
-                vg[q][u] = vld<V>(gy + gyr * B + off[u]);
+                vo[q][u] = vldr<TAIL, T, V>(x + int64_t(cur[q].y) * B + off[u]);
+                vg[q][u] = vldr<TAIL, T, V>(gy + gyr * B + off[u]);
             }
             // the finalize's per-neuron data is loaded with the rows, not after the moments
             if constexpr (WANT_GW) {
@@ -1341,7 +1391,7 @@ void k_bwd_rows(
                 T s1 = 0, s2 = 0, s3 = 0, s4 = 0;
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const V g = in[u] ? vg[q][u] : V(T(0));
+                    const V g = tail_keep<TAIL, T, VEC>(vg[q][u], over0 + 64 * VEC * u);
                     const V ga = g * xi[u];
                     s1 += hsum<T, VEC>(g);
                     s2 += hsum<T, VEC>(ga);
@@ -1377,13 +1427,13 @@ void k_bwd_rows(
         V va[U], vb[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            va[u] = vld<V>(first.x0 + ra * B + off[u]);
-            vb[u] = vld<V>(first.x0 + rb * B + off[u]);
+            va[u] = vldr<TAIL, T, V>(first.x0 + ra * B + off[u]);
+            vb[u] = vldr<TAIL, T, V>(first.x0 + rb * B + off[u]);
         }
         T s1 = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            acc[u] = in[u] ? acc[u] : V(T(0));
+            acc[u] = tail_keep<TAIL, T, VEC>(acc[u], over0 + 64 * VEC * u);
             s1 += hsum<T, VEC>(acc[u]);
         }
         const T m0 = wave_total(s1);
@@ -1413,12 +1463,12 @@ void k_bwd_rows(
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (in[u]) vst_stream<V>(gx + row * B + off[u], bad ? V(nan_of<T>()) : acc[u]);
+            if (in[u]) vstr<TAIL, T, V>(gx + row * B + off[u], bad ? V(nan_of<T>()) : acc[u]);
     }
 }
 
 // k_moments: the per-chunk moments of every run, per neuron (used when grad_x is not needed).
-template <typename T, int VEC, int LPN>
+template <typename T, int VEC, int LPN, bool TAIL>
 __global__ __launch_bounds__(256) void k_moments(const T* __restrict__ x, const T* __restrict__ gy,
                                                  const int32_t* __restrict__ run_ptr,
                                                  const int2* __restrict__ run_ab,
@@ -1434,19 +1484,20 @@ __global__ __launch_bounds__(256) void k_moments(const T* __restrict__ x, const 
     if (o >= out_dim) return;  // uniform per lane group
     const int64_t idx = c * (LPN * VEC) + int64_t(threadIdx.x % LPN) * VEC;
     const bool col = idx < B;
+    const int64_t off = col ? tail_off<TAIL, VEC>(idx, B) : 0;
     const bool leader = (threadIdx.x % LPN) == 0;
     int64_t r0 = run_ptr[o], r1 = run_ptr[o + 1];
     if (r0 < 0 || r1 < r0 || r1 > num_runs) return;
     V vg = V(T(0));
-    if (col) vg = vld<V>(gy + o * B + idx);
+    if (col) vg = tail_keep<TAIL, T, VEC>(vldr<TAIL, T, V>(gy + o * B + off), int(idx - off));
     const T s1 = group_sum<LPN>(hsum<T, VEC>(vg));
     for (int64_t r = r0; r < r1; ++r) {
         const int2 ab = run_ab[r];
         V va = V(T(0)), vb = V(T(0));
         const bool ok = uint32_t(ab.x) < uint64_t(in_dim) && uint32_t(ab.y) < uint64_t(in_dim);
         if (col && ok) {
-            va = vld<V>(x + int64_t(ab.x) * B + idx);
-            vb = vld<V>(x + int64_t(ab.y) * B + idx);
+            va = vldr<TAIL, T, V>(x + int64_t(ab.x) * B + off);
+            vb = vldr<TAIL, T, V>(x + int64_t(ab.y) * B + off);
         }
         const V ga = vg * va;
         const T sa = group_sum<LPN>(hsum<T, VEC>(ga));
@@ -1543,7 +1594,9 @@ __global__ __launch_bounds__(256) void k_zero(T* __restrict__ p, int64_t n) {
 // Host-side tiling choice.
 
 struct Tiling {
-    int vec;   // elements per 16-byte access (1 when the batch does not allow vectors)
+    int vec;   // elements per 16-byte access (1: batches shorter than one vector, and the head's
+               // batches that are no multiple of it)
+    bool tail;  // the batch is no multiple of vec (see vldr)
     int lpn;   // lanes per row segment
     int64_t chunk;
     TileMap map;
@@ -1551,12 +1604,13 @@ struct Tiling {
 
 // Narrowest lane group first that still leaves every XCD a chunk; bands of at most
 // `lpn_max` lanes keep a chunk's activation band within one XCD's L2.
-// Lane vector width: `mult` 16-byte vectors when the batch allows it, else one, else scalars.
 template <typename T>
-Tiling choose_tiling(int64_t B, int64_t rows, int mult, int lpn_max, int rows_per_group = 1) {
+Tiling choose_tiling(int64_t B, int64_t rows, int lpn_max, int rows_per_group = 1,
+                     bool tails = true) {
     Tiling tl;
     constexpr int W = wide_vec<T>();
-    tl.vec = B % (W * mult) == 0 ? W * mult : (B % W == 0 ? W : 1);
+    tl.vec = B % W == 0 || (tails && B >= W) ? W : 1;
+    tl.tail = B % tl.vec != 0;
     tl.lpn = lpn_max;
     while (tl.lpn > 4 && ceil_div(B, int64_t(tl.lpn) * tl.vec) < kXcds) tl.lpn >>= 1;
     tl.chunk = int64_t(tl.lpn) * tl.vec;
@@ -1585,9 +1639,9 @@ using namespace cl;
 
 namespace {
 
-// The tiling (and with it the chunk count of the moments buffer) depends on the batch alone:
-// 16-byte vectors whenever batch % (16 / sizeof(T)) == 0, which then requires 16-byte aligned
-// row buffers.
+// The tiling (and with it the chunk count of the moments buffer) depends on the batch alone.
+// Batches that are a multiple of the 16-byte vector take aligned vectors and need 16-byte
+// aligned row buffers; others take vectors at any element.
 template <typename T>
 bool vec_ok(int64_t B) {
     return B % wide_vec<T>() == 0;
@@ -1611,25 +1665,22 @@ int check_plan_dims(int64_t in_dim, int64_t out_dim, int64_t B, int64_t G, int64
 
 namespace {
 
-// Calls f(std::integral_constant<int, VEC>, std::integral_constant<int, LPN>) for the
-// tiling's vector width and lane-group size.
-template <typename T, int MULT, typename F>
+// Calls f(std::integral_constant<int, VEC>, std::integral_constant<int, LPN>,
+// std::bool_constant<TAIL>) for the tiling.
+template <typename T, typename F>
 void with_tiling(const Tiling& tl, F&& f) {
     constexpr int W = wide_vec<T>();
-    using I = std::integral_constant<int, 1>;
-    using IW = std::integral_constant<int, W>;
-    using IM = std::integral_constant<int, W * MULT>;
     using L4 = std::integral_constant<int, 4>;
     using L8 = std::integral_constant<int, 8>;
     using L16 = std::integral_constant<int, 16>;
-    auto by_lanes = [&](auto vc) {
-        if (tl.lpn == 16) f(vc, L16{});
-        else if (tl.lpn == 8) f(vc, L8{});
-        else f(vc, L4{});
+    auto by_lanes = [&](auto vc, auto tc) {
+        if (tl.lpn == 16) f(vc, L16{}, tc);
+        else if (tl.lpn == 8) f(vc, L8{}, tc);
+        else f(vc, L4{}, tc);
     };
-    if (MULT > 1 && tl.vec == W * MULT) by_lanes(IM{});
-    else if (tl.vec == W) by_lanes(IW{});
-    else by_lanes(I{});
+    if (tl.vec == 1) by_lanes(std::integral_constant<int, 1>{}, std::false_type{});
+    else if (tl.tail) by_lanes(std::integral_constant<int, W>{}, std::true_type{});
+    else by_lanes(std::integral_constant<int, W>{}, std::false_type{});
 }
 
 }  // namespace
@@ -1668,15 +1719,15 @@ extern "C" int cl_dense_forward_tiled(int dtype, const void* x, const void* run_
     CL_DTYPE_SWITCH(dtype, {
         using T = scalar_t;
         CL_ARG(!vec_ok<T>(batch) || all_aligned({x, y}), "x and y must be 16-byte aligned");
-        const Tiling tl = choose_tiling<T>(batch, out_dim, CL_FWD_VEC_MULT, CL_FWD_LPN, CL_FWD_NPG);
+        const Tiling tl = choose_tiling<T>(batch, out_dim, CL_FWD_LPN, CL_FWD_NPG);
         const unsigned grid = unsigned(tile_grid(tl.map));
         auto* xs = static_cast<const T*>(x);
         auto* kc = static_cast<const T*>(run_coef);
         auto* nb = reinterpret_cast<const int4*>(nab);
         auto* ab = reinterpret_cast<const int2*>(run_ab);
         auto* ys = static_cast<T*>(y);
-        with_tiling<T, CL_FWD_VEC_MULT>(tl, [&](auto vc, auto lc) {
-            k_fwd_tiled<T, decltype(vc)::value, decltype(lc)::value, CL_FWD_NPG>
+        with_tiling<T>(tl, [&](auto vc, auto lc, auto tc) {
+            k_fwd_tiled<T, decltype(vc)::value, decltype(lc)::value, CL_FWD_NPG, decltype(tc)::value>
                 <<<grid, 256, 0, s>>>(xs, kc, nb, ab, ys, in_dim, out_dim, num_runs, batch, tl.map);
         });
     });
@@ -1704,7 +1755,7 @@ extern "C" int cl_dense_forward_fused(int dtype, const void* x, const void* w, i
     CL_DTYPE_SWITCH(dtype, {
         using T = scalar_t;
         CL_ARG(!vec_ok<T>(batch) || all_aligned({x, y}), "x and y must be 16-byte aligned");
-        const Tiling tl = choose_tiling<T>(batch, out_dim, CL_FUSED_VEC_MULT, CL_FWD_LPN, CL_FWD_NPG);
+        const Tiling tl = choose_tiling<T>(batch, out_dim, CL_FWD_LPN, CL_FWD_NPG);
         const unsigned grid = unsigned(tile_grid(tl.map));
         auto* xs = static_cast<const T*>(x);
         auto* ws = static_cast<const T*>(w);
@@ -1712,14 +1763,15 @@ extern "C" int cl_dense_forward_fused(int dtype, const void* x, const void* w, i
         auto* pr = static_cast<T*>(probs);
         auto* ic = static_cast<T*>(inv_coef);
         auto* ys = static_cast<T*>(y);
-        with_tiling<T, CL_FUSED_VEC_MULT>(tl, [&](auto vc, auto lc) {
+        with_tiling<T>(tl, [&](auto vc, auto lc, auto tc) {
             constexpr int VEC = decltype(vc)::value, LPN = decltype(lc)::value;
+            constexpr bool TAIL = decltype(tc)::value;
             if (ic)
-                k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, true, false><<<grid, 256, 0, s>>>(
+                k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, true, false, TAIL><<<grid, 256, 0, s>>>(
                     xs, ws, softmax, gate_seq, nb, inv_pos, pr, ic, ys, in_dim, out_dim, num_runs,
                     batch, int(num_gates), tl.map, nullptr, 0);
             else
-                k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, false, false><<<grid, 256, 0, s>>>(
+                k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, false, false, TAIL><<<grid, 256, 0, s>>>(
                     xs, ws, softmax, gate_seq, nb, inv_pos, pr, ic, ys, in_dim, out_dim, num_runs,
                     batch, int(num_gates), tl.map, nullptr, 0);
         });
@@ -1752,30 +1804,40 @@ extern "C" int cl_dense_weight_grad(int dtype, const void* x, const void* grad_y
         auto* pr = static_cast<const T*>(probs);
         auto* ab = reinterpret_cast<const int2*>(run_ab);
         auto* gw = static_cast<T*>(grad_w);
-        if (v && batch > 0 && num_gates <= 64 && batch <= 64 * W * 8) {
+        const bool wide = batch >= W;
+        if (wide && num_gates <= 64 && batch <= 64 * W * 8) {
             const unsigned wgrid = unsigned(ceil_div(out_dim, int64_t(4)));
-            auto go = [&](auto uc) {
+            auto launch = [&](auto uc, auto tc) {
                 constexpr int U = decltype(uc)::value;
+                constexpr bool TAIL = decltype(tc)::value;
                 if (pr)
-                    k_wgrad_rows<T, W, U, true><<<wgrid, 256, 0, s>>>(
+                    k_wgrad_rows<T, W, U, true, TAIL><<<wgrid, 256, 0, s>>>(
                         xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw,
                         std::max<int64_t>(in_dim, 1), out_dim, num_runs, batch, int(num_gates));
                 else
-                    k_wgrad_rows<T, W, U, false><<<wgrid, 256, 0, s>>>(
+                    k_wgrad_rows<T, W, U, false, TAIL><<<wgrid, 256, 0, s>>>(
                         xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw,
                         std::max<int64_t>(in_dim, 1), out_dim, num_runs, batch, int(num_gates));
+            };
+            auto go = [&](auto uc) {
+                if (v) launch(uc, std::false_type{});
+                else launch(uc, std::true_type{});
             };
             const int64_t per_u = 64 * W;
             if (batch <= per_u) go(std::integral_constant<int, 1>{});
             else if (batch <= 2 * per_u) go(std::integral_constant<int, 2>{});
             else if (batch <= 4 * per_u) go(std::integral_constant<int, 4>{});
             else go(std::integral_constant<int, 8>{});
-        } else if (v)
-            k_wgrad_full<T, W><<<grid, 256, 0, s>>>(xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw,
+        } else if (wide && !v)
+            k_wgrad_full<T, W, true><<<grid, 256, 0, s>>>(
+                xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw, std::max<int64_t>(in_dim, 1),
+                out_dim, num_runs, batch, int(num_gates));
+        else if (wide)
+            k_wgrad_full<T, W, false><<<grid, 256, 0, s>>>(xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw,
                                                    std::max<int64_t>(in_dim, 1), out_dim, num_runs,
                                                    batch, int(num_gates));
         else
-            k_wgrad_full<T, 1><<<grid, 256, 0, s>>>(xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw,
+            k_wgrad_full<T, 1, false><<<grid, 256, 0, s>>>(xs, gys, gate_seq, pr, run_ptr, ab, run_gl, gw,
                                                    std::max<int64_t>(in_dim, 1), out_dim, num_runs,
                                                    batch, int(num_gates));
     });
@@ -1791,7 +1853,7 @@ extern "C" int cl_dense_tiled_chunks(int dtype, int64_t batch, int64_t in_dim, i
     (void)out_dim;
     CL_DTYPE_SWITCH(dtype, {
         const int64_t b = std::max<int64_t>(batch, 1);
-        *nchunks = choose_tiling<scalar_t>(b, 1, CL_BWD_VEC_MULT, CL_BWD_LPN).map.nchunks;
+        *nchunks = choose_tiling<scalar_t>(b, 1, CL_BWD_LPN).map.nchunks;
     });
     return CL_OK;
 }
@@ -1840,28 +1902,31 @@ extern "C" int cl_dense_backward_tiled(int dtype, const void* x, const void* gra
         auto* gxs = static_cast<T*>(grad_x);
         auto* mom = static_cast<T*>(moments);
         if (grad_x && in_dim > 0) {
-            const Tiling tl = choose_tiling<T>(batch, in_dim, CL_BWD_VEC_MULT, CL_BWD_LPN, CL_BWD_NPG);
+            const Tiling tl = choose_tiling<T>(batch, in_dim, CL_BWD_LPN, CL_BWD_NPG);
             const unsigned grid = unsigned(tile_grid(tl.map));
             if (moments) {
                 CL_ARG(nchunks == tl.map.nchunks, "moments buffer must use the backward chunk count");
-                with_tiling<T, CL_BWD_VEC_MULT>(tl, [&](auto vc, auto lc) {
-                    k_bwd_tiled<T, decltype(vc)::value, decltype(lc)::value, CL_BWD_NPG, true, true>
+                with_tiling<T>(tl, [&](auto vc, auto lc, auto tc) {
+                    k_bwd_tiled<T, decltype(vc)::value, decltype(lc)::value, CL_BWD_NPG, true, true,
+                                decltype(tc)::value>
                         <<<grid, 256, 0, s>>>(xs, gys, srec, rec, ic, gxs, mom,
                                               in_dim, out_dim, num_runs, batch, tl.map);
                 });
             } else {
-                with_tiling<T, CL_BWD_VEC_MULT>(tl, [&](auto vc, auto lc) {
-                    k_bwd_tiled<T, decltype(vc)::value, decltype(lc)::value, CL_BWD_NPG, true, false>
+                with_tiling<T>(tl, [&](auto vc, auto lc, auto tc) {
+                    k_bwd_tiled<T, decltype(vc)::value, decltype(lc)::value, CL_BWD_NPG, true, false,
+                                decltype(tc)::value>
                         <<<grid, 256, 0, s>>>(xs, gys, srec, rec, ic, gxs, mom,
                                               in_dim, out_dim, num_runs, batch, tl.map);
                 });
             }
         } else if (moments && out_dim > 0) {
-            const Tiling tl = choose_tiling<T>(batch, out_dim, CL_BWD_VEC_MULT, CL_BWD_LPN);
+            const Tiling tl = choose_tiling<T>(batch, out_dim, CL_BWD_LPN);
             CL_ARG(nchunks == tl.map.nchunks, "moments buffer must use the backward chunk count");
             const unsigned grid = unsigned(tile_grid(tl.map));
-            with_tiling<T, CL_BWD_VEC_MULT>(tl, [&](auto vc, auto lc) {
-                k_moments<T, decltype(vc)::value, decltype(lc)::value><<<grid, 256, 0, s>>>(
+            with_tiling<T>(tl, [&](auto vc, auto lc, auto tc) {
+                k_moments<T, decltype(vc)::value, decltype(lc)::value, decltype(tc)::value>
+                    <<<grid, 256, 0, s>>>(
                     xs, gys, run_ptr, ab, mom, in_dim, out_dim, num_runs, batch, tl.map);
             });
         }
@@ -1900,7 +1965,7 @@ extern "C" int cl_dense_backward_part(int dtype, const void* x, const void* grad
         using T = scalar_t;
         const bool v = vec_ok<T>(batch);
         CL_ARG(!v || all_aligned({x, grad_y, grad_x}), "row buffers must be 16-byte aligned");
-        const Tiling tl = choose_tiling<T>(batch, in_dim, CL_BWD_VEC_MULT, CL_BWD_LPN, 1);
+        const Tiling tl = choose_tiling<T>(batch, in_dim, CL_BWD_LPN, 1);
         if (moments)
             CL_ARG(nchunks == tl.map.nchunks, "moments buffer must use the backward chunk count");
         const unsigned grid = unsigned(tile_grid(tl.map));
@@ -1912,15 +1977,16 @@ extern "C" int cl_dense_backward_part(int dtype, const void* x, const void* grad
         auto* ic = static_cast<const T*>(inv_coef);
         auto* gxs = static_cast<T*>(grad_x);
         auto* mom = static_cast<T*>(moments);
-        with_tiling<T, CL_BWD_VEC_MULT>(tl, [&](auto vc, auto lc) {
+        with_tiling<T>(tl, [&](auto vc, auto lc, auto tc) {
             constexpr int VEC = decltype(vc)::value, LPN = decltype(lc)::value;
+            constexpr bool TAIL = decltype(tc)::value;
             const size_t lds = size_t(16 / LPN) * (kPartRows + part_slots) * LPN * VEC * sizeof(T);
             if (moments)
-                k_bwd_part<T, VEC, LPN, true, true><<<grid, 256, lds, s>>>(
+                k_bwd_part<T, VEC, LPN, true, true, TAIL><<<grid, 256, lds, s>>>(
                     xs, gys, srec, rec, ic, inv_slot, tile_ptr, trun, tile_loc, num_internal, gxs, mom, in_dim,
                     out_dim, num_runs, batch, int(part_slots), tl.map);
             else
-                k_bwd_part<T, VEC, LPN, true, false><<<grid, 256, lds, s>>>(
+                k_bwd_part<T, VEC, LPN, true, false, TAIL><<<grid, 256, lds, s>>>(
                     xs, gys, srec, rec, ic, inv_slot, tile_ptr, trun, tile_loc, num_internal, gxs, mom, in_dim,
                     out_dim, num_runs, batch, int(part_slots), tl.map);
         });
@@ -1944,7 +2010,7 @@ int backward_rows_impl(int dtype, const void* x, const void* grad_y, const int32
                        const void* probs, const int32_t* run_ptr, void* grad_w, void* grad_x,
                        int64_t in_dim, int64_t out_dim, int64_t num_runs, int64_t batch,
                        int64_t num_gates, uint32_t gy_magic, void* stream,
-                       const FirstArgs* fa = nullptr) {
+                       const FirstArgs* fa = nullptr, bool any_batch = false) {
     if (int rc = check_plan_dims(in_dim, out_dim, batch, num_gates, num_runs)) return rc;
     CL_ARG(num_gates <= 64, "the row backward takes at most 64 slots, got %lld",
            (long long)num_gates);
@@ -1961,15 +2027,17 @@ int backward_rows_impl(int dtype, const void* x, const void* grad_y, const int32
         CL_ARG(fa->G >= 1 && fa->G <= 64, "the first layer has 1 to 64 slots, got %lld",
                (long long)fa->G);
         CL_ARG(fa->in_dim >= 1 && fa->num_runs >= 0, "bad first-layer shape");
-        CL_ARG(aligned(fa->nab, 16) && aligned(fa->x0, 16), "nab and x0 must be 16-byte aligned");
+        CL_ARG(aligned(fa->nab, 16), "nab must be 16-byte aligned");
     }
     hipStream_t s = as_stream(stream);
     CL_DTYPE_SWITCH(dtype, {
         using T = scalar_t;
         constexpr int W = wide_vec<T>();
-        CL_ARG(batch % W == 0 && batch <= 64 * W * 8,
-               "the row backward needs batch %% %d == 0 and batch <= %d", W, 64 * W * 8);
-        CL_ARG(all_aligned({x, grad_y}) && (!grad_x || aligned(grad_x, 16)),
+        const bool tail = !vec_ok<T>(batch);
+        CL_ARG(any_batch || !tail, "the row backward needs batch %% %d == 0", W);
+        CL_ARG(batch >= W && batch <= 64 * W * 8,
+               "the row backward needs a batch in [%d, %d]", W, 64 * W * 8);
+        CL_ARG(tail || all_aligned({x, grad_y, grad_x, fa ? fa->x0 : nullptr}),
                "row buffers must be 16-byte aligned");
         FirstLayer<T> first{};
         if (fa)
@@ -1984,8 +2052,9 @@ int backward_rows_impl(int dtype, const void* x, const void* grad_y, const int32
         const int64_t nblk = ceil_div(ceil_div(in_dim, int64_t(4 / S)), int64_t(kXcds));
         CL_ARG(kXcds * nblk < (int64_t(1) << 31), "too many rows");
         const unsigned grid = unsigned(kXcds * nblk);
-        auto go = [&](auto uc) {
+        auto go_tail = [&](auto uc, auto tc) {
             constexpr int U = decltype(uc)::value;
+            constexpr bool TAIL = decltype(tc)::value;
             auto* xs = static_cast<const T*>(x);
             auto* gys = static_cast<const T*>(grad_y);
             auto* srec = reinterpret_cast<const int4*>(slot_rec);
@@ -1997,28 +2066,32 @@ int backward_rows_impl(int dtype, const void* x, const void* grad_y, const int32
             auto launch = [&](auto gwc, auto pc) {
                 constexpr bool GW = decltype(gwc)::value, HP = decltype(pc)::value;
                 if (S == 4)
-                    k_bwd_rows<T, W, U, GW, HP, false, 4><<<grid, 256, 0, s>>>(
+                    k_bwd_rows<T, W, U, GW, HP, TAIL, false, 4><<<grid, 256, 0, s>>>(
                         xs, gys, srec, rec, ic, gate_seq, pr, run_ptr, gw, gxs, in_dim, out_dim,
                         num_runs, batch, int(num_gates), nblk, gy_magic);
                 else if (S == 2)
-                    k_bwd_rows<T, W, U, GW, HP, false, 2><<<grid, 256, 0, s>>>(
+                    k_bwd_rows<T, W, U, GW, HP, TAIL, false, 2><<<grid, 256, 0, s>>>(
                         xs, gys, srec, rec, ic, gate_seq, pr, run_ptr, gw, gxs, in_dim, out_dim,
                         num_runs, batch, int(num_gates), nblk, gy_magic);
                 else
-                    k_bwd_rows<T, W, U, GW, HP><<<grid, 256, 0, s>>>(
+                    k_bwd_rows<T, W, U, GW, HP, TAIL><<<grid, 256, 0, s>>>(
                         xs, gys, srec, rec, ic, gate_seq, pr, run_ptr, gw, gxs, in_dim, out_dim,
                         num_runs, batch, int(num_gates), nblk, gy_magic);
             };
             using Y = std::true_type;
             using N = std::false_type;
             if (fa)
-                k_bwd_rows<T, W, U, true, true, true>
+                k_bwd_rows<T, W, U, true, true, TAIL, true>
                     <<<grid, 256, 0, s>>>(xs, gys, srec, rec, ic, gate_seq, pr, run_ptr, gw,
                                           nullptr, in_dim, out_dim, num_runs, batch,
                                           int(num_gates), nblk, gy_magic, first);
             else if (grad_w && probs) launch(Y{}, Y{});
             else if (grad_w) launch(Y{}, N{});
             else launch(N{}, N{});
+        };
+        auto go = [&](auto uc) {
+            if (tail) go_tail(uc, std::true_type{});
+            else go_tail(uc, std::false_type{});
         };
         const int64_t per_u = 64 * W;
         if (batch <= per_u) go(std::integral_constant<int, 1>{});
@@ -2057,6 +2130,33 @@ extern "C" int cl_dense_backward_rows(int dtype, const void* x, const void* grad
                               num_gates, 0, stream);
 }
 
+extern "C" int cl_dense_backward_rows_first_any(
+    int dtype, const void* x, const void* grad_y, const int32_t* slot_rec,
+    const int32_t* inv_rec, const void* inv_coef, const uint8_t* gate_seq, const void* probs,
+    const int32_t* run_ptr, void* grad_w, int64_t in_dim, int64_t out_dim, int64_t num_runs,
+    int64_t batch, int64_t num_gates, const void* x0, int64_t in0_dim, const int32_t* nab0,
+    int64_t num_runs0, const uint8_t* gate_seq0, const void* probs0, void* grad_w0,
+    int64_t num_gates0, void* stream) {
+    clear_error();
+    const FirstArgs fa{x0, nab0, gate_seq0, probs0, grad_w0, in0_dim, num_runs0, num_gates0};
+    return backward_rows_impl(dtype, x, grad_y, slot_rec, inv_rec, inv_coef, gate_seq, probs,
+                              run_ptr, grad_w, nullptr, in_dim, out_dim, num_runs, batch,
+                              num_gates, 0, stream, &fa, true);
+}
+
+extern "C" int cl_dense_backward_rows_any(int dtype, const void* x, const void* grad_y,
+                                          const int32_t* slot_rec, const int32_t* inv_rec,
+                                          const void* inv_coef, const uint8_t* gate_seq,
+                                          const void* probs, const int32_t* run_ptr, void* grad_w,
+                                          void* grad_x, int64_t in_dim, int64_t out_dim,
+                                          int64_t num_runs, int64_t batch, int64_t num_gates,
+                                          void* stream) {
+    clear_error();
+    return backward_rows_impl(dtype, x, grad_y, slot_rec, inv_rec, inv_coef, gate_seq, probs,
+                              run_ptr, grad_w, grad_x, in_dim, out_dim, num_runs, batch,
+                              num_gates, 0, stream, nullptr, true);
+}
+
 // ------------------------------------------------------------------------------------------
 // The classifier head: the last dense layer, GroupSum(k, tau) and the mean cross-entropy in
 // one autograd step.  The forward runs the fused forward kernel in its HEAD mode (the layer's
@@ -2076,7 +2176,7 @@ struct HeadShape {
 
 template <typename T>
 bool head_shape(int64_t out_dim, int64_t batch, int64_t k, HeadShape& h) {
-    h.tl = choose_tiling<T>(batch, out_dim, CL_FUSED_VEC_MULT, CL_FWD_LPN, CL_FWD_NPG);
+    h.tl = choose_tiling<T>(batch, out_dim, CL_FWD_LPN, CL_FWD_NPG, false);
     h.tile_rows = int64_t(256 / h.tl.lpn) * CL_FWD_NPG;
     h.gsz = ceil_div(out_dim, k);
     h.part_elems = h.tl.map.ntiles * 2 * batch;
@@ -2139,9 +2239,9 @@ extern "C" int cl_dense_group_sum_cross_entropy_forward(
         T* slices = part + h.part_elems;
         T* term = slices + h.slice_elems;
         const unsigned grid = unsigned(tile_grid(h.tl.map));
-        with_tiling<T, CL_FUSED_VEC_MULT>(h.tl, [&](auto vc, auto lc) {
+        with_tiling<T>(h.tl, [&](auto vc, auto lc, auto) {
             constexpr int VEC = decltype(vc)::value, LPN = decltype(lc)::value;
-            k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, true, true><<<grid, 256, 0, s>>>(
+            k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, true, true, false><<<grid, 256, 0, s>>>(
                 static_cast<const T*>(x), static_cast<const T*>(w), softmax, gate_seq,
                 reinterpret_cast<const int4*>(nab), inv_pos, static_cast<T*>(probs),
                 static_cast<T*>(inv_coef), nullptr, in_dim, out_dim, num_runs, batch,

@@ -196,12 +196,9 @@ class LogicLayerRunsFunction(torch.autograd.Function):
         stream = _dl.stream_of(x)
         batch = x.shape[1]
         with torch.cuda.device(x.device):
-            wide = 16 // x.element_size()
-            if (need_x and LogicLayerRunsFunction.row_backward and plan.single_run
-                    and plan.num_gates <= 64 and 0 < batch <= 64 * wide * 8
-                    and batch % wide == 0):
+            if need_x and LogicLayerRunsFunction.row_backward and _row_backward_fits(plan, x):
                 timing.timed(f"cl_dense_backward_rows[{plan.in_dim}->{plan.out_dim}]", lambda: _capi.call(
-                    "cl_dense_backward_rows", code, x.data_ptr(), grad_y.data_ptr(),
+                    _rows_entry("cl_dense_backward_rows", x), code, x.data_ptr(), grad_y.data_ptr(),
                     plan.slot_rec.data_ptr(), plan.inv_rec.data_ptr(), inv_coef.data_ptr(),
                     gate_sequence.data_ptr(), _dl.ptr(probs), plan.run_ptr.data_ptr(),
                     _dl.ptr(grad_w), grad_x.data_ptr(), plan.in_dim, plan.out_dim,
@@ -253,8 +250,13 @@ def _row_backward_fits(plan: RunPlan, x: torch.Tensor) -> bool:
     """Whether cl_dense_backward_rows takes this layer at this batch (x: [in_dim, batch])."""
     wide = 16 // x.element_size()
     batch = x.shape[1]
-    return (plan.single_run and plan.num_gates <= 64 and 0 < batch <= 64 * wide * 8
-            and batch % wide == 0)
+    return plan.single_run and plan.num_gates <= 64 and wide <= batch <= 64 * wide * 8
+
+
+def _rows_entry(name: str, x: torch.Tensor) -> str:
+    """The entry point of a row backward for x's batch: `name` itself takes multiples of the
+    16-byte vector only."""
+    return name + "_any" if x.shape[1] % (16 // x.element_size()) else name
 
 
 class LogicLayerFirstPairFunction(torch.autograd.Function):
@@ -294,7 +296,7 @@ class LogicLayerFirstPairFunction(torch.autograd.Function):
         grad_w1 = torch.empty((plan1.out_dim, plan1.num_gates), dtype=y1.dtype, device=dev)
         with torch.cuda.device(dev):
             timing.timed(f"cl_dense_backward_rows_first[{plan2.in_dim}->{plan2.out_dim}]", lambda: _capi.call(
-                "cl_dense_backward_rows_first", _dl.dtype_code(y1), y1.data_ptr(),
+                _rows_entry("cl_dense_backward_rows_first", y1), _dl.dtype_code(y1), y1.data_ptr(),
                 grad_y.data_ptr(), plan2.slot_rec.data_ptr(), plan2.inv_rec.data_ptr(),
                 inv_coef.data_ptr(), gs2.data_ptr(), probs2.data_ptr(), plan2.run_ptr.data_ptr(),
                 grad_w2.data_ptr(), plan2.in_dim, plan2.out_dim, plan2.num_runs, y1.shape[1],

@@ -243,6 +243,25 @@ int cl_dense_backward_rows_first(int dtype, const void* x, const void* grad_y,
                                  const uint8_t* gate_seq0, const void* probs0, void* grad_w0,
                                  int64_t num_gates0, void* stream);
 
+/* The two row backwards for any batch of 16 / sizeof(T) to 64 * 8 * (16 / sizeof(T)) samples (4
+ * to 2048 in fp32); the row buffers need 16-byte alignment only when batch is a multiple of
+ * 16 / sizeof(T). */
+int cl_dense_backward_rows_any(int dtype, const void* x, const void* grad_y,
+                               const int32_t* slot_rec, const int32_t* inv_rec,
+                               const void* inv_coef, const uint8_t* gate_seq, const void* probs,
+                               const int32_t* run_ptr, void* grad_w, void* grad_x,
+                               int64_t in_dim, int64_t out_dim, int64_t num_runs, int64_t batch,
+                               int64_t num_gates, void* stream);
+int cl_dense_backward_rows_first_any(int dtype, const void* x, const void* grad_y,
+                                 const int32_t* slot_rec, const int32_t* inv_rec,
+                                 const void* inv_coef, const uint8_t* gate_seq,
+                                 const void* probs, const int32_t* run_ptr, void* grad_w,
+                                 int64_t in_dim, int64_t out_dim, int64_t num_runs,
+                                 int64_t batch, int64_t num_gates, const void* x0,
+                                 int64_t in0_dim, const int32_t* nab0, int64_t num_runs0,
+                                 const uint8_t* gate_seq0, const void* probs0, void* grad_w0,
+                                 int64_t num_gates0, void* stream);
+
 /* Weight gradient from the moments: grad_w[o, g] = (c0, c1, c2, c3)[gate_seq[o,g]] . (moments
  * of g's run summed over the chunks in chunk order); with `probs` (not NULL) followed by the
  * softmax backward, giving the gradient of the logits. */

@@ -520,3 +520,37 @@ def test_row_backward_entry_point_checks(device):
     multi = (plan.run_ptr[1:] - plan.run_ptr[:-1]) != 1
     assert bool(multi.any())
     assert torch.isnan(gw[multi]).all() and not torch.isnan(gw[~multi]).any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 7, 15, 63, 65, 127, 253, 257, 1021, 1023, 1025,
+                                   2047, 2049, 2051])
+def test_batches_off_the_vector_width(device, dtype, shared, batch):
+    """The module path at batches that are no multiple of a 16-byte vector (rows then start at
+    any element and the last vector overlaps the one before): around the vector, the chunks, a
+    wave's samples per vector and the row backward's largest batch; single- and multi-run
+    neurons, with the input gradient and with the weight gradient alone; every buffer ends with
+    its allocation."""
+    in_dim, out_dim, g_n = 37, 70, 16
+    L = make_layer(batch, in_dim, out_dim, g_n, batch, shared)
+    logits = np.log(L["w"])
+    layer = cl.LogicLayer(in_dim, out_dim, num_gates=g_n).to(device=device, dtype=dtype)
+    with torch.no_grad():
+        layer.weights.copy_(torch.as_tensor(logits))
+        layer.indices.copy_(torch.as_tensor(np.stack([L["a"], L["b"]])))
+        layer.gate_sequence.copy_(torch.as_tensor(L["gs"]))
+    layer.refresh_backward_index()
+    gy = torch.as_tensor(L["gy"]).to(device=device, dtype=dtype).t()
+    ref_y = O.dense_forward(L["x"], L["a"], L["b"], L["w"], L["gs"])
+    ref_p = O.dense_backward_w(L["x"], L["a"], L["b"], L["gs"], L["gy"])
+    ref_gw = L["w"] * (ref_p - (L["w"] * ref_p).sum(1, keepdims=True))
+    ref_gx = O.dense_backward_x_direct(L["x"], L["a"], L["b"], L["w"], L["gs"], L["gy"])
+    for need_x in (True, False):
+        x = torch.as_tensor(L["x"]).to(device=device, dtype=dtype).t().requires_grad_(need_x)
+        y = layer(x)
+        np.testing.assert_allclose(np_(y).T, ref_y, **TOL[dtype])
+        got = torch.autograd.grad(y, ([x] if need_x else []) + [layer.weights], gy)
+        np.testing.assert_allclose(np_(got[-1]), ref_gw, **TOL[dtype])
+        if need_x:
+            np.testing.assert_allclose(np_(got[0]).T, ref_gx, **TOL[dtype])

@@ -41,6 +41,10 @@ def grads(model, x, labels, pair: bool):
     ([(64, 256), (256, 320), (320, 300)], 10, 256, torch.float32),
     ([(100, 400), (400, 800)], 8, 64, torch.float64),
     ([(30, 90), (90, 200), (200, 120)], 4, 2048, torch.float32),
+    # batches off the vector width
+    ([(64, 256), (256, 640)], 10, 1023, torch.float32),
+    ([(30, 90), (90, 200)], 4, 5, torch.float32),
+    ([(100, 400), (400, 800)], 8, 129, torch.float64),
 ])
 def test_pair_gradients_are_bitwise_the_unpaired_ones(device, dims, k, batch, dtype):
     model = net(device, dims, k, dtype, seed=batch)
