@@ -45,6 +45,9 @@ SIGNATURES: dict[str, list] = {
                                _i64, _i64, _p],
     "cl_dense_backward_rows_any": [_int, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64,
                                _i64, _i64, _p],
+    "cl_dense_forward_fused_half": [_p] * 8 + [_i64] * 5 + [_p],
+    "cl_dense_backward_rows_half": [_p] * 10 + [_i64] * 5 + [_p],
+    "cl_dense_weight_grad_half": [_p] * 8 + [_i64] * 5 + [_p],
     "cl_transpose": [_int, _p, _p, _i64, _i64, _p],
     "cl_tree_conv_forward": [_int, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _int, _int, _int,
                              _int, _int, _int, _int, _p, _p, _p, _p, _p],

@@ -71,6 +71,27 @@ __device__ __forceinline__ void vstr(T* p, V v) {
     }
 }
 
+// Rows stored as S (T itself, or half with T = float: widened on load, rounded once on store).
+// A half lane then holds eight samples in one 16-byte access and everything between the
+// loads and the store is the fp32 kernel's arithmetic.
+template <bool TAIL, typename S, typename T, int VEC>
+__device__ __forceinline__ typename VT<T, VEC>::type ldrow(const S* p) {
+    using V = typename VT<T, VEC>::type;
+    if constexpr (std::is_same<S, T>::value)
+        return vldr<TAIL, T, V>(p);
+    else
+        return __builtin_convertvector((vldr<TAIL, S, typename VT<S, VEC>::type>(p)), V);
+}
+
+template <bool TAIL, typename S, typename T, int VEC>
+__device__ __forceinline__ void strow(S* p, typename VT<T, VEC>::type v) {
+    if constexpr (std::is_same<S, T>::value)
+        vstr<TAIL, T, typename VT<T, VEC>::type>(p, v);
+    else
+        vstr<TAIL, S, typename VT<S, VEC>::type>(
+            p, __builtin_convertvector(v, typename VT<S, VEC>::type));
+}
+
 // Where the lane whose vector starts at sample idx < B reads and writes its row.
 template <bool TAIL, int VEC>
 __device__ __forceinline__ int64_t tail_off(int64_t idx, int64_t B) {
@@ -488,13 +509,13 @@ __device__ __forceinline__ T fused_rcp(T v) {
 // the tile's first row, and the next class), the tile's lane groups add theirs in LDS in row
 // order, and the tile writes part[(t * 2 + slot) * B + n]; a tile spans at most two classes
 // (gsz >= 256 / LPN * NPG rows, checked by the host).
-template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD, bool TAIL>
-__device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T* __restrict__ w,
+template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD, bool TAIL, typename S>
+__device__ __forceinline__ void fwd_fused_tile(const S* __restrict__ x, const T* __restrict__ w,
                                                int softmax, const uint8_t* __restrict__ gs,
                                                const int4* __restrict__ nab,
                                                const int32_t* __restrict__ inv_pos,
                                                T* __restrict__ probs, T* __restrict__ inv_coef,
-                                               T* __restrict__ y, int64_t in_dim, int64_t out_dim,
+                                               S* __restrict__ y, int64_t in_dim, int64_t out_dim,
                                                int64_t num_runs, int64_t B, int G,
                                                const TileMap& tm, int64_t c, int64_t t,
                                                T* __restrict__ part, int64_t gsz,
@@ -539,8 +560,8 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
     for (int j = 0; j < NPG; ++j) {
         ok[j] = live[j] && rec[j].z >= 0 && rec[j].w == rec[j].z + 1 && rec[j].w <= num_runs &&
                 uint32_t(rec[j].x) < uint64_t(in_dim) && uint32_t(rec[j].y) < uint64_t(in_dim);
-        va[j] = vldr<TAIL, T, V>(x + int64_t(ok[j] ? rec[j].x : 0) * B + off);
-        vb[j] = vldr<TAIL, T, V>(x + int64_t(ok[j] ? rec[j].y : 0) * B + off);
+        va[j] = ldrow<TAIL, S, T, VEC>(x + int64_t(ok[j] ? rec[j].x : 0) * B + off);
+        vb[j] = ldrow<TAIL, S, T, VEC>(x + int64_t(ok[j] ? rec[j].y : 0) * B + off);
         // entry positions of the run's two sides, for the tile's writer chunk
         if constexpr (COEF) {
             const int64_t rz = ok[j] ? rec[j].z : 0;
@@ -622,7 +643,7 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
                 if (o < bound) h0 += acc;
                 else h1 += acc;
             } else {
-                vstr<TAIL, T, V>(y + o * B + off, acc);
+                strow<TAIL, S, T, VEC>(y + o * B + off, acc);
             }
         }
     }
@@ -651,20 +672,21 @@ __device__ __forceinline__ void fwd_fused_tile(const T* __restrict__ x, const T*
     }
 }
 
-template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD, bool TAIL>
-__global__ __launch_bounds__(256) void k_fwd_fused(const T* __restrict__ x, const T* __restrict__ w,
+template <typename T, int VEC, int LPN, int NPG, bool COEF, bool HEAD, bool TAIL,
+          typename S = T>
+__global__ __launch_bounds__(256) void k_fwd_fused(const S* __restrict__ x, const T* __restrict__ w,
                                                    int softmax, const uint8_t* __restrict__ gs,
                                                    const int4* __restrict__ nab,
                                                    const int32_t* __restrict__ inv_pos,
                                                    T* __restrict__ probs, T* __restrict__ inv_coef,
-                                                   T* __restrict__ y, int64_t in_dim,
+                                                   S* __restrict__ y, int64_t in_dim,
                                                    int64_t out_dim, int64_t num_runs, int64_t B,
                                                    int G, TileMap tm, T* __restrict__ part,
                                                    int64_t gsz) {
     __shared__ T red[HEAD ? 2 * 256 * VEC : 1];
     int64_t c, t;
     if (map_tile(tm, blockIdx.x, c, t))  // uniform per workgroup
-        fwd_fused_tile<T, VEC, LPN, NPG, COEF, HEAD, TAIL>(x, w, softmax, gs, nab, inv_pos, probs,
+        fwd_fused_tile<T, VEC, LPN, NPG, COEF, HEAD, TAIL, S>(x, w, softmax, gs, nab, inv_pos, probs,
                                                      inv_coef, y, in_dim, out_dim, num_runs, B,
                                                      G, tm, c, t, part, gsz, red);
 }
@@ -825,9 +847,9 @@ __global__ __launch_bounds__(256) void k_wgrad_full(const T* __restrict__ x, con
 // unconditional (clamped, masked afterwards) so they are in flight together, and run o's
 // pair is fetched with run_ptr[o]: in a layer of single-run neurons run o is neuron o's
 // only run, and its row gathers need no second round trip.
-template <typename T, int VEC, int U, bool HAS_P, bool TAIL>
-__global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
-                                                    const T* __restrict__ gy,
+template <typename T, int VEC, int U, bool HAS_P, bool TAIL, typename S = T>
+__global__ __launch_bounds__(256) void k_wgrad_rows(const S* __restrict__ x,
+                                                    const S* __restrict__ gy,
                                                     const uint8_t* __restrict__ gs,
                                                     const T* __restrict__ probs,
                                                     const int32_t* __restrict__ run_ptr,
@@ -847,7 +869,7 @@ __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
     for (int u = 0; u < U; ++u) {
         const int64_t idx = int64_t(u * 64 + lane) * VEC;
         off[u] = idx < B ? tail_off<TAIL, VEC>(idx, B) : 0;
-        vg[u] = vldr<TAIL, T, V>(gy + o * B + off[u]);
+        vg[u] = ldrow<TAIL, S, T, VEC>(gy + o * B + off[u]);
     }
     const int gl = lane < G ? lane : 0;
     const int code = gs[o * G + gl];
@@ -885,8 +907,8 @@ __global__ __launch_bounds__(256) void k_wgrad_rows(const T* __restrict__ x,
         V va[U], vb[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            va[u] = vldr<TAIL, T, V>(x + int64_t(ab.x) * B + off[u]);
-            vb[u] = vldr<TAIL, T, V>(x + int64_t(ab.y) * B + off[u]);
+            va[u] = ldrow<TAIL, S, T, VEC>(x + int64_t(ab.x) * B + off[u]);
+            vb[u] = ldrow<TAIL, S, T, VEC>(x + int64_t(ab.y) * B + off[u]);
         }
         T m1, m2, m3;
         run_moments<T, VEC, U>(vg, va, vb, m1, m2, m3);
@@ -1244,8 +1266,10 @@ __global__ __launch_bounds__(256) void k_bwd_part(
 #ifndef CL_FIRST_EPI4
 #define CL_FIRST_EPI4 1
 #endif
-template <typename T, int U, bool FIRST = false>
-constexpr int bwd_rows_waves() { return sizeof(T) == 4 && U <= 4 ? (FIRST ? CL_FIRST_WAVES : 4) : 1; }
+template <typename T, int ELEMS, bool FIRST = false>
+constexpr int bwd_rows_waves() {
+    return sizeof(T) == 4 && ELEMS <= 16 ? (FIRST ? CL_FIRST_WAVES : 4) : 1;
+}
 
 #ifndef CL_BWD_ROWS_EPI4
 #define CL_BWD_ROWS_EPI4 2
@@ -1274,20 +1298,21 @@ struct FirstLayer {
 // [deg * part / S, deg * (part + 1) / S); the parts' input-gradient sums meet in LDS and are
 // added in part order (deterministic; the association differs from S = 1 by rounding).
 template <typename T, int VEC, int U, bool WANT_GW, bool HAS_P, bool TAIL, bool FIRST = false,
-          int S = 1>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_rows_waves<T, U, FIRST>())))
+          int S = 1, typename ST = T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(bwd_rows_waves<T, VEC * U, FIRST>())))
 void k_bwd_rows(
-    const T* __restrict__ x, const T* __restrict__ gy, const int4* __restrict__ slot_rec,
+    const ST* __restrict__ x, const ST* __restrict__ gy, const int4* __restrict__ slot_rec,
     const int4* __restrict__ inv_rec, const T* __restrict__ inv_coef,
     const uint8_t* __restrict__ gs, const T* __restrict__ probs,
-    const int32_t* __restrict__ run_ptr, T* __restrict__ grad_w, T* __restrict__ gx,
+    const int32_t* __restrict__ run_ptr, T* __restrict__ grad_w, ST* __restrict__ gx,
     int64_t in_dim, int64_t out_dim, int64_t num_runs, int64_t B, int G, int64_t nblk,
     uint32_t gy_magic, FirstLayer<T> first = {}) {
     static_assert(S == 1 || S == 2 || S == 4, "1, 2 or 4 waves per row");
     static_assert(S == 1 || !FIRST, "the first-layer mode takes one wave per row");
     using V = typename VT<T, VEC>::type;
     using V2 = typename VT<T, 2>::type;
-    constexpr int EPI = U <= 2 ? 2 : U <= 4 ? (FIRST || TAIL ? CL_FIRST_EPI4 : CL_BWD_ROWS_EPI4) : 1;
+    constexpr int L = sizeof(T) == 4 ? VEC * U / 4 : U;  // 16-byte registers per row and lane
+    constexpr int EPI = L <= 2 ? 2 : L <= 4 ? (FIRST || TAIL ? CL_FIRST_EPI4 : CL_BWD_ROWS_EPI4) : 1;
     const int lane = threadIdx.x & 63;
     const int64_t w = blockIdx.x;
     const int wv = wave_id();
@@ -1323,7 +1348,7 @@ void k_bwd_rows(
     for (int u = 0; u < U; ++u) {
         acc[u] = V(T(0));
         xi[u] = V(T(0));
-        if constexpr (WANT_GW) xi[u] = vldr<TAIL, T, V>(x + row * B + off[u]);
+        if constexpr (WANT_GW) xi[u] = ldrow<TAIL, ST, T, VEC>(x + row * B + off[u]);
     }
     const int gl = lane < G ? lane : 0;  // slot of this lane in the finalize (clamped)
     bool bad = false;
@@ -1362,8 +1387,8 @@ void k_bwd_rows(
                                          : int64_t(cur[q].x);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                vo[q][u] = vldr<TAIL, T, V>(x + int64_t(cur[q].y) * B + off[u]);
-                vg[q][u] = vldr<TAIL, T, V>(gy + gyr * B + off[u]);
+                vo[q][u] = ldrow<TAIL, ST, T, VEC>(x + int64_t(cur[q].y) * B + off[u]);
+                vg[q][u] = ldrow<TAIL, ST, T, VEC>(gy + gyr * B + off[u]);
             }
             // the finalize's per-neuron data is loaded with the rows, not after the moments
             if constexpr (WANT_GW) {
@@ -1463,7 +1488,7 @@ void k_bwd_rows(
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (in[u]) vstr<TAIL, T, V>(gx + row * B + off[u], bad ? V(nan_of<T>()) : acc[u]);
+            if (in[u]) strow<TAIL, ST, T, VEC>(gx + row * B + off[u], bad ? V(nan_of<T>()) : acc[u]);
     }
 }
 
@@ -2083,7 +2108,7 @@ int backward_rows_impl(int dtype, const void* x, const void* grad_y, const int32
             if (fa)
                 k_bwd_rows<T, W, U, true, true, TAIL, true>
                     <<<grid, 256, 0, s>>>(xs, gys, srec, rec, ic, gate_seq, pr, run_ptr, gw,
-                                          nullptr, in_dim, out_dim, num_runs, batch,
+                                          static_cast<T*>(nullptr), in_dim, out_dim, num_runs, batch,
                                           int(num_gates), nblk, gy_magic, first);
             else if (grad_w && probs) launch(Y{}, Y{});
             else if (grad_w) launch(Y{}, N{});
@@ -2155,6 +2180,143 @@ extern "C" int cl_dense_backward_rows_any(int dtype, const void* x, const void* 
     return backward_rows_impl(dtype, x, grad_y, slot_rec, inv_rec, inv_coef, gate_seq, probs,
                               run_ptr, grad_w, grad_x, in_dim, out_dim, num_runs, batch,
                               num_gates, 0, stream, nullptr, true);
+}
+
+// ------------------------------------------------------------------------------------------
+// Half rows (x, y and their gradients) with fp32 logits: the fused forward, the row backward
+// and the weight gradient of single-run neurons on half storage.  The reference-interface
+// kernels they stand in for walk the 16 slots of every inverse-index entry, round the
+// softmax to half first and return its gradient in half.  12000 -> 12000 at batch 1024: forward
+// 17 -> 13 us, input and weight gradient 140 + 23 -> 22 us (a launch of 73.7 MB each way of the
+// layer at 3.3 TB/s, bound by the rows in flight as the fp32 kernel), error against 64 bits
+// 3.7e-4 -> 2.2e-4.  Batches of up to 2048 samples, whose rows a wave's registers hold.
+namespace {
+using Half = _Float16;
+constexpr int kHalfVec = 8;
+constexpr int64_t kHalfMaxBatch = 64 * kHalfVec * 4;
+
+int check_half(int64_t batch, int64_t num_gates) {
+    CL_ARG(num_gates <= 16, "the half kernels take at most 16 slots, got %lld",
+           (long long)num_gates);
+    CL_ARG(batch >= kHalfVec && batch <= kHalfMaxBatch, "the half kernels need a batch in [%d, %lld]",
+           kHalfVec, (long long)kHalfMaxBatch);
+    return CL_OK;
+}
+
+template <typename F>
+void half_units(int64_t batch, F&& f) {
+    auto by_tail = [&](auto uc) {
+        if (batch % kHalfVec) f(uc, std::true_type{});
+        else f(uc, std::false_type{});
+    };
+    if (batch <= 64 * kHalfVec) by_tail(std::integral_constant<int, 1>{});
+    else if (batch <= 2 * 64 * kHalfVec) by_tail(std::integral_constant<int, 2>{});
+    else by_tail(std::integral_constant<int, 4>{});
+}
+}  // namespace
+
+extern "C" int cl_dense_forward_fused_half(const void* x, const float* w, const uint8_t* gate_seq,
+                                           const int32_t* nab, const int32_t* inv_pos,
+                                           float* probs, float* inv_coef, void* y, int64_t in_dim,
+                                           int64_t out_dim, int64_t num_runs, int64_t batch,
+                                           int64_t num_gates, void* stream) {
+    clear_error();
+    if (int rc = check_plan_dims(in_dim, out_dim, batch, num_gates, num_runs)) return rc;
+    if (int rc = check_half(batch, num_gates)) return rc;
+    if (out_dim == 0) return CL_OK;
+    CL_ARG(in_dim > 0 && num_runs >= 1, "in_dim and num_runs must be >= 1 when out_dim > 0");
+    CL_ARG(x && w && gate_seq && nab && inv_pos && probs && inv_coef && y,
+           "null pointer argument");
+    CL_ARG(aligned(nab, 16), "nab misaligned");
+    CL_ARG(batch % kHalfVec || all_aligned({x, y}), "x and y must be 16-byte aligned");
+    const Tiling tl = choose_tiling<Half>(batch, out_dim, CL_FWD_LPN, CL_FWD_NPG);
+    const unsigned grid = unsigned(tile_grid(tl.map));
+    auto launch = [&](auto lc, auto tc) {
+        k_fwd_fused<float, kHalfVec, decltype(lc)::value, CL_FWD_NPG, true, false,
+                    decltype(tc)::value, Half><<<grid, 256, 0, as_stream(stream)>>>(
+            static_cast<const Half*>(x), w, 1, gate_seq, reinterpret_cast<const int4*>(nab),
+            inv_pos, probs, inv_coef, static_cast<Half*>(y), in_dim, out_dim, num_runs, batch,
+            int(num_gates), tl.map, nullptr, 0);
+    };
+    auto by_tail = [&](auto lc) {
+        if (tl.tail) launch(lc, std::true_type{});
+        else launch(lc, std::false_type{});
+    };
+    if (tl.lpn == 16) by_tail(std::integral_constant<int, 16>{});
+    else if (tl.lpn == 8) by_tail(std::integral_constant<int, 8>{});
+    else by_tail(std::integral_constant<int, 4>{});
+    return check_launch("cl_dense_forward_fused_half");
+}
+
+extern "C" int cl_dense_backward_rows_half(const void* x, const void* grad_y,
+                                           const int32_t* slot_rec, const int32_t* inv_rec,
+                                           const float* inv_coef, const uint8_t* gate_seq,
+                                           const float* probs, const int32_t* run_ptr,
+                                           float* grad_w, void* grad_x, int64_t in_dim,
+                                           int64_t out_dim, int64_t num_runs, int64_t batch,
+                                           int64_t num_gates, void* stream) {
+    clear_error();
+    if (int rc = check_plan_dims(in_dim, out_dim, batch, num_gates, num_runs)) return rc;
+    if (int rc = check_half(batch, num_gates)) return rc;
+    if (in_dim == 0) return CL_OK;
+    CL_ARG(x && grad_y && slot_rec && inv_rec && inv_coef && grad_x, "null pointer argument");
+    CL_ARG(!grad_w || (gate_seq && run_ptr && probs), "grad_w needs gate_seq, run_ptr and probs");
+    CL_ARG(aligned(slot_rec, 16) && aligned(inv_rec, 16) && aligned(inv_coef, 8),
+           "slot_rec / inv_rec must be 16-byte aligned, inv_coef 8-byte aligned");
+    CL_ARG(batch % kHalfVec || all_aligned({x, grad_y, grad_x}),
+           "row buffers must be 16-byte aligned");
+    const int64_t avg = 2 * num_runs / in_dim;
+    const int S = avg >= CL_BWD_ROWS_S4 ? 4 : avg >= CL_BWD_ROWS_S2 ? 2 : 1;
+    const int64_t nblk = ceil_div(ceil_div(in_dim, int64_t(4 / S)), int64_t(kXcds));
+    CL_ARG(kXcds * nblk < (int64_t(1) << 31), "too many rows");
+    const unsigned grid = unsigned(kXcds * nblk);
+    half_units(batch, [&](auto uc, auto tc) {
+        constexpr int U = decltype(uc)::value;
+        constexpr bool TAIL = decltype(tc)::value;
+        auto launch = [&](auto gwc, auto sc) {
+            constexpr bool GW = decltype(gwc)::value;
+            k_bwd_rows<float, kHalfVec, U, GW, GW, TAIL, false, decltype(sc)::value, Half>
+                <<<grid, 256, 0, as_stream(stream)>>>(
+                    static_cast<const Half*>(x), static_cast<const Half*>(grad_y),
+                    reinterpret_cast<const int4*>(slot_rec),
+                    reinterpret_cast<const int4*>(inv_rec), inv_coef, gate_seq, probs, run_ptr,
+                    grad_w, static_cast<Half*>(grad_x), in_dim, out_dim, num_runs, batch,
+                    int(num_gates), nblk, 0, FirstLayer<float>{});
+        };
+        auto by_share = [&](auto gwc) {
+            if (S == 4) launch(gwc, std::integral_constant<int, 4>{});
+            else if (S == 2) launch(gwc, std::integral_constant<int, 2>{});
+            else launch(gwc, std::integral_constant<int, 1>{});
+        };
+        if (grad_w) by_share(std::true_type{});
+        else by_share(std::false_type{});
+    });
+    return check_launch("cl_dense_backward_rows_half");
+}
+
+extern "C" int cl_dense_weight_grad_half(const void* x, const void* grad_y,
+                                         const uint8_t* gate_seq, const float* probs,
+                                         const int32_t* run_ptr, const int32_t* run_ab,
+                                         const int32_t* run_gl, float* grad_w, int64_t in_dim,
+                                         int64_t out_dim, int64_t num_runs, int64_t batch,
+                                         int64_t num_gates, void* stream) {
+    clear_error();
+    if (int rc = check_plan_dims(in_dim, out_dim, batch, num_gates, num_runs)) return rc;
+    if (int rc = check_half(batch, num_gates)) return rc;
+    if (out_dim == 0) return CL_OK;
+    CL_ARG(x && grad_y && gate_seq && probs && run_ptr && run_ab && run_gl && grad_w,
+           "null pointer argument");
+    CL_ARG(aligned(run_ab, 8), "run_ab misaligned");
+    CL_ARG(in_dim >= 1 && num_runs >= 1, "in_dim and num_runs must be >= 1 when out_dim > 0");
+    CL_ARG(batch % kHalfVec || all_aligned({x, grad_y}), "x and grad_y must be 16-byte aligned");
+    half_units(batch, [&](auto uc, auto tc) {
+        k_wgrad_rows<float, kHalfVec, decltype(uc)::value, true, decltype(tc)::value, Half>
+            <<<unsigned(ceil_div(out_dim, int64_t(4))), 256, 0, as_stream(stream)>>>(
+                static_cast<const Half*>(x), static_cast<const Half*>(grad_y), gate_seq, probs,
+                run_ptr, reinterpret_cast<const int2*>(run_ab), run_gl, grad_w, in_dim, out_dim,
+                num_runs, batch, int(num_gates));
+    });
+    return check_launch("cl_dense_weight_grad_half");
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2244,8 +2406,8 @@ extern "C" int cl_dense_group_sum_cross_entropy_forward(
             k_fwd_fused<T, VEC, LPN, CL_FWD_NPG, true, true, false><<<grid, 256, 0, s>>>(
                 static_cast<const T*>(x), static_cast<const T*>(w), softmax, gate_seq,
                 reinterpret_cast<const int4*>(nab), inv_pos, static_cast<T*>(probs),
-                static_cast<T*>(inv_coef), nullptr, in_dim, out_dim, num_runs, batch,
-                int(num_gates), h.tl.map, part, h.gsz);
+                static_cast<T*>(inv_coef), static_cast<T*>(nullptr), in_dim, out_dim, num_runs,
+                batch, int(num_gates), h.tl.map, part, h.gsz);
         });
         if (int rc = check_launch("cl_dense_group_sum_cross_entropy_forward(layer)")) return rc;
         return ce_from_tile_partials(dtype, part, batch, out_dim, k, h.tile_rows, tau, labels,

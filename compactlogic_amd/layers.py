@@ -306,6 +306,64 @@ class LogicLayerFirstPairFunction(torch.autograd.Function):
         return None, grad_w2, None, None, grad_w1, None, None, None, None
 
 
+# Batches the half module path takes (cl_dense_forward_fused_half): one 16-byte vector of
+# samples to what a wave's registers hold.
+_HALF_BATCH = (8, 2048)
+
+
+class LogicLayerHalfFunction(torch.autograd.Function):
+    """LogicLayerRunsFunction on float16 rows with fp32 logits, for layers of single-run neurons
+    of at most 16 slots (the softmax inside, all sums and the logits gradient fp32, rows rounded
+    once on store).  The reference-interface kernels, which other half layers train through,
+    take the softmax rounded to half and walk every slot of every input's uses: 140 us for the
+    input gradient of a 12000 -> 12000 layer at batch 1024 and 23 us for the weight gradient,
+    where the row backward takes 22 us for both (the forward: 17 and 13 us)."""
+
+    @staticmethod
+    def forward(ctx, x, w, gate_sequence, plan: RunPlan):
+        _dl._check(x, "x")
+        if x.shape[0] != plan.in_dim:
+            raise RuntimeError(f"x has {x.shape[0]} rows, the layer expects {plan.in_dim}")
+        w = w.contiguous()
+        dev = x.device
+        probs = torch.empty_like(w)
+        inv_coef = torch.empty((2 * plan.num_runs, 2), dtype=w.dtype, device=dev)
+        y = torch.empty((plan.out_dim, x.shape[1]), dtype=x.dtype, device=dev)
+        with torch.cuda.device(dev):
+            timing.timed(f"cl_dense_forward_fused_half[{plan.in_dim}->{plan.out_dim}]", lambda: _capi.call(
+                "cl_dense_forward_fused_half", x.data_ptr(), w.data_ptr(),
+                gate_sequence.data_ptr(), plan.nab.data_ptr(), plan.inv_pos.data_ptr(),
+                probs.data_ptr(), inv_coef.data_ptr(), y.data_ptr(), plan.in_dim, plan.out_dim,
+                plan.num_runs, x.shape[1], plan.num_gates, _dl.stream_of(x)))
+        ctx.save_for_backward(x, inv_coef, gate_sequence, probs)
+        ctx.plan = plan
+        return y
+
+    @staticmethod
+    def backward(ctx, grad_y):
+        x, inv_coef, gate_sequence, probs = ctx.saved_tensors
+        plan: RunPlan = ctx.plan
+        grad_y = grad_y.contiguous()
+        need_x, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        grad_x = torch.empty_like(x) if need_x else None
+        grad_w = torch.empty_like(probs) if need_w else None
+        dims = (plan.in_dim, plan.out_dim, plan.num_runs, x.shape[1], plan.num_gates,
+                _dl.stream_of(x))
+        with torch.cuda.device(x.device):
+            if need_x:
+                timing.timed(f"cl_dense_backward_rows_half[{plan.in_dim}->{plan.out_dim}]", lambda: _capi.call(
+                    "cl_dense_backward_rows_half", x.data_ptr(), grad_y.data_ptr(),
+                    plan.slot_rec.data_ptr(), plan.inv_rec.data_ptr(), inv_coef.data_ptr(),
+                    gate_sequence.data_ptr(), probs.data_ptr(), plan.run_ptr.data_ptr(),
+                    _dl.ptr(grad_w), grad_x.data_ptr(), *dims))
+            elif need_w:
+                timing.timed(f"cl_dense_weight_grad_half[{plan.in_dim}->{plan.out_dim}]", lambda: _capi.call(
+                    "cl_dense_weight_grad_half", x.data_ptr(), grad_y.data_ptr(),
+                    gate_sequence.data_ptr(), probs.data_ptr(), plan.run_ptr.data_ptr(),
+                    plan.run_ab.data_ptr(), plan.run_gl.data_ptr(), grad_w.data_ptr(), *dims))
+        return grad_x, grad_w, None, None
+
+
 def _transpose_rows(x: torch.Tensor) -> torch.Tensor:
     """Contiguous [cols, rows] transpose of a contiguous 2-D device tensor [rows, cols]."""
     out = torch.empty((x.shape[1], x.shape[0]), dtype=x.dtype, device=x.device)
@@ -460,8 +518,15 @@ class LogicLayer(torch.nn.Module):
         x = to_rows(x)
         assert x.shape[0] == self.in_dim, (x.shape, self.in_dim)
         if x.dtype == torch.float16:
-            # half: the reference-interface kernels (half storage, fp32 sums) with the
-            # reference's own argument list and inverse index
+            if (self.weights.dtype == torch.float32 and self.num_gates <= 16
+                    and x.device.type == "cuda"
+                    and _HALF_BATCH[0] <= x.shape[1] <= _HALF_BATCH[1]):
+                plan = self.run_plan()
+                if plan.single_run:
+                    return LogicLayerHalfFunction.apply(x, self.weights, self.gate_sequence,
+                                                        plan).transpose(0, 1)
+            # other half layers: the reference-interface kernels (half storage, fp32 sums) with
+            # the reference's own argument list and inverse index
             w = torch.nn.functional.softmax(self.weights, dim=-1).to(x.dtype)
             return LogicLayerCudaFunction.apply(
                 x, self.indices[0], self.indices[1], w, self.gate_sequence,

@@ -262,6 +262,28 @@ int cl_dense_backward_rows_first_any(int dtype, const void* x, const void* grad_
                                  const uint8_t* gate_seq0, const void* probs0, void* grad_w0,
                                  int64_t num_gates0, void* stream);
 
+/* The module path on float16 rows (x, y, grad_y, grad_x) with fp32 logits: the fused forward,
+ * the row backward and the weight gradient of single-run neurons of at most 16 slots, batches
+ * of 8 to 2048 samples (row buffers 16-byte aligned when batch % 8 == 0).  Sums, softmax and
+ * the gradient of the logits are fp32; rows are rounded once on store.  Arguments as for
+ * cl_dense_forward_fused (softmax inside), cl_dense_backward_rows and cl_dense_weight_grad. */
+int cl_dense_forward_fused_half(const void* x, const float* w, const uint8_t* gate_seq,
+                                const int32_t* nab, const int32_t* inv_pos, float* probs,
+                                float* inv_coef, void* y, int64_t in_dim, int64_t out_dim,
+                                int64_t num_runs, int64_t batch, int64_t num_gates, void* stream);
+int cl_dense_backward_rows_half(const void* x, const void* grad_y, const int32_t* slot_rec,
+                                const int32_t* inv_rec, const float* inv_coef,
+                                const uint8_t* gate_seq, const float* probs,
+                                const int32_t* run_ptr, float* grad_w, void* grad_x,
+                                int64_t in_dim, int64_t out_dim, int64_t num_runs, int64_t batch,
+                                int64_t num_gates, void* stream);
+int cl_dense_weight_grad_half(const void* x, const void* grad_y, const uint8_t* gate_seq,
+                              const float* probs, const int32_t* run_ptr, const int32_t* run_ab,
+                              const int32_t* run_gl, float* grad_w, int64_t in_dim,
+                              int64_t out_dim, int64_t num_runs, int64_t batch, int64_t num_gates,
+                              void* stream);
+
+
 /* Weight gradient from the moments: grad_w[o, g] = (c0, c1, c2, c3)[gate_seq[o,g]] . (moments
  * of g's run summed over the chunks in chunk order); with `probs` (not NULL) followed by the
  * softmax backward, giving the gradient of the logits. */

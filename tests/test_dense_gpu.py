@@ -554,3 +554,40 @@ def test_batches_off_the_vector_width(device, dtype, shared, batch):
         np.testing.assert_allclose(np_(got[-1]), ref_gw, **TOL[dtype])
         if need_x:
             np.testing.assert_allclose(np_(got[0]).T, ref_gx, **TOL[dtype])
+
+
+@pytest.mark.parametrize("batch", [8, 9, 15, 64, 127, 505, 512, 513, 1024, 1031, 2041, 2048])
+@pytest.mark.parametrize("in_dim,out_dim,g_n", [(37, 70, 16), (60, 130, 5), (12, 90, 1)])
+def test_half_module_path(device, batch, in_dim, out_dim, g_n):
+    """Half rows through the module path of single-run layers (one row per wave, and rows
+    shared by two and four waves): the smallest and largest batches, around a wave's 512
+    samples per vector, off the 8-sample vector; with the input gradient and the weight gradient
+    alone.  Half inputs are exact in the oracle; y and grad_x are rounded to half once (2^-11
+    relative, plus fp32 sums far below it), the logits gradient is fp32."""
+    L = make_layer(batch + g_n, in_dim, out_dim, g_n, batch, True)
+    x16, gy16 = (torch.as_tensor(L[k]).half() for k in ("x", "gy"))
+    X, GY = x16.double().numpy(), gy16.double().numpy()
+    layer = cl.LogicLayer(in_dim, out_dim, connections="original", num_gates=g_n).to(device)
+    with torch.no_grad():
+        layer.weights.copy_(torch.as_tensor(np.log(L["w"])))
+        layer.indices.copy_(torch.as_tensor(np.stack([L["a"], L["b"]])))
+        layer.gate_sequence.copy_(torch.as_tensor(L["gs"]))
+    layer.refresh_backward_index()
+    ref_y = O.dense_forward(X, L["a"], L["b"], L["w"], L["gs"])
+    ref_p = O.dense_backward_w(X, L["a"], L["b"], L["gs"], GY)
+    ref_gw = L["w"] * (ref_p - (L["w"] * ref_p).sum(1, keepdims=True))
+    ref_gx = O.dense_backward_x_direct(X, L["a"], L["b"], L["w"], L["gs"], GY)
+    half = dict(rtol=2.0 ** -10, atol=1e-6)
+    small = dict(rtol=2.0 ** -10, atol=max(1e-7, 2.0 ** -24))     # half subnormals of gradients
+    for need_x in (True, False):
+        x = x16.to(device).t().requires_grad_(need_x)
+        with cl.layers.timing.record() as rec:
+            y = layer(x)
+            got = torch.autograd.grad(y, ([x] if need_x else []) + [layer.weights],
+                                      gy16.to(device).t())
+        assert any(n.startswith("cl_dense_forward_fused_half") for n in rec.summary())
+        assert y.dtype == torch.float16 and got[-1].dtype == torch.float32
+        np.testing.assert_allclose(np_(y).T.astype(np.float64), ref_y, **half)
+        np.testing.assert_allclose(np_(got[-1]), ref_gw, **TOL[torch.float32])
+        if need_x:
+            np.testing.assert_allclose(np_(got[0]).T.astype(np.float64), ref_gx, **small)
