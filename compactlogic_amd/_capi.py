@@ -139,6 +139,10 @@ SIGNATURES: dict[str, list] = {
     "cl_eval_packed_indexed_columns": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p],
     "cl_eval_packed_indexed_pair_columns": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64,
                                             _i64, _i64, _i64, _p],
+    "cl_packed_rows_to_columns": [_p, _p, _i64, _i64, _i64, _p],
+    "cl_tree_columns_layout": [ctypes.POINTER(_i64), _i64] + [ctypes.POINTER(_i64)] * 4,
+    "cl_tree_columns": [_p, _i64, _i64, ctypes.POINTER(_i64), _i64, ctypes.POINTER(_p),
+                        ctypes.POINTER(_p), _p, _p, _i64, _p],
     "cl_packed_network_columns": [_p, _i64, _i64, _i64, _p, ctypes.POINTER(_i64), _i64, _i64,
                                   _p, _p],
 }

@@ -10,6 +10,7 @@ same argmax-slot semantics as compactlogic/compactlogic.py:120-130.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -18,6 +19,7 @@ from . import _capi
 from . import timing
 from . import difflogic_hip as _dl
 from .layers import ConvLayer, GroupSum, LogicLayer, PackBitsTensor
+from .treelogic import ConvLogicLayer
 
 
 def _limits():
@@ -142,6 +144,34 @@ def producer_order(tabs: list, in_rows: int) -> np.ndarray:
                       ).astype(np.int32)
 
 
+def _tree_front(prefix: list) -> list | None:
+    """The complete ConvLogicLayers that make up `prefix` (Flatten modules pass a PackBitsTensor
+    through unchanged); None when it holds anything else or nothing."""
+    blocks = [m for m in prefix if type(m) is not torch.nn.Flatten]
+    ok = all(type(m) is ConvLogicLayer and m.complete for m in blocks)
+    return blocks if blocks and ok else None
+
+
+def tree_columns_layout(blocks: list, rows: int) -> tuple | None:
+    """(geometry array, output rows, table words) of cl_tree_columns for the blocks on a square
+    input of `rows` features, or None when the pass does not take them
+    (cl_tree_columns_layout)."""
+    if rows % blocks[0].in_channels:
+        return None
+    h = w = math.isqrt(rows // blocks[0].in_channels)
+    if h * w * blocks[0].in_channels != rows:
+        return None
+    geo = []
+    for m in blocks:
+        (sh, sw), (ph, pw), (kh, kw) = m.stride, m.padding, m.kernel
+        geo += [m.in_channels, h, w, m.out_channels, sh, sw, ph, pw, kh, kw]
+        h, w = ((h + 2 * ph - kh) // sh + 1) // 2, ((w + 2 * pw - kw) // sw + 1) // 2
+    arr = (ctypes.c_int64 * len(geo))(*geo)
+    out = [ctypes.c_int64(0) for _ in range(4)]
+    _capi.call("cl_tree_columns_layout", arr, len(blocks), *[ctypes.byref(v) for v in out])
+    return (arr, out[2].value, out[3].value) if out[0].value else None
+
+
 def _table_layer_before(body: list, j: int):
     """Index of the module before body[j] (Flatten modules pass a PackBitsTensor through
     unchanged) when it is a packed layer from index tables (ConvLayer or LogicLayer); else
@@ -152,6 +182,15 @@ def _table_layer_before(body: list, j: int):
     if j < 0 or type(body[j]) not in (ConvLayer, LogicLayer):
         return None
     return j
+
+
+def _column_words(layout: dict, layer: int, pos: np.ndarray) -> np.ndarray:
+    """LDS words of layer `layer`'s rows at positions pos under a columns_layout (banks as the
+    positions': every base is a multiple of 32 words)."""
+    if layer == 0:
+        return np.where(pos < layout["split"], layout["base"][0] + pos,
+                        layout["hold_base"] + pos - layout["split"])
+    return layout["base"][layer] + pos
 
 
 class PackedNetwork:
@@ -167,7 +206,9 @@ class PackedNetwork:
     (columns_layout): that layer writes its output column-major
     (cl_eval_packed_indexed_columns) and the tail runs on those columns
     (cl_packed_network_columns).  When no tail qualifies every module runs layer by
-    layer and the counts come from the group popcount.  The gate tables are built once here;
+    layer and the counts come from the group popcount.  A fused tail whose prefix is complete
+    ConvLogicLayers alone takes its input column-major from them (cl_tree_columns: all blocks on
+    one column in LDS).  The gate tables are built once here;
     rebuild after changing the model.  With `bank_aware` (default), each fused layer's rows
     are laid out in LDS by bank_aware_positions, so that the row reads of the kernel's
     half-waves hit distinct LDS banks; the counts do not depend on the layout.
@@ -220,7 +261,14 @@ class PackedNetwork:
         if self.rows[-1] % self.k:
             raise ValueError(f"in_dim ({self.rows[-1]}) has to be divisible by k ({self.k}) "
                              "but it is not")
-        entries = []
+        # complete logic-tree blocks before the tail: they can hand it columns
+        self.front = self.front_layout = None
+        if self.producer is None:
+            self.front = _tree_front(self.prefix)
+            self.front_layout = columns_layout(self.rows) if self.front else None
+            if self.front_layout is None:
+                self.front = None
+        entries, front_entries = [], []
         with torch.no_grad():
             wiring = []
             for m in layers:
@@ -255,6 +303,7 @@ class PackedNetwork:
                 prev_pos = np.empty(self.rows[0], dtype=np.int64)
                 prev_pos[order] = np.arange(self.rows[0], dtype=np.int64)
                 self.col_order = torch.as_tensor(order, device=layers[0].weights.device)
+            front_word = np.arange(self.rows[0], dtype=np.int64)  # LDS words in the columns
             for i, (m, (a, b, g, dev)) in enumerate(zip(layers, wiring)):
                 pa, pb = prev_pos[a], prev_pos[b]
                 if not bank_aware:
@@ -272,15 +321,15 @@ class PackedNetwork:
                     prev_pos = pos
                 else:
                     ent[pos] = pa | (pb << 16) | (g << 32)               # LDS words
-                    # the LDS word of each row (banks as the positions': every base is a
-                    # multiple of 32 words)
-                    if i == 0:
-                        prev_pos = np.where(pos < lay["split"], lay["base"][0] + pos,
-                                            lay["hold_base"] + pos - lay["split"])
-                    else:
-                        prev_pos = lay["base"][i] + pos
+                    prev_pos = _column_words(lay, i, pos)
                 entries.append(torch.as_tensor(ent, device=dev))
+                if self.front is not None:   # the same positions for the column-major input
+                    ent = np.empty(m.out_dim, dtype=np.int64)
+                    ent[pos] = front_word[a] | (front_word[b] << 16) | (g << 32)
+                    front_word = _column_words(self.front_layout, i, pos)
+                    front_entries.append(torch.as_tensor(ent, device=dev))
         self.tables = torch.cat(entries).contiguous()
+        self.front_tables = torch.cat(front_entries).contiguous() if front_entries else None
         self.device = self.tables.device
         self._rows_host = (ctypes.c_int64 * len(self.rows))(*self.rows)
 
@@ -288,6 +337,9 @@ class PackedNetwork:
         if self.producer is not None:
             return self._call_columns(x)
         if self.prefix:
+            counts = self._call_front(x) if self.rows is not None and self.front else None
+            if counts is not None:
+                return counts
             if isinstance(x, PackBitsTensor):
                 h = PackBitsTensor.from_packed(x.t, x.pad_len)   # the caller's object stays
             else:
@@ -370,5 +422,50 @@ class PackedNetwork:
                          lambda: _capi.call(
                 "cl_packed_network_columns", colmaj.data_ptr(), cols, in_words, n,
                 self.tables.data_ptr(), self._rows_host, len(self.rows) - 1, self.k,
+                counts.data_ptr(), stream))
+        return counts
+
+    def _call_front(self, x):
+        """The logic-tree blocks and the tail on columns: the packed rows turned to columns, all
+        blocks on one column in LDS, then the fused tail.  None when the blocks' shape or taps
+        (or the rows' width) ask for the layer-by-layer kernels."""
+        words = x.t if isinstance(x, PackBitsTensor) else x
+        _dl._check(words, "x")
+        if words.dim() != 2 or words.device != self.device:
+            return None
+        rows, row_bytes = words.shape[0], words.shape[1] * words.element_size()
+        blocks = self.front
+        plan = tree_columns_layout(blocks, rows) if row_bytes and row_bytes % 8 == 0 else None
+        if (plan is None or plan[1] != self.rows[0] or any(m.training for m in blocks)
+                or not all(m._regular_taps() for m in blocks)
+                or any(m.weights.device != self.device for m in blocks)
+                or any(m._forward_hooks or m._forward_pre_hooks for m in blocks)):
+            return None
+        geo, _, table_words = plan
+        n = x.num_samples if isinstance(x, PackBitsTensor) else row_bytes * 8
+        cols, in_words = row_bytes // 4, self.front_layout["in_words"]
+        dev, stream = words.device, _dl.stream_of(words)
+
+        def ints(*shape):
+            return torch.empty(shape, dtype=torch.int32, device=dev)
+
+        with torch.no_grad(), torch.cuda.device(dev):
+            gates = [m.weights.argmax(-1).to(torch.uint8).contiguous() for m in blocks]
+            taps = [m.selection.to(torch.int32).contiguous() for m in blocks]
+            ptrs = [(ctypes.c_void_p * len(blocks))(*[t.data_ptr() for t in ts])
+                    for ts in (gates, taps)]
+            colmaj, tables = ints(cols, rows), ints(table_words)
+            timing.timed(f"cl_packed_rows_to_columns[{rows}]", lambda: _capi.call(
+                "cl_packed_rows_to_columns", words.data_ptr(), colmaj.data_ptr(), rows,
+                row_bytes, rows, stream))
+            mid = ints(cols, in_words)
+            timing.timed(f"cl_tree_columns[{rows}->{self.rows[0]}]", lambda: _capi.call(
+                "cl_tree_columns", colmaj.data_ptr(), cols, rows, geo, len(blocks), *ptrs,
+                tables.data_ptr(), mid.data_ptr(), in_words, stream))
+            counts = ints(n, self.k)
+            timing.timed(f"cl_packed_network_columns[{self.rows[0]}->{self.rows[-1]}]",
+                         lambda: _capi.call(
+                "cl_packed_network_columns", mid.data_ptr(), cols, in_words, n,
+                self.front_tables.data_ptr(), self._rows_host, len(self.rows) - 1, self.k,
                 counts.data_ptr(), stream))
         return counts

@@ -649,6 +649,29 @@ int cl_packed_network_columns(const void* x, int64_t cols, int64_t in_words, int
                               const uint64_t* tables, const int64_t* rows_host,
                               int64_t num_layers, int64_t k, int32_t* counts, void* stream);
 
+/* Packed rows to columns: y[c * out_words + r] (32-bit words) = word c of row r of x
+ * [rows, row_bytes], out_words >= rows; words past the rows of a column are not written. */
+int cl_packed_rows_to_columns(const void* x, void* y, int64_t rows, int64_t row_bytes,
+                              int64_t out_words, void* stream);
+
+/* Complete logic-tree blocks on column-major words (the packed reading of cl_tree_conv_eval_packed
+ * with complete = 1), up to four in a row, a 32-sample column at a time with its activations in
+ * LDS.  geometry: int64 [num_blocks, 10], (c_in, h, w, c_out, stride_h, stride_w, pad_h, pad_w,
+ * kernel_h, kernel_w) per block, each block reading the one before.
+ * cl_tree_columns_layout (host only) says whether the chain fits (*applies), its input and output
+ * rows and the 32-bit words of device scratch (16-byte aligned) it needs for its tables.
+ * cl_tree_columns: x [cols, in_words], y [cols, out_words] column-major; gates[b] (uint8
+ * [c_out, 7]) and selections[b] (int32 [c_out, 8]) as for cl_tree_conv_eval_packed, host arrays of
+ * device pointers.  Every tap must lie inside its kernel window (the caller checks); a channel
+ * with a tap on a channel >= c_in is all ones, as there. */
+int cl_tree_columns_layout(const int64_t* geometry, int64_t num_blocks, int64_t* applies,
+                           int64_t* in_rows, int64_t* out_rows, int64_t* table_words);
+int cl_tree_columns(const void* x, int64_t cols, int64_t in_words, const int64_t* geometry,
+                    int64_t num_blocks, const uint8_t* const* gates,
+                    const int32_t* const* selections, void* tables, void* y, int64_t out_words,
+                    void* stream);
+
+
 /* -------------------------------------------------------------------------------------------
  * Logic-tree convolution block (third-party ConvLogic, convlogic_cuda extension,
  * third_party/convlogic_source_code/src/convlogic/cuda/convlogic.cpp:31-43).

@@ -322,3 +322,90 @@ def test_bank_aware_layout_gives_the_same_counts(device):
     b = cl.PackedNetwork(model, bank_aware=False)(x)
     assert torch.equal(a, b)
     assert np.array_equal(np_(a), oracle_counts(model, np_(x.t).view(np.uint64), n))
+
+
+def tree_net(blocks, dense, k, seed, device):
+    torch.manual_seed(seed)
+    mods = [cl.ConvLogicLayer(ci, co, stride=s, padding=p, kernel=ks, complete=True, num_chn=0)
+            for ci, co, s, p, ks in blocks]
+    model = torch.nn.Sequential(*mods, torch.nn.Flatten(),
+                                *[cl.LogicLayer(i, o) for i, o in dense], cl.GroupSum(k, 1.0))
+    model = model.to(device)
+    configs.freeze_argmax(model)
+    return model
+
+
+@pytest.mark.parametrize("side,blocks,dense,n", [
+    # 8 x 8 pooled positions (a wave per channel), then 4 per channel (a lane per position)
+    (32, [(3, 40, 2, 1, 3), (40, 32, 2, 1, 3)], [(128, 300), (300, 200)], 1000),
+    (32, [(9, 16, 2, 1, 3)], [(1024, 600)], 64),                   # one block
+    (16, [(2, 17, 1, 1, 3)], [(1088, 1000), (1000, 990)], 333),    # stride 1: dy = pitch, 64 positions
+    (64, [(1, 5, 2, 2, 5)], [(1280, 700)], 130),                   # 256 positions, kernel 5, pad 2
+    (12, [(3, 10, 1, 1, 3), (10, 12, 1, 1, 3)], [(108, 200)], 77), # 36 positions, 9 positions
+    (33, [(2, 9, 2, 0, 2)], [(576, 500)], 50),                     # odd side, even kernel, no halo
+    (16, [(2, 6, 1, 1, 3), (6, 7, 1, 1, 3), (7, 8, 1, 1, 3)], [(32, 100)], 200),  # three blocks
+])
+def test_tree_front_on_columns(device, side, blocks, dense, n):
+    """PackedNetwork runs complete logic-tree blocks on columns (cl_tree_columns): counts equal to
+    the layer-by-layer kernels', which the oracle pins, at word counts off the column tiles."""
+    from compactlogic_amd import timing
+    model = tree_net(blocks, dense, 10, n, device)
+    bits = torch.rand((n, blocks[0][0] * side * side), device=device) < 0.5
+    x = cl.PackBitsTensor(bits, 64)
+    net = cl.PackedNetwork(model)
+    with timing.record() as rec:
+        counts = net(x)
+    assert any(c.startswith("cl_tree_columns") for c in rec.summary())
+    ref = model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len))
+    assert torch.equal(counts, ref)
+
+
+def test_tree_front_every_gate_and_bad_channel(device):
+    """cl_tree_columns against cl_tree_conv_eval_packed on one block with random gates for a wave
+    per channel and a lane per position, every opcode at every node (all pairs over the
+    channels), and channels whose taps name a channel past the input."""
+    import ctypes
+    from compactlogic_amd import _capi
+    from compactlogic_amd import treelogic as TL
+    rng = np.random.default_rng(5)
+    for side, cin, cout, stride in ((32, 2, 700, 2), (8, 3, 700, 2)):
+        gates = torch.as_tensor(rng.integers(0, 16, (cout, 7)).astype(np.uint8), device=device)
+        sel = (rng.integers(0, cin, (cout, 8)) << 16) | (rng.integers(0, 3, (cout, 8)) << 8) \
+            | rng.integers(0, 3, (cout, 8))
+        sel[::97, 3] = cin << 16
+        sel = torch.as_tensor(sel.astype(np.int32), device=device)
+        words = 5
+        xw = torch.as_tensor(rng.integers(-2**31, 2**31, (cin * side * side, 2 * words)),
+                             dtype=torch.int32, device=device).view(torch.int64)
+        ref = TL.tree_conv_eval_packed(xw, gates, sel, (cin, side, side), stride, 1, 3, True)
+        geo = (ctypes.c_int64 * 10)(cin, side, side, cout, stride, stride, 1, 1, 3, 3)
+        v = [ctypes.c_int64(0) for _ in range(4)]
+        _capi.call("cl_tree_columns_layout", geo, 1, *[ctypes.byref(i) for i in v])
+        assert v[0].value == 1 and v[1].value == xw.shape[0] and v[2].value == ref.shape[0]
+        cols = 2 * words
+        x32 = xw.view(torch.int32)
+        colmaj = torch.empty((cols, xw.shape[0]), dtype=torch.int32, device=device)
+        s = torch.cuda.current_stream().cuda_stream
+        _capi.call("cl_packed_rows_to_columns", x32.data_ptr(), colmaj.data_ptr(), xw.shape[0],
+                   cols * 4, xw.shape[0], s)
+        assert torch.equal(colmaj, x32.t())
+        tables = torch.empty(v[3].value, dtype=torch.int32, device=device)
+        out = torch.empty((cols, ref.shape[0]), dtype=torch.int32, device=device)
+        one = lambda t: (ctypes.c_void_p * 1)(t.data_ptr())
+        _capi.call("cl_tree_columns", colmaj.data_ptr(), cols, xw.shape[0], geo, 1, one(gates),
+                   one(sel), tables.data_ptr(), out.data_ptr(), ref.shape[0], s)
+        assert torch.equal(out.t(), ref.view(torch.int32))
+        assert bool((out.t().reshape(cout, -1)[::97] == -1).all())
+
+
+def test_tree_front_steps_aside(device):
+    """Taps outside the kernel window, rows of an odd number of words and a non-square input take
+    the layer-by-layer kernels as before."""
+    model = tree_net([(2, 8, 2, 1, 3)], [(32, 100)], 10, 3, device)
+    x = cl.PackBitsTensor(torch.rand((100, 2 * 64), device=device) < 0.5, 64)
+    net = cl.PackedNetwork(model)
+    assert net._call_front(x) is not None
+    with torch.no_grad():
+        model[0].selection[0, 0] = 7 << 8            # row 7 of a 3 x 3 window
+    assert net._call_front(x) is None
+    assert torch.equal(net(x), model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
