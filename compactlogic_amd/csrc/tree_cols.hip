@@ -68,14 +68,17 @@ __device__ __forceinline__ void exchange(uint32_t& a, uint32_t& b) {
 // ------------------------------------------------------------------------------------------
 // Tables of one block, a thread per channel: word k < 8 holds the LDS words of tap k at pooled
 // position 0 for the two conv columns of the window (first | second << 16), word 8 the gates as
-// 4-bit codes for tree_block_uniform, word 9 their opcodes (nibbles) for tree_block_lanes, whose
-// tap order is the block's own (words 0-7 are then unswapped).
+// 4-bit codes for tree_block_uniform with the live taps in word 10, word 9 the opcodes (nibbles)
+// for tree_block_lanes, whose tap order is the block's own.
 //
 // Codes.  An opcode that is 1 at a = b = 0 is replaced by its complement and its reader's table
 // turned round to match, which leaves one inversion at the root (bit 31 of word 8).  A gate
-// that then passes a, or a & ~b, has its operands swapped: two taps, or two subtrees with all
-// that hangs from them.  What is left is 0, b, a & b, ~a & b, a | b and a ^ b.  The first five
-// are majority(t, b, s) with t = (a & v) ^ u: code bits v, u, s; bit 3 marks a ^ b.
+// that then ignores an operand, or reads one that is always 0, passes the other or is always 0
+// itself; one that passes a, or is a & ~b, has its operands swapped: two taps, or two subtrees
+// with all that hangs from them.  What is left is: pass b (code 0), a & b, ~a & b (code 1, bit 2
+// for the second), a ^ b, a | b (code 3, bit 2 for the second).  Bit 30 of word 8: always 0.
+// Taps and gates that no live gate reads have no code and are not evaluated: of random gates
+// a quarter passes one operand and an eighth none, and 42 % of the taps are live.
 // A channel with a tap on a channel past the input is all ones, as in the row-major block.
 __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restrict__ gates,
                                                           const int32_t* __restrict__ sel,
@@ -86,7 +89,7 @@ __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restr
     if (c == 0) *desc = g;  // read back through the scalar cache at a run-time block index
     if (c >= g.cout) return;
     uint32_t* t = tab + int64_t(c) * kTcTabWords;
-    uint32_t tap[8];
+    uint32_t tap[8], t0[8];  // in the order of the codes, in the block's own
     bool bad = false;
 #pragma unroll
     for (int k = 0; k < 8; ++k) bad |= ((sel[c * 8 + k] >> 16) & 0xFFFF) >= g.cin;
@@ -99,74 +102,123 @@ __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restr
         const int row = g.base + ch * g.cs + ky * g.pitch;
         const uint32_t o0 = in ? row + phase_slot(g, kx) : g.base;
         const uint32_t o1 = in ? row + phase_slot(g, kx + g.sw) : g.base;
-        tap[k] = o0 | (o1 << 16);
+        tap[k] = t0[k] = o0 | (o1 << 16);
     }
-    uint32_t ops = 0, code[7], inv[7];
+    uint32_t ops = 0, code[7], inv[7], kind[7];  // kind: 0 always 0, 1 passes b, 2 reads both
+    uint32_t raw[7];
 #pragma unroll
     for (int q = 0; q < 7; ++q) {
         uint32_t f = gates[c * 7 + q] & 15u;  // bits 3..0: (a, b) = 00, 01, 10, 11
         if (bad) f = 15u;
+        raw[q] = f;
         ops |= f << (4 * q);
-        const uint32_t ia = q < 4 ? 0u : q < 6 ? inv[2 * (q - 4)] : inv[4];
-        const uint32_t ib = q < 4 ? 0u : q < 6 ? inv[2 * (q - 4) + 1] : inv[5];
+        const int l = 2 * (q - 4);
+        const uint32_t ia = q < 4 ? 0u : q < 6 ? inv[l] : inv[4];
+        const uint32_t ib = q < 4 ? 0u : q < 6 ? inv[l + 1] : inv[5];
         if (ia) f = ((f & 12u) >> 2) | ((f & 3u) << 2);
         if (ib) f = ((f & 10u) >> 1) | ((f & 5u) << 1);
         inv[q] = f >> 3;
         if (inv[q]) f ^= 15u;  // now the value at 00 is 0: bits 2..0 = 01, 10, 11
-        const bool swap = f == 2u || f == 3u;  // a & ~b, a
-        if (swap) f = f == 2u ? 4u : 5u;       // ~a & b, b
-        //            0   ab      ~ab     b       a^b  a|b
-        code[q] = f == 1u ? 1u : f == 4u ? 3u : f == 5u ? 2u : f == 6u ? 8u : f == 7u ? 5u : 0u;
-        if (g.uniform && swap) {
+        const bool za = q >= 4 && kind[q < 6 ? l : 4] == 0u;      // an operand that is always 0
+        const bool zb = q >= 4 && kind[q < 6 ? l + 1 : 5] == 0u;
+        if (za) f = (f & 4u) ? 5u : 0u;          // f(0, b): b or 0
+        if (zb) f = (f & 2u) && !za ? 3u : 0u;   // f(a, 0): a or 0
+        const bool swap = f == 2u || f == 3u;    // a & ~b, a
+        if (swap) f = f == 2u ? 4u : 5u;         // ~a & b, b
+        kind[q] = f == 0u ? 0u : f == 5u ? 1u : 2u;
+        //        ab           ~ab            a^b            a|b
+        code[q] = f == 1u ? 1u : f == 4u ? 5u : f == 6u ? 3u : f == 7u ? 7u : 0u;
+        if (swap) {
             if (q < 4) {
                 exchange(tap[2 * q], tap[2 * q + 1]);
             } else if (q < 6) {
-                const int l = 2 * (q - 4);
                 exchange(code[l], code[l + 1]);
+                exchange(kind[l], kind[l + 1]);
                 exchange(tap[2 * l], tap[2 * l + 2]);
                 exchange(tap[2 * l + 1], tap[2 * l + 3]);
             } else {
                 exchange(code[4], code[5]);
+                exchange(kind[4], kind[5]);
                 exchange(code[0], code[2]);
                 exchange(code[1], code[3]);
+                exchange(kind[0], kind[2]);
+                exchange(kind[1], kind[3]);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) exchange(tap[k], tap[k + 4]);
             }
         }
     }
-    uint32_t codes = inv[6] << 31;
+    // liveness from the root down; a live gate is never always 0 below the root
+    uint32_t on[7], taps = 0, codes = (inv[6] << 31) | (kind[6] == 0u ? 1u << 30 : 0u);
+    on[6] = kind[6] != 0u;
 #pragma unroll
-    for (int q = 0; q < 7; ++q) codes |= code[q] << (4 * q);
+    for (int q = 6; q >= 0; --q) {
+        const uint32_t na = on[q] && kind[q] == 2u, nb = on[q];
+        if (q == 6) on[4] = na, on[5] = nb;
+        else if (q >= 4) on[2 * (q - 4)] = na, on[2 * (q - 4) + 1] = nb;
+        else taps |= (na << (2 * q)) | (nb << (2 * q + 1));
+        codes |= (on[q] ? code[q] : 0u) << (4 * q);
+    }
+    if (!g.uniform) {
+        // the lanes read every tap: one whose value cannot reach the root goes to one shared
+        // word, which costs no bank conflicts
+        uint32_t need[7];
+        need[6] = 1u;
+#pragma unroll
+        for (int q = 6; q >= 0; --q) {
+            const uint32_t f = raw[q];
+            const uint32_t na = need[q] && ((f ^ (f >> 2)) & 3u);
+            const uint32_t nb = need[q] && ((f ^ (f >> 1)) & 5u);
+            if (q == 6) need[4] = na, need[5] = nb;
+            else if (q >= 4) need[2 * (q - 4)] = na, need[2 * (q - 4) + 1] = nb;
+            else {
+                tap[2 * q] = na ? t0[2 * q] : uint32_t(g.base) * 0x10001u;
+                tap[2 * q + 1] = nb ? t0[2 * q + 1] : uint32_t(g.base) * 0x10001u;
+            }
+        }
+    }
 #pragma unroll
     for (int k = 0; k < 8; ++k) t[k] = tap[k];
     t[8] = codes;
     t[9] = ops;
-    t[10] = t[11] = 0u;
+    t[10] = taps;
+    t[11] = 0u;
 }
 
-// Four words of a node: the conv positions of a pooling window (a vector type, so that every
-// word stays a register of its own across the branches).
-typedef uint32_t U4 __attribute__((ext_vector_type(4)));
+// Four words of a node, one per conv position of a pooling window (named words, so that each
+// stays a register of its own across the branches).
+struct Win {
+    uint32_t x, y, z, w;
+};
 
-// gate(a, b) from the code's low four bits (uniform): one branch for a ^ b, else two three-input
-// operations per word, each with one scalar mask.
-__device__ __forceinline__ U4 gate_coded(uint32_t code, U4 a, U4 b) {
-    U4 r;
-    if (code & 8u) {
-        r = a ^ b;
-        asm volatile("");  // a branch, not selects
-    } else {
-        const uint32_t v = uint32_t(__builtin_amdgcn_sbfe(int(code), 0, 1));
-        const uint32_t u = uint32_t(__builtin_amdgcn_sbfe(int(code), 1, 1));
-        const uint32_t s = uint32_t(__builtin_amdgcn_sbfe(int(code), 2, 1));
-        // truth-table immediates over (first, second, third) = 0xF0, 0xCC, 0xAA: (a & v) ^ u
-        // and the majority of (t, b, s)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            r[i] = __builtin_amdgcn_bitop3_b32(__builtin_amdgcn_bitop3_b32(a[i], v, u, 0x6A), b[i],
-                                               s, 0xE8);
+// b = gate(a, b) from the code's low four bits (uniform): nothing for a gate that passes b,
+// else a branch on the pair of gates and one three-input operation per word with a scalar mask.
+// Truth-table immediates over (first, second, third) = 0xF0, 0xCC, 0xAA.
+__device__ __forceinline__ void gate_coded(uint32_t code, const Win& a, Win& b) {
+    if (code & 1u) {
+        const uint32_t m = uint32_t(__builtin_amdgcn_sbfe(int(code), 2, 1));
+        if (code & 2u) {  // m ? a | b : a ^ b
+            b.x = __builtin_amdgcn_bitop3_b32(a.x, b.x, m, 0xBC);
+            b.y = __builtin_amdgcn_bitop3_b32(a.y, b.y, m, 0xBC);
+            b.z = __builtin_amdgcn_bitop3_b32(a.z, b.z, m, 0xBC);
+            b.w = __builtin_amdgcn_bitop3_b32(a.w, b.w, m, 0xBC);
+        } else {  // m ? ~a & b : a & b
+            b.x = __builtin_amdgcn_bitop3_b32(a.x, b.x, m, 0x48);
+            b.y = __builtin_amdgcn_bitop3_b32(a.y, b.y, m, 0x48);
+            b.z = __builtin_amdgcn_bitop3_b32(a.z, b.z, m, 0x48);
+            b.w = __builtin_amdgcn_bitop3_b32(a.w, b.w, m, 0x48);
+            asm volatile("");  // a branch, not selects
+        }
     }
-    return r;
+}
+
+// One channel's table words in scalar registers.
+struct ChanTab {
+    uint32_t t0, t1, t2, t3, t4, t5, t6, t7, codes, on;
+};
+
+__device__ __forceinline__ ChanTab load_tab(const uint32_t* __restrict__ t) {
+    return ChanTab{t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[10]};
 }
 
 __device__ __forceinline__ uint32_t gate_bits(uint32_t f, uint32_t a, uint32_t b) {
@@ -208,21 +260,47 @@ __device__ __forceinline__ void tree_block_uniform(uint32_t* lds, const uint32_t
         const int cs = nx ? nx->cs : g.P, cout = g.cout;
         const bool last = !nx;
         const uint32_t* src = lds + posb;
+        ChanTab next = load_tab(tab + min(wave_id(), cout - 1) * kTcTabWords);
         for (int c = wave_id(); c < cout; c += kTcThreads / 64) {
-            const uint32_t* t = tab + c * kTcTabWords;
-            auto tap = [&](uint32_t o) -> U4 {
-                const uint32_t* p0 = src + (o & 0xffffu);
-                const uint32_t* p1 = src + (o >> 16);
-                return U4{p0[0], p1[0], p0[DY], p1[DY]};
+            // the next channel's table is loaded while this one is evaluated; the empty asm
+            // keeps this one's loads ahead of the branches that use them
+            ChanTab t = next;
+            asm volatile(""
+                         : "+s"(t.t0), "+s"(t.t1), "+s"(t.t2), "+s"(t.t3), "+s"(t.t4), "+s"(t.t5),
+                           "+s"(t.t6), "+s"(t.t7), "+s"(t.codes), "+s"(t.on));
+            next = load_tab(tab + min(c + kTcThreads / 64, cout - 1) * kTcTabWords);
+            Win v0, v1, v2, v3, v4, v5, v6, v7;
+            auto tap = [&](uint32_t bit, uint32_t o, Win& v) {
+                if (t.on & bit) {
+                    const uint32_t* p0 = src + (o & 0xffffu);
+                    const uint32_t* p1 = src + (o >> 16);
+                    v.x = p0[0];
+                    v.y = p0[DY];
+                    v.z = p1[0];
+                    v.w = p1[DY];
+                }
             };
-            const uint32_t codes = t[8];
-            const U4 v0 = tap(t[0]), v1 = tap(t[1]), v2 = tap(t[2]), v3 = tap(t[3]);
-            const U4 v4 = tap(t[4]), v5 = tap(t[5]), v6 = tap(t[6]), v7 = tap(t[7]);
-            const U4 n0 = gate_coded(codes, v0, v1), n1 = gate_coded(codes >> 4, v2, v3);
-            const U4 n2 = gate_coded(codes >> 8, v4, v5), n3 = gate_coded(codes >> 12, v6, v7);
-            const U4 m0 = gate_coded(codes >> 16, n0, n1), m1 = gate_coded(codes >> 20, n2, n3);
-            const U4 z = gate_coded(codes >> 24, m0, m1) ^ uint32_t(int(codes) >> 31);
-            const uint32_t r = (z.x | z.y) | (z.z | z.w);
+            tap(1u, t.t0, v0);
+            tap(2u, t.t1, v1);
+            tap(4u, t.t2, v2);
+            tap(8u, t.t3, v3);
+            tap(16u, t.t4, v4);
+            tap(32u, t.t5, v5);
+            tap(64u, t.t6, v6);
+            tap(128u, t.t7, v7);
+            gate_coded(t.codes, v0, v1);
+            gate_coded(t.codes >> 4, v2, v3);
+            gate_coded(t.codes >> 8, v4, v5);
+            gate_coded(t.codes >> 12, v6, v7);
+            gate_coded(t.codes >> 16, v1, v3);
+            gate_coded(t.codes >> 20, v5, v7);
+            gate_coded(t.codes >> 24, v3, v7);
+            // pool: the OR of the four words, each inverted when the root is
+            const uint32_t root = uint32_t(int(t.codes) >> 31);
+            uint32_t r = root;
+            if (!(t.codes & (1u << 30)))
+                r = __builtin_amdgcn_bitop3_b32(v7.x, v7.y, root, 0x7E) |
+                    __builtin_amdgcn_bitop3_b32(v7.z, v7.w, root, 0x7E);
             if (last) dst_out[c * cs] = r;
             else if (keep) dst_lds[c * cs] = r;
         }
