@@ -8,10 +8,12 @@
 // position per lane: the channel's taps and gates are wave-uniform (scalar loads, scalar
 // branches on the gate), a tap is one LDS read at lane base + channel offset, and neither the
 // address arithmetic nor the gate choice costs vector instructions per word.  Between the
-// blocks nothing leaves LDS.  9x32x32 -> 256 -> 512 channels at 2^20 samples: 2.72 ms and 0.48 ms
+// blocks nothing leaves LDS.  9x32x32 -> 256 -> 512 channels at 2^20 samples: 1.75 ms and 0.48 ms
 // for the rows turned to columns, where the row-major blocks took 3.30 + 0.60 ms and 0.40 ms for
-// widening their input rows.  VALU-bound (about 86 vector instructions per channel and 64
-// positions of the first block).
+// widening their input rows.  Bound by the instructions a SIMD issues, vector and scalar ones
+// together (a column takes 32000 cycles: 22000 in the first block, 6500 in the second, the
+// rest staging and barriers): every tap and gate evaluated 2.72 ms, only live ones with a
+// branch per tap 2.13, a branch per subtree and unshared table words 1.75.
 //
 // LDS layout of a block's input: one plane per channel, zero halo included (a tap outside the
 // image reads 0), rows of `pitch` words, a row's columns split by their phase modulo 2 * sw:
@@ -29,7 +31,7 @@ constexpr int kTcThreads = 1024;
 constexpr int kTcMaxBlocks = 4;
 constexpr int kTcLdsWords = 40960;       // 160 KiB
 constexpr int kTcDescWords = 32;         // words of a block's descriptor before the tables
-constexpr int kTcTabWords = 12;          // table words per channel: 8 taps, codes, opcodes
+constexpr int kTcTabWords = 20;          // table words per channel: 16 tap offsets, codes, opcodes
 constexpr int kTcMaxIpt = 16;            // input words per thread
 constexpr int kTcDy[] = {36, 68, 132};   // conv-row distances with two-word LDS reads
 
@@ -66,19 +68,20 @@ __device__ __forceinline__ void exchange(uint32_t& a, uint32_t& b) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Tables of one block, a thread per channel: word k < 8 holds the LDS words of tap k at pooled
-// position 0 for the two conv columns of the window (first | second << 16), word 8 the gates as
-// 4-bit codes for tree_block_uniform with the live taps in word 10, word 9 the opcodes (nibbles)
-// for tree_block_lanes, whose tap order is the block's own.
+// Tables of one block, a thread per channel: words 2k and 2k + 1 hold the LDS byte offsets of tap k
+// at pooled position 0 for the two conv columns of the window, word 16 the gates as 4-bit codes
+// for tree_block_uniform, word 17 the opcodes (nibbles) for tree_block_lanes, whose tap order is
+// the block's own.
 //
 // Codes.  An opcode that is 1 at a = b = 0 is replaced by its complement and its reader's table
-// turned round to match, which leaves one inversion at the root (bit 31 of word 8).  A gate
+// turned round to match, which leaves one inversion at the root (bit 31 of word 16).  A gate
 // that then ignores an operand, or reads one that is always 0, passes the other or is always 0
 // itself; one that passes a, or is a & ~b, has its operands swapped: two taps, or two subtrees
-// with all that hangs from them.  What is left is: pass b (code 0), a & b, ~a & b (code 1, bit 2
-// for the second), a ^ b, a | b (code 3, bit 2 for the second).  Bit 30 of word 8: always 0.
-// Taps and gates that no live gate reads have no code and are not evaluated: of random gates
-// a quarter passes one operand and an eighth none, and 42 % of the taps are live.
+// with all that hangs from them.  What is left is: pass b (code 0), a & b, ~a & b (bit 0, bit 2
+// for the second), a ^ b, a | b (bit 1, bit 2 for the second).  Bit 3 marks a gate that reads
+// both; bit 30 of word 16 a channel that is always 0.
+// Taps and gates that no live gate reads are not evaluated: of random gates a quarter passes
+// one operand and an eighth none, and 42 % of the taps are live.
 // A channel with a tap on a channel past the input is all ones, as in the row-major block.
 __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restrict__ gates,
                                                           const int32_t* __restrict__ sel,
@@ -89,7 +92,8 @@ __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restr
     if (c == 0) *desc = g;  // read back through the scalar cache at a run-time block index
     if (c >= g.cout) return;
     uint32_t* t = tab + int64_t(c) * kTcTabWords;
-    uint32_t tap[8], t0[8];  // in the order of the codes, in the block's own
+    // LDS words of the taps, first | second << 16: in the order of the codes, in the block's own
+    uint32_t tap[8], t0[8];
     bool bad = false;
 #pragma unroll
     for (int k = 0; k < 8; ++k) bad |= ((sel[c * 8 + k] >> 16) & 0xFFFF) >= g.cin;
@@ -126,8 +130,8 @@ __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restr
         const bool swap = f == 2u || f == 3u;    // a & ~b, a
         if (swap) f = f == 2u ? 4u : 5u;         // ~a & b, b
         kind[q] = f == 0u ? 0u : f == 5u ? 1u : 2u;
-        //        ab           ~ab            a^b            a|b
-        code[q] = f == 1u ? 1u : f == 4u ? 5u : f == 6u ? 3u : f == 7u ? 7u : 0u;
+        //        ab           ~ab             a^b             a|b
+        code[q] = f == 1u ? 9u : f == 4u ? 13u : f == 6u ? 10u : f == 7u ? 14u : 0u;
         if (swap) {
             if (q < 4) {
                 exchange(tap[2 * q], tap[2 * q + 1]);
@@ -148,17 +152,10 @@ __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restr
             }
         }
     }
-    // liveness from the root down; a live gate is never always 0 below the root
-    uint32_t on[7], taps = 0, codes = (inv[6] << 31) | (kind[6] == 0u ? 1u << 30 : 0u);
-    on[6] = kind[6] != 0u;
+    // a gate is evaluated when its reader is: dead ones keep their codes, which nothing looks at
+    uint32_t codes = (inv[6] << 31) | (kind[6] == 0u ? 1u << 30 : 0u);
 #pragma unroll
-    for (int q = 6; q >= 0; --q) {
-        const uint32_t na = on[q] && kind[q] == 2u, nb = on[q];
-        if (q == 6) on[4] = na, on[5] = nb;
-        else if (q >= 4) on[2 * (q - 4)] = na, on[2 * (q - 4) + 1] = nb;
-        else taps |= (na << (2 * q)) | (nb << (2 * q + 1));
-        codes |= (on[q] ? code[q] : 0u) << (4 * q);
-    }
+    for (int q = 0; q < 7; ++q) codes |= code[q] << (4 * q);
     if (!g.uniform) {
         // the lanes read every tap: one whose value cannot reach the root goes to one shared
         // word, which costs no bank conflicts
@@ -178,11 +175,13 @@ __global__ __launch_bounds__(256) void k_tree_cols_tables(const uint8_t* __restr
         }
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) t[k] = tap[k];
-    t[8] = codes;
-    t[9] = ops;
-    t[10] = taps;
-    t[11] = 0u;
+    for (int k = 0; k < 8; ++k) {
+        t[2 * k] = 4u * (tap[k] & 0xffffu);
+        t[2 * k + 1] = 4u * (tap[k] >> 16);
+    }
+    t[16] = codes;
+    t[17] = ops;
+    t[18] = t[19] = 0u;
 }
 
 // Four words of a node, one per conv position of a pooling window (named words, so that each
@@ -191,34 +190,25 @@ struct Win {
     uint32_t x, y, z, w;
 };
 
-// b = gate(a, b) from the code's low four bits (uniform): nothing for a gate that passes b,
-// else a branch on the pair of gates and one three-input operation per word with a scalar mask.
-// Truth-table immediates over (first, second, third) = 0xF0, 0xCC, 0xAA.
+// b = gate(a, b) from the code's low four bits (uniform): nothing for a gate that passes b, else
+// one three-input operation per word with a scalar mask.  Truth-table immediates over (first,
+// second, third) = 0xF0, 0xCC, 0xAA.
 __device__ __forceinline__ void gate_coded(uint32_t code, const Win& a, Win& b) {
-    if (code & 1u) {
-        const uint32_t m = uint32_t(__builtin_amdgcn_sbfe(int(code), 2, 1));
-        if (code & 2u) {  // m ? a | b : a ^ b
-            b.x = __builtin_amdgcn_bitop3_b32(a.x, b.x, m, 0xBC);
-            b.y = __builtin_amdgcn_bitop3_b32(a.y, b.y, m, 0xBC);
-            b.z = __builtin_amdgcn_bitop3_b32(a.z, b.z, m, 0xBC);
-            b.w = __builtin_amdgcn_bitop3_b32(a.w, b.w, m, 0xBC);
-        } else {  // m ? ~a & b : a & b
-            b.x = __builtin_amdgcn_bitop3_b32(a.x, b.x, m, 0x48);
-            b.y = __builtin_amdgcn_bitop3_b32(a.y, b.y, m, 0x48);
-            b.z = __builtin_amdgcn_bitop3_b32(a.z, b.z, m, 0x48);
-            b.w = __builtin_amdgcn_bitop3_b32(a.w, b.w, m, 0x48);
-            asm volatile("");  // a branch, not selects
-        }
+    const uint32_t m = uint32_t(__builtin_amdgcn_sbfe(int(code), 2, 1));
+    if (code & 1u) {  // m ? ~a & b : a & b
+        b.x = __builtin_amdgcn_bitop3_b32(a.x, b.x, m, 0x48);
+        b.y = __builtin_amdgcn_bitop3_b32(a.y, b.y, m, 0x48);
+        b.z = __builtin_amdgcn_bitop3_b32(a.z, b.z, m, 0x48);
+        b.w = __builtin_amdgcn_bitop3_b32(a.w, b.w, m, 0x48);
+        asm volatile("");  // a branch, not selects
     }
-}
-
-// One channel's table words in scalar registers.
-struct ChanTab {
-    uint32_t t0, t1, t2, t3, t4, t5, t6, t7, codes, on;
-};
-
-__device__ __forceinline__ ChanTab load_tab(const uint32_t* __restrict__ t) {
-    return ChanTab{t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[10]};
+    if (code & 2u) {  // m ? a | b : a ^ b
+        b.x = __builtin_amdgcn_bitop3_b32(a.x, b.x, m, 0xBC);
+        b.y = __builtin_amdgcn_bitop3_b32(a.y, b.y, m, 0xBC);
+        b.z = __builtin_amdgcn_bitop3_b32(a.z, b.z, m, 0xBC);
+        b.w = __builtin_amdgcn_bitop3_b32(a.w, b.w, m, 0xBC);
+        asm volatile("");
+    }
 }
 
 __device__ __forceinline__ uint32_t gate_bits(uint32_t f, uint32_t a, uint32_t b) {
@@ -260,45 +250,55 @@ __device__ __forceinline__ void tree_block_uniform(uint32_t* lds, const uint32_t
         const int cs = nx ? nx->cs : g.P, cout = g.cout;
         const bool last = !nx;
         const uint32_t* src = lds + posb;
-        ChanTab next = load_tab(tab + min(wave_id(), cout - 1) * kTcTabWords);
-        for (int c = wave_id(); c < cout; c += kTcThreads / 64) {
-            // the next channel's table is loaded while this one is evaluated; the empty asm
-            // keeps this one's loads ahead of the branches that use them
-            ChanTab t = next;
-            asm volatile(""
-                         : "+s"(t.t0), "+s"(t.t1), "+s"(t.t2), "+s"(t.t3), "+s"(t.t4), "+s"(t.t5),
-                           "+s"(t.t6), "+s"(t.t7), "+s"(t.codes), "+s"(t.on));
-            next = load_tab(tab + min(c + kTcThreads / 64, cout - 1) * kTcTabWords);
+        const char* srcb = reinterpret_cast<const char*>(src);
+        const uint32_t* t = tab + wave_id() * kTcTabWords;
+        for (int c = wave_id(); c < cout; c += kTcThreads / 64, t += kTcThreads / 64 * kTcTabWords) {
+            // The instruction count bounds this loop (vector and scalar ones together), so a
+            // branch guards each subtree, not each tap.  The empty asm keeps the table's loads
+            // ahead of the branches.
+            uint32_t o[16], codes = t[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) o[k] = t[k];
+            asm volatile("" ::"s"(codes), "s"(o[0]), "s"(o[1]), "s"(o[2]), "s"(o[3]), "s"(o[4]),
+                         "s"(o[5]), "s"(o[6]), "s"(o[7]), "s"(o[8]), "s"(o[9]), "s"(o[10]),
+                         "s"(o[11]), "s"(o[12]), "s"(o[13]), "s"(o[14]), "s"(o[15]));
             Win v0, v1, v2, v3, v4, v5, v6, v7;
-            auto tap = [&](uint32_t bit, uint32_t o, Win& v) {
-                if (t.on & bit) {
-                    const uint32_t* p0 = src + (o & 0xffffu);
-                    const uint32_t* p1 = src + (o >> 16);
-                    v.x = p0[0];
-                    v.y = p0[DY];
-                    v.z = p1[0];
-                    v.w = p1[DY];
-                }
+            auto tap = [&](uint32_t o0, uint32_t o1, Win& v) {
+                const uint32_t* p0 = reinterpret_cast<const uint32_t*>(srcb + o0);
+                const uint32_t* p1 = reinterpret_cast<const uint32_t*>(srcb + o1);
+                v.x = p0[0];
+                v.y = p0[DY];
+                v.z = p1[0];
+                v.w = p1[DY];
             };
-            tap(1u, t.t0, v0);
-            tap(2u, t.t1, v1);
-            tap(4u, t.t2, v2);
-            tap(8u, t.t3, v3);
-            tap(16u, t.t4, v4);
-            tap(32u, t.t5, v5);
-            tap(64u, t.t6, v6);
-            tap(128u, t.t7, v7);
-            gate_coded(t.codes, v0, v1);
-            gate_coded(t.codes >> 4, v2, v3);
-            gate_coded(t.codes >> 8, v4, v5);
-            gate_coded(t.codes >> 12, v6, v7);
-            gate_coded(t.codes >> 16, v1, v3);
-            gate_coded(t.codes >> 20, v5, v7);
-            gate_coded(t.codes >> 24, v3, v7);
+            auto both = [&](int q) { return (codes & (8u << (4 * q))) != 0u; };
+            if (both(6)) {
+                if (both(4)) {
+                    if (both(0)) tap(o[0], o[1], v0);
+                    tap(o[2], o[3], v1);
+                }
+                if (both(1)) tap(o[4], o[5], v2);
+                tap(o[6], o[7], v3);
+            }
+            if (both(5)) {
+                if (both(2)) tap(o[8], o[9], v4);
+                tap(o[10], o[11], v5);
+            }
+            if (both(3)) tap(o[12], o[13], v6);
+            tap(o[14], o[15], v7);
+            if (both(6)) {
+                if (both(4)) gate_coded(codes, v0, v1);
+                gate_coded(codes >> 4, v2, v3);
+                gate_coded(codes >> 16, v1, v3);
+            }
+            if (both(5)) gate_coded(codes >> 8, v4, v5);
+            gate_coded(codes >> 12, v6, v7);
+            gate_coded(codes >> 20, v5, v7);
+            gate_coded(codes >> 24, v3, v7);
             // pool: the OR of the four words, each inverted when the root is
-            const uint32_t root = uint32_t(int(t.codes) >> 31);
+            const uint32_t root = uint32_t(int(codes) >> 31);
             uint32_t r = root;
-            if (!(t.codes & (1u << 30)))
+            if (!(codes & (1u << 30)))
                 r = __builtin_amdgcn_bitop3_b32(v7.x, v7.y, root, 0x7E) |
                     __builtin_amdgcn_bitop3_b32(v7.z, v7.w, root, 0x7E);
             if (last) dst_out[c * cs] = r;
@@ -311,23 +311,28 @@ __device__ __forceinline__ void tree_block_uniform(uint32_t* lds, const uint32_t
 __device__ __forceinline__ void tree_block_lanes(uint32_t* lds, const uint32_t* __restrict__ tab,
                                                  const TreeColsBlock& g, const TreeColsBlock* nx,
                                                  uint32_t* __restrict__ out) {
+    const int dy = g.dy;
     for (int item = threadIdx.x; item < g.cout * g.P; item += kTcThreads) {
         const int c = int(fast_div(uint32_t(item), g.div_p)), p = item - c * g.P;
         const int py = int(fast_div(uint32_t(p), g.div_wp)), px = p - py * g.wp;
-        const int posb = py * 2 * g.dy + px;
+        const int posb = py * 2 * dy + px;
         const uint4* t4 = reinterpret_cast<const uint4*>(tab + c * kTcTabWords);
-        const uint4 ta = t4[0], tb = t4[1], tc = t4[2];
-        const uint32_t off[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
+        const uint32_t ops = tab[c * kTcTabWords + 17];
+        const char* row0 = reinterpret_cast<const char*>(lds + posb);
+        const char* row1 = row0 + 4 * dy;
         uint32_t v[8][4];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int a0 = posb + int(off[k] & 0xffffu), a1 = posb + int(off[k] >> 16);
-            v[k][0] = lds[a0];
-            v[k][1] = lds[a1];
-            v[k][2] = lds[a0 + g.dy];
-            v[k][3] = lds[a1 + g.dy];
+        for (int k = 0; k < 8; k += 2) {
+            const uint4 o = t4[k / 2];  // two taps
+            v[k][0] = *reinterpret_cast<const uint32_t*>(row0 + o.x);
+            v[k][1] = *reinterpret_cast<const uint32_t*>(row0 + o.y);
+            v[k][2] = *reinterpret_cast<const uint32_t*>(row1 + o.x);
+            v[k][3] = *reinterpret_cast<const uint32_t*>(row1 + o.y);
+            v[k + 1][0] = *reinterpret_cast<const uint32_t*>(row0 + o.z);
+            v[k + 1][1] = *reinterpret_cast<const uint32_t*>(row0 + o.w);
+            v[k + 1][2] = *reinterpret_cast<const uint32_t*>(row1 + o.z);
+            v[k + 1][3] = *reinterpret_cast<const uint32_t*>(row1 + o.w);
         }
-        const uint32_t ops = tc.y;
         uint32_t r = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
