@@ -120,6 +120,10 @@ SIGNATURES: dict[str, list] = {
     "cl_packed_bank_layout": [ctypes.POINTER(_i32), ctypes.POINTER(_i32),
                               ctypes.POINTER(_i32), ctypes.POINTER(_i32), _i64, _i64,
                               ctypes.POINTER(_i32)],
+    "cl_packed_bank_orient": [ctypes.POINTER(_i32), ctypes.POINTER(_i32), _i64,
+                              ctypes.POINTER(_i32)],
+    "cl_packed_bank_slots": [ctypes.POINTER(_i64), ctypes.POINTER(_i32), _i64, _i64,
+                             ctypes.POINTER(_i64), ctypes.POINTER(_i32)],
     "cl_adam_clip_max_tensors": [ctypes.POINTER(_i64)],
     "cl_adam_clip_workspace": [_i64, ctypes.POINTER(_i64), ctypes.POINTER(_i64)],
     "cl_adam_clip_step": [_int, _i64, _p, _p, _p, _p, ctypes.POINTER(_i64), _p, _f64, _f64,
@@ -139,6 +143,8 @@ SIGNATURES: dict[str, list] = {
     "cl_eval_packed_indexed_columns": [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p],
     "cl_eval_packed_indexed_pair_columns": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64,
                                             _i64, _i64, _i64, _p],
+    "cl_packed_circuit_limits": [ctypes.POINTER(_i64)] * 4,
+    "cl_packed_circuit": [_p, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)] + [_p] * 7,
     "cl_packed_rows_to_columns": [_p, _p, _i64, _i64, _i64, _p],
     "cl_tree_columns_layout": [ctypes.POINTER(_i64), _i64] + [ctypes.POINTER(_i64)] * 4,
     "cl_tree_columns": [_p, _i64, _i64, ctypes.POINTER(_i64), _i64, ctypes.POINTER(_p),

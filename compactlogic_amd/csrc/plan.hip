@@ -416,3 +416,84 @@ extern "C" int cl_packed_bank_layout(const int32_t* ka, const int32_t* kb, const
     }
     return CL_OK;
 }
+
+// Which gates of a group should read their operands swapped so that every bank is read about as
+// often as operand a as it is as operand b: the gates are the edges of a graph on the banks, a
+// trail that takes every edge once (the edges at a bank paired off, unpaired ends start trails)
+// leaves a bank as often as it enters it, and a gate swaps when the trail takes it from b to a.
+extern "C" int cl_packed_bank_orient(const int32_t* ka, const int32_t* kb, int64_t n,
+                                     int32_t* swap) {
+    cl::clear_error();
+    constexpr int kBanks = 32;
+    CL_ARG(n >= 0 && n < (int64_t(1) << 30), "bad sizes");
+    CL_ARG(n == 0 || (ka && kb && swap), "null pointer argument");
+    std::vector<std::vector<int32_t>> at(kBanks);
+    for (int64_t i = 0; i < n; ++i) {
+        CL_ARG(ka[i] >= 0 && ka[i] < kBanks && kb[i] >= 0 && kb[i] < kBanks,
+               "gate %lld has a bank outside [0, %d)", (long long)i, kBanks);
+        at[size_t(ka[i])].push_back(int32_t(i));
+        at[size_t(kb[i])].push_back(int32_t(i));
+    }
+    std::vector<char> done(size_t(n), 0);
+    auto walk = [&](int v) {
+        while (true) {
+            auto& edges = at[size_t(v)];
+            while (!edges.empty() && done[size_t(edges.back())]) edges.pop_back();
+            if (edges.empty()) return;
+            const int32_t e = edges.back();
+            done[size_t(e)] = 1;
+            swap[e] = ka[e] == v ? 0 : 1;
+            v = ka[e] == v ? kb[e] : ka[e];
+        }
+    };
+    for (int v = 0; v < kBanks; ++v)
+        if (at[size_t(v)].size() % 2) walk(v);  // a trail from an odd bank ends at an odd bank
+    for (int v = 0; v < kBanks; ++v) {
+        size_t left = 1;
+        while (left) {
+            walk(v);
+            auto& edges = at[size_t(v)];
+            while (!edges.empty() && done[size_t(edges.back())]) edges.pop_back();
+            left = edges.size();
+        }
+    }
+    return CL_OK;
+}
+
+// Slots (banks) of gates inside their blocks of 32: gate i is read by the groups
+// grp[ptr[i] .. ptr[i + 1]), load[group][bank] counts the reads placed so far.  The most read
+// gates of a block choose first, each the free slot whose bank its readers read least.
+extern "C" int cl_packed_bank_slots(const int64_t* ptr, const int32_t* grp, int64_t n,
+                                    int64_t groups, int64_t* load, int32_t* slot) {
+    cl::clear_error();
+    constexpr int64_t kBanks = 32;
+    CL_ARG(n >= 0 && groups >= 0, "bad sizes");
+    if (n == 0) return CL_OK;
+    CL_ARG(ptr && slot && ptr[0] >= 0, "null pointer argument");
+    for (int64_t i = 0; i < n; ++i) CL_ARG(ptr[i + 1] >= ptr[i], "bad row pointers");
+    CL_ARG(ptr[n] == ptr[0] || (grp && load), "null pointer argument");
+    for (int64_t i = ptr[0]; i < ptr[n]; ++i)
+        CL_ARG(grp[i] >= 0 && grp[i] < groups, "group outside [0, %lld)", (long long)groups);
+    for (int64_t b0 = 0; b0 < n; b0 += kBanks) {
+        const int64_t size = std::min(n - b0, kBanks);
+        std::vector<int64_t> order(static_cast<size_t>(size));
+        std::iota(order.begin(), order.end(), b0);
+        std::stable_sort(order.begin(), order.end(), [&](int64_t x, int64_t y) {
+            return ptr[x + 1] - ptr[x] > ptr[y + 1] - ptr[y];
+        });
+        bool used[kBanks] = {};
+        for (int64_t g : order) {
+            int64_t best = -1, cost = 0;
+            for (int64_t j = 0; j < size; ++j) {
+                if (used[j]) continue;
+                int64_t c = 0;
+                for (int64_t i = ptr[g]; i < ptr[g + 1]; ++i) c += load[grp[i] * kBanks + j];
+                if (best < 0 || c < cost) best = j, cost = c;
+            }
+            used[best] = true;
+            for (int64_t i = ptr[g]; i < ptr[g + 1]; ++i) ++load[grp[i] * kBanks + best];
+            slot[g] = int32_t(best);
+        }
+    }
+    return CL_OK;
+}

@@ -18,6 +18,7 @@ import torch
 from . import _capi
 from . import timing
 from . import difflogic_hip as _dl
+from . import packed_circuit as _pc
 from .layers import ConvLayer, GroupSum, LogicLayer, PackBitsTensor
 from .treelogic import ConvLogicLayer
 
@@ -193,6 +194,34 @@ def _column_words(layout: dict, layer: int, pos: np.ndarray) -> np.ndarray:
     return layout["base"][layer] + pos
 
 
+class _Circuit:
+    """A tail's pruned circuit (packed_circuit.build) on the device."""
+
+    @classmethod
+    def of(cls, layers: list, in_rows: int, k: int, device):
+        """The circuit of layers [(a, b, opcode), ...], or None where it does not fit."""
+        plan = _pc.build(_pc.fold(layers, in_rows), k)
+        return None if plan is None else cls(plan, in_rows, device)
+
+    def __init__(self, plan: dict, in_rows: int, device):
+        def dev(name, dtype=np.int32):
+            return torch.as_tensor(plan[name].view(dtype), device=device)
+
+        self.in_rows, self.k = in_rows, plan["shape"][5]
+        self.shape = (ctypes.c_int64 * 8)(*plan["shape"])
+        self.tabs = [dev(name) for name in ("ent", "dst", "in", "cnt", "ones")]
+        self.gates = plan["gates"]
+
+    def __call__(self, words, cols: int, columns_major: bool, in_words: int, n: int):
+        counts = torch.empty((n, self.k), dtype=torch.int32, device=words.device)
+        with torch.cuda.device(words.device):
+            timing.timed(f"cl_packed_circuit[{self.in_rows}]", lambda: _capi.call(
+                "cl_packed_circuit", words.data_ptr(), cols, int(columns_major), in_words, n,
+                self.shape, *[t.data_ptr() for t in self.tabs], counts.data_ptr(),
+                _dl.stream_of(words)))
+        return counts
+
+
 class PackedNetwork:
     """Fused packed evaluator of `model` (frozen or in eval mode; each neuron uses its argmax
     slot `w`), ending in a GroupSum.  Call it with a PackBitsTensor of the network's input (or
@@ -208,7 +237,8 @@ class PackedNetwork:
     (cl_packed_network_columns).  When no tail qualifies every module runs layer by
     layer and the counts come from the group popcount.  A fused tail whose prefix is complete
     ConvLogicLayers alone takes its input column-major from them (cl_tree_columns: all blocks on
-    one column in LDS).  The gate tables are built once here;
+    one column in LDS).  A fused tail without a producer is reduced to the two-input gates that
+    reach an output (packed_circuit) where those fit.  The gate tables are built once here;
     rebuild after changing the model.  With `bank_aware` (default), each fused layer's rows
     are laid out in LDS by bank_aware_positions, so that the row reads of the kernel's
     half-waves hit distinct LDS banks; the counts do not depend on the layout.
@@ -253,6 +283,7 @@ class PackedNetwork:
         if not layers:
             self.rows = None            # no fused tail: layer by layer, then the popcount
             self.device = None
+            self.circuit = None
             return
         self.rows = [int(layers[0].in_dim)] + [int(m.out_dim) for m in layers]
         for i, (prev, m) in enumerate(zip(self.rows[:-1], layers)):
@@ -283,6 +314,17 @@ class PackedNetwork:
                         int(b.max()) >= m.in_dim:
                     raise IndexError("connection indices out of range")
                 wiring.append((a.cpu().numpy(), b.cpu().numpy(), g.cpu().numpy(), a.device))
+            self.device = layers[0].weights.device
+            # the pruned circuit of the tail, where it fits, in place of the row tables: 22800
+            # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.47 ms for 4 M samples, all
+            # rows 3.94; the 2 x 16000 tail of a logic-tree network 0.32 ms for 1 M, 0.57
+            self.circuit = None
+            if (bank_aware and self.producer is None and self.rows[0] <= _LDS_INPUT_ROWS
+                    and self.k <= 1024):
+                self.circuit = _Circuit.of([w[:3] for w in wiring], self.rows[0], self.k,
+                                           self.device)
+            if self.circuit is not None:
+                return
             prev_pos = np.arange(self.rows[0], dtype=np.int64)   # input rows stay in place
             lay = self.layout
             self.col_order = None
@@ -330,7 +372,6 @@ class PackedNetwork:
                     front_entries.append(torch.as_tensor(ent, device=dev))
         self.tables = torch.cat(entries).contiguous()
         self.front_tables = torch.cat(front_entries).contiguous() if front_entries else None
-        self.device = self.tables.device
         self._rows_host = (ctypes.c_int64 * len(self.rows))(*self.rows)
 
     def __call__(self, x) -> torch.Tensor:
@@ -360,6 +401,10 @@ class PackedNetwork:
         if words.dim() != 2 or words.shape[0] != self.rows[0]:
             raise RuntimeError(f"x must be [{self.rows[0]}, words], got {tuple(words.shape)}")
         row_bytes = words.shape[1] * words.element_size()
+        if self.circuit is not None:
+            if row_bytes % 4:
+                raise RuntimeError("packed rows must be a multiple of 4 bytes")
+            return self.circuit(words, row_bytes // 4, False, 0, n)
         counts = torch.empty((n, self.k), dtype=torch.int32, device=words.device)
         with torch.cuda.device(words.device):
             timing.timed(f"cl_packed_network[{self.rows[0]}->{self.rows[-1]}]", lambda: _capi.call(
@@ -462,6 +507,8 @@ class PackedNetwork:
             timing.timed(f"cl_tree_columns[{rows}->{self.rows[0]}]", lambda: _capi.call(
                 "cl_tree_columns", colmaj.data_ptr(), cols, rows, geo, len(blocks), *ptrs,
                 tables.data_ptr(), mid.data_ptr(), in_words, stream))
+            if self.circuit is not None:
+                return self.circuit(mid, cols, True, in_words, n)
             counts = ints(n, self.k)
             timing.timed(f"cl_packed_network_columns[{self.rows[0]}->{self.rows[-1]}]",
                          lambda: _capi.call(

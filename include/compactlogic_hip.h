@@ -137,6 +137,16 @@ int cl_plan_locality_order(const int32_t* ra, const int32_t* rb, int64_t num_run
 int cl_packed_bank_layout(const int32_t* ka, const int32_t* kb, const int32_t* fa,
                           const int32_t* fb, int64_t n, int64_t class_size, int32_t* pos);
 
+/* Host functions that level the bank reads of a group of gates before and after the layout above.
+ * cl_packed_bank_orient: swap[i] is 1 where gate i should read its operands in the other order, so
+ * that every bank is read about as often as operand a as it is as operand b.
+ * cl_packed_bank_slots: n gates in blocks of 32; gate i is read by the groups grp[ptr[i] ..
+ * ptr[i + 1]), load (int64 [groups, 32], updated) counts a group's reads per bank; slot[i] is the
+ * gate's place in its block, chosen so that the groups read every bank about equally often. */
+int cl_packed_bank_orient(const int32_t* ka, const int32_t* kb, int64_t n, int32_t* swap);
+int cl_packed_bank_slots(const int64_t* ptr, const int32_t* grp, int64_t n, int64_t groups,
+                         int64_t* load, int32_t* slot);
+
 /* Probabilities (softmax of w over the slots when `softmax` is non-zero, else w itself;
  * written to `probs` when not NULL) and the run coefficients K (run_coef, 16-byte aligned).
  * With inv_coef (T [2 * num_runs, 2], may be NULL) the coefficients of every inverse-index
@@ -648,6 +658,25 @@ int cl_eval_packed_indexed_pair_columns(const void* x, const int32_t* ia1, const
 int cl_packed_network_columns(const void* x, int64_t cols, int64_t in_words, int64_t nsamples,
                               const uint64_t* tables, const int64_t* rows_host,
                               int64_t num_layers, int64_t k, int32_t* counts, void* stream);
+
+/* A pruned packed network on LDS pages (packed_circuit.py builds the tables): step by step, the
+ * two-input gates left of a frozen network, then the class counts, 64 samples at a time.
+ * cl_packed_circuit_limits (host only): the most LDS words per 32-sample plane (pages of 64), gate
+ * slots per thread, count steps and input rows.
+ * cl_packed_circuit: x is [rows, cols] 32-bit words, or column-major [cols, in_words] when
+ * columns_major; shape (host int64 [8]) = batches of four slots, bit mask of the batches that
+ * begin a step, count groups, inverted count groups, input rows staged, k, LDS words, 1 if the
+ * counts read inputs.  ent [slots, 1024]: LDS byte addresses of the operands, a | b << 16, with
+ * the gate's values for ab = 01, 10, 11 in bits 0, 1 and 16 (00 gives 0); dst [16, max slots /
+ * 2]: a wave's page words, two slots to an entry (0xffff: none); in [rows staged]: input row | LDS
+ * word << 16; cnt [groups + inverted groups, k, 64, 2]: LDS byte addresses, two to an entry; ones
+ * [k]: added to the counts.  counts int32 [nsamples, k].  Page 0 holds zeros; a step reads pages of earlier steps only. */
+int cl_packed_circuit_limits(int64_t* max_words, int64_t* max_slots, int64_t* max_steps,
+                             int64_t* max_inputs);
+int cl_packed_circuit(const void* x, int64_t cols, int64_t columns_major, int64_t in_words,
+                      int64_t nsamples, const int64_t* shape, const uint32_t* ent,
+                      const uint32_t* dst, const uint32_t* in, const uint32_t* cnt,
+                      const int32_t* ones, int32_t* counts, void* stream);
 
 /* Packed rows to columns: y[c * out_words + r] (32-bit words) = word c of row r of x
  * [rows, row_bytes], out_words >= rows; words past the rows of a column are not written. */

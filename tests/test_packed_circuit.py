@@ -1,0 +1,130 @@
+"""The pruned circuit of a packed network (packed_circuit.fold / build): its tables, evaluated as
+the kernel does, give the layers' class counts; on the GPU the kernel over several columns per
+workgroup."""
+import numpy as np
+import pytest
+import torch
+
+from compactlogic_amd import packed_circuit as PC
+from compactlogic_amd.packed_net import _Circuit
+
+ALL = np.uint64(0xFFFFFFFFFFFFFFFF)
+
+
+def random_layers(dims, seed, gates=range(16), strays=False):
+    r = np.random.default_rng(seed)
+    layers = []
+    for i, o in dims:
+        lo, hi = (-1, i + 1) if strays else (0, i)
+        layers.append((r.integers(lo, hi, o), r.integers(lo, hi, o),
+                       r.choice(np.array(list(gates)), o)))
+    return layers
+
+
+def words_of(gate, a, b):
+    f = [np.where((gate >> s) & 1, ALL, np.uint64(0)) for s in (3, 2, 1, 0)]
+    return (~a & ~b & f[0]) | (~a & b & f[1]) | (a & ~b & f[2]) | (a & b & f[3])
+
+
+def reference_counts(layers, k, x):
+    """A negative row reads 0; a row past the layer before makes the gate 0."""
+    h = x
+    for a, b, g in layers:
+        rows = h.size
+        h = np.append(h, np.uint64(0))
+        bad = (a >= rows) | (b >= rows)
+        av, bv = (h[np.where((v < 0) | (v >= rows), rows, v)] for v in (a, b))
+        h = words_of(np.where(bad, 0, g), av, bv)
+    bits = (h[:, None] >> np.arange(64, dtype=np.uint64)) & np.uint64(1)
+    return bits.reshape(k, -1, 64).sum(1).T.astype(np.int64)
+
+
+def table_counts(plan, k, x, rng):
+    """The kernel's walk over the tables on one column of 64 samples; every step reads the words
+    as they were when it began, and the next column's input is staged before the counts."""
+    batches, start, groups, inverted, in_rows, kk, words, hold = plan["shape"]
+    assert kk == k
+    lds = rng.integers(0, 2**63, words).astype(np.uint64)
+    lds[:64] = 0
+    rows, at = plan["in"][:in_rows] & 0xFFFF, plan["in"][:in_rows] >> 16
+    lds[at] = x[rows]
+    dst = np.stack([plan["dst"] & 0xFFFF, plan["dst"] >> 16], 2).reshape(16, -1)
+    for b in range(batches):
+        if b == 0 or (start >> b) & 1:
+            old = lds.copy()
+        for q in range(4 * b, 4 * b + 4):
+            for w in range(16):
+                tag = int(dst[w, q])
+                if tag == 0xFFFF:
+                    continue
+                e = plan["ent"][q, 64 * w:64 * w + 64].astype(np.int64)
+                f01, f10, f11 = e & 1, (e >> 1) & 1, (e >> 16) & 1
+                lds[tag:tag + 64] = words_of(f01 << 2 | f10 << 1 | f11, old[(e & 0xFFFC) // 4],
+                                             old[((e >> 16) & 0xFFFC) // 4])
+    if not hold:
+        lds[at] = rng.integers(0, 2**63, in_rows).astype(np.uint64)
+    out = np.tile(plan["ones"].astype(np.int64), (64, 1))
+    if groups + inverted:
+        cnt = plan["cnt"]
+        at = np.stack([cnt & 0xFFFF, cnt >> 16], 4).reshape(groups + inverted, k, 64, 4) // 4
+        v = lds[at]
+        v[groups:] = ~v[groups:]
+        bits = (v[..., None] >> np.arange(64, dtype=np.uint64)) & np.uint64(1)
+        out += bits.sum((0, 2, 3)).T.astype(np.int64)
+    return out
+
+
+CASES = [
+    ([(40, 64), (64, 60)], 6, range(16), False),
+    ([(17, 33), (33, 40)], 5, range(16), True),              # rows outside the layer before
+    ([(12, 20)] + [(20, 20)] * 14 + [(20, 30)], 3, range(16), False),
+    ([(6, 10)], 10, (3, 5, 10, 12), False),                  # outputs are inputs only
+    ([(6, 10)], 2, (0, 15), False),                          # constants only
+    ([(50, 700), (700, 640)], 1, (1, 6, 8, 9), False),       # one class, whole pages of a kind
+    ([(300, 6000), (6000, 5000)], 20, range(16), False),
+    ([(64, 8000), (8000, 10000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # steps split
+]
+
+
+@pytest.mark.parametrize("dims,k,gates,strays", CASES)
+def test_tables_give_the_layers_counts(dims, k, gates, strays):
+    rng = np.random.default_rng(k)
+    layers = random_layers(dims, k, gates, strays)
+    plan = PC.build(PC.fold(layers, dims[0][0]), k)
+    for _ in range(2):
+        x = rng.integers(0, 2**63, dims[0][0]).astype(np.uint64)
+        assert np.array_equal(table_counts(plan, k, x, rng), reference_counts(layers, k, x))
+
+
+def test_what_does_not_fit_is_refused():
+    lim = PC.limits()
+    wide = random_layers([(lim["inputs"], lim["words"] + 64)], 1, (1, 6))
+    assert PC.build(PC.fold(wide, lim["inputs"]), 1) is None                 # LDS words
+    many = random_layers([(lim["inputs"] + 900, 16000)], 2, (1, 6))
+    assert PC.build(PC.fold(many, lim["inputs"] + 900), 1000) is None        # input rows
+    tall = random_layers([(64, 128 * lim["steps"])], 3, (3, 5))
+    assert PC.build(PC.fold(tall, 64), 1) is None                            # entries of a class
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,k,gates,strays", CASES)
+@pytest.mark.parametrize("n", [40000, 33])
+def test_circuit_kernel(device, dims, k, gates, strays, n):
+    """Several columns per workgroup (256 workgroups take 16384 samples at a time), row-major and
+    column-major input."""
+    rng = np.random.default_rng(k)
+    layers = random_layers(dims, k, gates, strays)
+    rows = dims[0][0]
+    cols = -(-n // 32)
+    x = rng.integers(0, 2**32, (rows, cols), dtype=np.uint64).astype(np.uint32)
+    wide = np.zeros((rows, cols + cols % 2), dtype=np.uint32)
+    wide[:, :cols] = x
+    ref = np.concatenate([reference_counts(layers, k, c)
+                          for c in wide.view(np.uint64).T])[:n]
+    circuit = _Circuit.of(layers, rows, k, device)
+    xt = torch.as_tensor(x.view(np.int32), device=device)
+    assert np.array_equal(circuit(xt, cols, False, 0, n).cpu().numpy(), ref)
+    pitch = rows + 3
+    xc = torch.full((cols, pitch), -1, dtype=torch.int32, device=device)
+    xc[:, :rows] = xt.t()
+    assert np.array_equal(circuit(xc, cols, True, pitch, n).cpu().numpy(), ref)
