@@ -615,18 +615,22 @@ def bench_packed_fused(model, in_features: int, log2n: int, passes: int, checksu
     with timing.record() as rec:
         net(x)
     calls = rec.summary()
-    fused_call = next((v for k, v in calls.items() if k.startswith("cl_packed_network")), None)
+    fused_call = next((v for k, v in calls.items()
+                       if k.startswith(("cl_packed_circuit", "cl_packed_network"))), None)
+    circuit = net.circuit
     fused_rows = net.rows or []
     prefix = len(net.prefix)
-    producer = net.producer is not None
+    producer = net.producer is not None and circuit is None
     del xw, counts, net
     torch.cuda.empty_cache()
     out = {"workload": ("the same network and inputs through PackedNetwork: "
                         + (f"{prefix} modules layer by layer, then " if prefix else "")
                         + ("the layer before the dense tail written column-major, then "
                            if producer else "")
-                        + f"the dense layers {fused_rows} and the class counts in one launch, "
-                          "32-sample columns held in LDS through all fused layers"),
+                        + (f"the {circuit.gates} two-input gates that reach an output of the "
+                           f"layers of {circuit.in_rows} inputs" if circuit is not None
+                           else f"the dense layers {fused_rows}")
+                        + " and the class counts in one launch, columns held in LDS"),
            "value": round(n / dt / 1e9, 4), "unit": "Gsamples/s", "ms_per_pass": round(dt * 1e3, 3),
            "counts_match_layerwise": same, "speedup_vs_layerwise": None,
            "kernels": {k: {"ms": round(v["mean_ms"], 4), "calls_per_step": v["calls"]}
@@ -636,7 +640,7 @@ def bench_packed_fused(model, in_features: int, log2n: int, passes: int, checksu
         out["fused_compulsory_bytes_per_sample"] = fused_bytes
         out["hbm_frac_of_fused_bytes"] = round(fused_bytes * n / dt / 1e9 / HBM_PEAK_GBS, 4)
     if fused_call is not None:
-        # the fused kernel keeps its activations in LDS and is bound by VALU issue
+        # the fused kernel keeps its activations in LDS: against VALU issue, not memory
         roof = valu_roofline(key, fused_call["mean_ms"] * 1e-3)
         if roof is not None:
             out["roofline"] = roof

@@ -144,7 +144,7 @@ SIGNATURES: dict[str, list] = {
     "cl_eval_packed_indexed_pair_columns": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i64,
                                             _i64, _i64, _i64, _p],
     "cl_packed_circuit_limits": [ctypes.POINTER(_i64)] * 4,
-    "cl_packed_circuit": [_p, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)] + [_p] * 7,
+    "cl_packed_circuit": [_p, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)] + [_p] * 8,
     "cl_packed_rows_to_columns": [_p, _p, _i64, _i64, _i64, _p],
     "cl_tree_columns_layout": [ctypes.POINTER(_i64), _i64] + [ctypes.POINTER(_i64)] * 4,
     "cl_tree_columns": [_p, _i64, _i64, ctypes.POINTER(_i64), _i64, ctypes.POINTER(_p),

@@ -8,8 +8,8 @@ pruning idea of the reference's compiler (compiler/prune.py:164-367) applied to 
 evaluator's tables.
 
 `build` schedules the gates in steps (a barrier between them; a gate's sources come from earlier
-steps), places every signal in LDS and lays the tables out.  A page is 64 words, the gates of one
-wave; it is reused after the last step that reads one of its signals, so signals that are last
+steps), places every signal in LDS and lays the tables out.  A page is 64 signals, the gates of
+one wave; it is reused after the last step that reads one of its signals, so signals that are last
 read in the same step share pages.
 """
 from __future__ import annotations
@@ -22,9 +22,14 @@ import numpy as np
 from . import _capi
 
 _PAGE = 64
+_PAGE_WORDS = 128   # two words of 32 samples per signal
 _WAVES = 16
 _THREADS = 1024
-_BATCH = 4          # slots per batch; a step begins with a batch
+_NONE = 0xFFFF
+# a step begins with a slot that is a multiple of this, in the order tried: reads of four slots
+# are in flight together, and a step that begins between them cuts that in two
+_ALIGN = (4, 2)
+_MAX_SPLIT = 4
 # smallest number of a step's gates with a death step of their own, in the order tried: fewer
 # groups read LDS with fewer bank conflicts, more free pages earlier
 _MIN_GROUPS = (1024, 192)
@@ -33,7 +38,7 @@ _MIN_GROUPS = (1024, 192)
 def limits() -> dict:
     v = [ctypes.c_int64(0) for _ in range(4)]
     _capi.call("cl_packed_circuit_limits", *[ctypes.byref(c) for c in v])
-    return dict(zip(("words", "slots", "steps", "inputs"), (c.value for c in v)))
+    return dict(zip(("pages", "slots", "steps", "input_pages"), (c.value for c in v)))
 
 
 # truth tables as columns (00, 01, 10, 11) over (a, b); column orders of the foldings below
@@ -89,11 +94,14 @@ def fold(layers: list, in_rows: int) -> dict:
             "out_inv": inv, "out_const": const, "live": live}
 
 
-def _groups(death: np.ndarray, smallest: int) -> list:
+def _groups(death: np.ndarray, smallest: int, end: int) -> list:
     """Index groups of equal death step, earliest first; groups below `smallest` join the next
-    later one."""
+    later one, but not the signals that the counts read (death step `end`)."""
     out, rest = [], np.zeros(0, dtype=np.int64)
     for d in np.unique(death):
+        if d == end and rest.size:
+            out.append(rest)
+            rest = np.zeros(0, dtype=np.int64)
         rest = np.concatenate((rest, np.nonzero(death == d)[0]))
         if rest.size >= smallest:
             out.append(rest)
@@ -154,66 +162,98 @@ def _by_bank(w: np.ndarray) -> np.ndarray:
     return w[np.lexsort((w % 32, rank))]
 
 
-def build(c: dict, k: int, splits=(1, 2, 3, 4)) -> dict | None:
-    """Tables for fold's result c with k classes, or None when the circuit does not fit.  A level
-    split into more steps frees its sources' pages earlier and costs barriers: the first split
-    that fits is taken."""
+def build(c: dict, k: int) -> dict | None:
+    """Tables for fold's result c with k classes, or None when the circuit does not fit.  A layer
+    split into more steps frees its sources' pages earlier and costs barriers and slots: a layer
+    whose gates find no page is split once more."""
     lim = limits()
-    for split in splits:
-        for smallest in _MIN_GROUPS:
-            plan = _build(c, k, split, smallest, lim)
+    for smallest in _MIN_GROUPS:
+        for align in _ALIGN:
+            split = {}
+            while True:
+                plan = _build(c, k, split, smallest, align, lim)
+                if not isinstance(plan, int):
+                    break
+                split[plan] = split.get(plan, 1) + 1
+                if split[plan] > _MAX_SPLIT:
+                    plan = None
+                    break
             if plan is not None:
                 return plan
     return None
 
 
-def _build(c: dict, k: int, split: int, smallest: int, lim: dict) -> dict | None:
+def _copied_outputs(c: dict) -> dict:
+    """c with outputs that are inputs read from gates of the last layer that copy them: the next
+    column's input is staged while the counts run."""
+    n_in, gates = c["in_rows"], c["a"].size
+    is_in = (c["out_const"] < 0) & (c["out"] < n_in)
+    ids = np.unique(c["out"][is_in])
+    if not ids.size:
+        return c
+    out = c["out"].copy()
+    out[is_in] = n_in + gates + np.searchsorted(ids, out[is_in])
+    last = int(c["layer"][c["live"][n_in:]].max(initial=0))
+    return {**c, "a": np.concatenate((c["a"], ids)), "b": np.concatenate((c["b"], ids)),
+            "bits": np.concatenate((c["bits"], np.full(ids.size, 7))),
+            "layer": np.concatenate((c["layer"], np.full(ids.size, last))), "out": out,
+            "live": np.concatenate((c["live"], np.ones(ids.size, dtype=bool)))}
+
+
+def _build(c: dict, k: int, split: dict, smallest: int, align: int, lim: dict):
+    """The tables, the layer that finds no page, or None when something else does not fit."""
     from .packed_net import bank_aware_positions
 
+    c = _copied_outputs(c)
     n_in, a, b, bits = c["in_rows"], c["a"].copy(), c["b"].copy(), c["bits"].copy()
     live, layer = c["live"], c["layer"]
+    is_out = c["out_const"] < 0
+    counted = np.zeros(live.size, dtype=bool)
+    counted[c["out"][is_out]] = True
     steps = []
     for l in np.unique(layer):
         q = np.nonzero((layer == l) & live[n_in:])[0]
+        # the gates that the counts read last: they stay off the pages of input (below), and the
+        # other pages are free by then
+        q = q[np.argsort(counted[n_in + q], kind="stable")]
         if q.size:
-            parts = min(split, max(1, q.size // (_PAGE * _WAVES)))
+            parts = min(split.get(int(l), 1), max(1, q.size // (_PAGE * _WAVES)))
             steps += np.array_split(q, parts)
     end = len(steps)
     death = np.full(live.size, -1, dtype=np.int64)
     for s, q in enumerate(steps):
         death[a[q]] = death[b[q]] = s
-    is_out = c["out_const"] < 0
-    death[c["out"][is_out]] = end
-    steps = [[q[g] for g in _groups(death[n_in + q], smallest)] for q in steps]
+    death[counted] = end
+    steps = [[q[g] for g in _groups(death[n_in + q], smallest, end)] for q in steps]
     groups = [g for step in steps for g in step]
     gates = np.concatenate(groups) if groups else np.zeros(0, dtype=np.int64)
     gid = np.repeat(np.arange(len(groups)), [g.size for g in groups])
     banks = _Banks(np.concatenate((gid, gid)), np.concatenate((a[gates], b[gates])), live.size,
                    len(groups))
 
-    max_pages = lim["words"] // _PAGE
-    free = list(range(1, max_pages))               # page 0: zeros
+    free = list(range(1, lim["pages"]))            # page 0: zeros
     word = np.full(live.size, -1, dtype=np.int64)
     dying = [[] for _ in range(end + 1)]
     peak = 1
 
     ins = np.nonzero(live[:n_in])[0]
-    if ins.size > lim["inputs"]:
-        return None
-    in_pages = 0
-    for grp in _groups(death[ins], smallest):
+    in_rows = []
+    for grp in _groups(death[ins], smallest, end):
         ids = banks.slots(ins[grp])
         for p0 in range(0, ids.size, _PAGE):
-            if not free:
+            if not free or len(in_rows) == lim["input_pages"]:
                 return None
-            page = heapq.heappop(free)
+            page = heapq.heappop(free)             # pages 1, 2, ... in turn
             part = ids[p0:p0 + _PAGE]
-            word[part] = page * _PAGE + np.arange(part.size)
+            word[part] = page * _PAGE_WORDS + np.arange(part.size)
             dying[int(death[part].max())].append(page)
-            in_pages = max(in_pages, page + 1)
-    peak = max(peak, in_pages)
+            in_rows.append(np.pad(part, (0, _PAGE - part.size), constant_values=_NONE))
+    if ins.size and ins[-1] >= _NONE:
+        return None
+    in_pages = len(in_rows)
+    peak += in_pages
 
-    slots, start, ent, dst = 0, 0, [], []
+    slots, start, ent, ops, dst = 0, 0, [], [], []
     for s, step in enumerate(steps):
         pages = []
         for g in step:
@@ -230,37 +270,43 @@ def _build(c: dict, k: int, split: int, smallest: int, lim: dict) -> dict | None
                 # gates the counts read stay off the input pages, which the next column's
                 # input is staged to while the counts run
                 skip = []
-                while free and last == end and free[0] < in_pages:
+                while free and last == end and free[0] <= in_pages:
                     skip.append(heapq.heappop(free))
                 if not free:
-                    return None
+                    return int(layer[part[0]])
                 page = heapq.heappop(free)
                 for v in skip:
                     heapq.heappush(free, v)
                 peak = max(peak, page + 1)
-                word[n_in + part] = page * _PAGE + np.arange(part.size)
+                word[n_in + part] = page * _PAGE_WORDS + np.arange(part.size)
                 dying[last].append(page)
                 pages.append((page, part))
         need = -(-len(pages) // _WAVES)
-        need = -(-need // _BATCH) * _BATCH
+        need = -(-need // align) * align
         if slots + need > lim["slots"]:
             return None
-        start |= 1 << (slots // _BATCH)
+        start |= 1 << (slots // 2)
         e = np.zeros((need, _THREADS), dtype=np.uint32)
-        d = np.full((_WAVES, need), 0xFFFF, dtype=np.uint32)
+        o = np.zeros((need, _THREADS), dtype=np.uint32)
+        d = np.full((_WAVES, need), _NONE, dtype=np.uint32)
         for i, (page, part) in enumerate(pages):
             w, j = i % _WAVES, i // _WAVES
-            t = bits[part]
-            e[j, w * _PAGE + np.arange(part.size)] = \
-                4 * word[a[part]] | 4 * word[b[part]] << 16 | t & 3 | (t & 4) << 14
-            d[w, j] = page * _PAGE
+            lanes = w * _PAGE + np.arange(part.size)
+            e[j, lanes] = word[a[part]] | word[b[part]] << 16
+            o[j, lanes] = bits[part]
+            d[w, j] = page * _PAGE_WORDS
         slots += need
-        ent.append(e), dst.append(d)
+        ent.append(e), ops.append(o), dst.append(d)
         for page in dying[s]:
             heapq.heappush(free, page)
 
-    pad = lim["slots"] - slots
-    dst_all = np.concatenate(dst + [np.full((_WAVES, pad), 0xFFFF, dtype=np.uint32)], 1)
+    none = np.zeros((0, _THREADS), dtype=np.uint32)
+    ent = np.concatenate(ent + [none])
+    ops = np.concatenate(ops + [np.zeros((-slots % 8, _THREADS), dtype=np.uint32)])
+    ops = np.bitwise_or.reduce(ops.reshape(-1, 8, _THREADS) <<
+                               (4 * np.arange(8, dtype=np.uint32)).reshape(1, 8, 1), axis=1)
+    pad = np.full((_WAVES, lim["slots"] - slots), _NONE, dtype=np.uint32)
+    dst = np.concatenate(dst + [pad], 1)
 
     # outputs: per class the words counted as they are and those counted inverted, each padded
     # with the zero page to whole groups of four entries per lane
@@ -280,20 +326,20 @@ def _build(c: dict, k: int, split: int, smallest: int, lim: dict) -> dict | None
             if flip:
                 ones[cls] -= 4 * n * _PAGE - v.size
         groups.append(n)
-        # [group][class][lane][2]: four byte addresses of 16 bits
-        t = 4 * tab.reshape(k, n, 2, 2, _PAGE)
+        t = tab.reshape(k, n, 2, 2, _PAGE)         # to [group][class][lane][2], 16 bits each
         cnt.append((t[:, :, :, 0] | (t[:, :, :, 1] << 16)).transpose(1, 0, 3, 2))
     if 4 * sum(groups) > lim["steps"]:
         return None
     cnt = np.ascontiguousarray(np.concatenate(cnt)).astype(np.uint32)
+
+    def some(t):                                   # a table the kernel gets a pointer to
+        return t if t.size else np.zeros(1, dtype=t.dtype)
+
     return {
-        "shape": (slots // _BATCH, start, groups[0], groups[1], int(ins.size), k, peak * _PAGE,
-                  int((out[is_out] < n_in).any())),
-        "ent": np.concatenate(ent) if ent else np.zeros((1, _THREADS), dtype=np.uint32),
-        "dst": (dst_all[:, 0::2] | (dst_all[:, 1::2] << 16)).astype(np.uint32),
-        "in": (ins | (word[ins] << 16)).astype(np.uint32) if ins.size else
-        np.zeros(1, dtype=np.uint32),
-        "cnt": cnt if cnt.size else np.zeros(1, dtype=np.uint32),
-        "ones": ones.astype(np.int32),
+        "shape": (slots // 2, start, groups[0], groups[1], in_pages, k, peak),
+        "ent": some(ent), "ops": some(ops),
+        "dst": (dst[:, 0::2] | (dst[:, 1::2] << 16)).astype(np.uint32),
+        "in": some(np.array(in_rows).astype(np.uint16).reshape(-1)),
+        "cnt": some(cnt), "ones": ones.astype(np.int32),
         "gates": int(gates.size), "levels": end,
     }

@@ -204,12 +204,13 @@ class _Circuit:
         return None if plan is None else cls(plan, in_rows, device)
 
     def __init__(self, plan: dict, in_rows: int, device):
-        def dev(name, dtype=np.int32):
-            return torch.as_tensor(plan[name].view(dtype), device=device)
+        def dev(name):
+            a = plan[name]
+            return torch.as_tensor(a.view(np.int16 if a.itemsize == 2 else np.int32), device=device)
 
         self.in_rows, self.k = in_rows, plan["shape"][5]
-        self.shape = (ctypes.c_int64 * 8)(*plan["shape"])
-        self.tabs = [dev(name) for name in ("ent", "dst", "in", "cnt", "ones")]
+        self.shape = (ctypes.c_int64 * 7)(*plan["shape"])
+        self.tabs = [dev(name) for name in ("ent", "ops", "dst", "in", "cnt", "ones")]
         self.gates = plan["gates"]
 
     def __call__(self, words, cols: int, columns_major: bool, in_words: int, n: int):
@@ -237,8 +238,9 @@ class PackedNetwork:
     (cl_packed_network_columns).  When no tail qualifies every module runs layer by
     layer and the counts come from the group popcount.  A fused tail whose prefix is complete
     ConvLogicLayers alone takes its input column-major from them (cl_tree_columns: all blocks on
-    one column in LDS).  A fused tail without a producer is reduced to the two-input gates that
-    reach an output (packed_circuit) where those fit.  The gate tables are built once here;
+    one column in LDS).  Where it fits, a fused tail, or the whole network when the layers that
+    write its columns come first, is reduced to the two-input gates that reach an output
+    (packed_circuit).  The gate tables are built once here;
     rebuild after changing the model.  With `bank_aware` (default), each fused layer's rows
     are laid out in LDS by bank_aware_positions, so that the row reads of the kernel's
     half-waves hit distinct LDS banks; the counts do not depend on the layout.
@@ -316,31 +318,33 @@ class PackedNetwork:
                 wiring.append((a.cpu().numpy(), b.cpu().numpy(), g.cpu().numpy(), a.device))
             self.device = layers[0].weights.device
             # the pruned circuit of the tail, where it fits, in place of the row tables: 22800
-            # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.47 ms for 4 M samples, all
-            # rows 3.94; the 2 x 16000 tail of a logic-tree network 0.32 ms for 1 M, 0.57
-            self.circuit = None
-            if (bank_aware and self.producer is None and self.rows[0] <= _LDS_INPUT_ROWS
-                    and self.k <= 1024):
-                self.circuit = _Circuit.of([w[:3] for w in wiring], self.rows[0], self.k,
-                                           self.device)
-            if self.circuit is not None:
-                return
+            # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.51 ms for 4 M samples, all
+            # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.33 ms for 1 M, 0.57
+            self.circuit = self.circuit_tabs = None
+            tail = [w[:3] for w in wiring]
+            if bank_aware and self.producer is None and self.k <= 1024:
+                self.circuit = _Circuit.of(tail, self.rows[0], self.k, self.device)
+                if self.circuit is not None:
+                    return
+            if bank_aware and self.producer is not None and not self.prefix and self.k <= 1024:
+                # the layers that write the tail's columns and the tail as one circuit: 29000
+                # two-input gates of the 122600 rows of two convolutions of 9 x 32 x 32 and
+                # 2 x 16000 take 1.27 ms for 1 M samples, producer and tail 2.45.  It stands for
+                # these tables of the layers: with others the call takes the way below
+                tabs = self._producer_tables()
+                self.circuit = _Circuit.of(
+                    [tuple(t.cpu().numpy().astype(np.int64) for t in tab) for tab in tabs] + tail,
+                    self._producer_rows(), self.k, self.device)
+                self.circuit_tabs = tabs
             prev_pos = np.arange(self.rows[0], dtype=np.int64)   # input rows stay in place
             lay = self.layout
             self.col_order = None
             if self.producer is not None:
                 # the producer writes its rows in producer_order; input row r of the tail is
                 # then at position inv[r] of a column
-                tabs = []
-                for m in self.producer:
-                    w = getattr(m, "w", None)
-                    if w is None:
-                        w = m._argmax_slots()
-                    ia, ib = m.packed_tables(w)[:2]
-                    tabs.append((ia.cpu().numpy().astype(np.int64),
-                                 ib.cpu().numpy().astype(np.int64)))
-                m0 = self.producer[0]
-                in_rows = m0.in_dim if type(m0) is LogicLayer else int(np.prod(m0.in_shape))
+                tabs = [tuple(t.cpu().numpy().astype(np.int64) for t in tab[:2])
+                        for tab in self._producer_tables()]
+                in_rows = self._producer_rows()
                 order = producer_order(tabs, in_rows)
                 prev_pos = np.empty(self.rows[0], dtype=np.int64)
                 prev_pos[order] = np.arange(self.rows[0], dtype=np.int64)
@@ -373,6 +377,18 @@ class PackedNetwork:
         self.tables = torch.cat(entries).contiguous()
         self.front_tables = torch.cat(front_entries).contiguous() if front_entries else None
         self._rows_host = (ctypes.c_int64 * len(self.rows))(*self.rows)
+
+    def _producer_tables(self) -> list:
+        """(ia, ib, gate) of the producer's layers as they are now."""
+        tabs = []
+        for m in self.producer:
+            w = getattr(m, "w", None)
+            tabs.append(m.packed_tables(m._argmax_slots() if w is None else w)[:3])
+        return tabs
+
+    def _producer_rows(self) -> int:
+        m = self.producer[0]
+        return m.in_dim if type(m) is LogicLayer else int(np.prod(m.in_shape))
 
     def __call__(self, x) -> torch.Tensor:
         if self.producer is not None:
@@ -420,22 +436,16 @@ class PackedNetwork:
             h = PackBitsTensor.from_packed(x.t, x.pad_len)   # the caller's object stays
         else:
             h = PackBitsTensor.from_packed(x)
-        tabs = []
         with torch.no_grad():
             for m in self.prefix:
                 h = m(h)
-            for m in self.producer:
-                w = getattr(m, "w", None)
-                if w is None:
-                    w = m._argmax_slots()
-                tabs.append(m.packed_tables(w)[:3])
+            tabs = self._producer_tables()
         words, n = h.t, h.num_samples
         _dl._check(words, "x")
         if words.device != self.device:
             raise RuntimeError(f"x is on {words.device}, the network on {self.device}")
         in_rows = words.shape[0]
-        m = self.producer[0]
-        expect = m.in_dim if type(m) is LogicLayer else int(np.prod(m.in_shape))
+        expect = self._producer_rows()
         if in_rows != expect:
             raise RuntimeError(f"the layer before the fused tail gets {in_rows} rows, "
                                f"expects {expect}")
@@ -446,6 +456,16 @@ class PackedNetwork:
         if row_bytes % 4:
             raise RuntimeError("packed rows must be a multiple of 4 bytes")
         cols, in_words = row_bytes // 4, self.layout["in_words"]
+        if self.circuit is not None and all(t is c for tab, old in zip(tabs, self.circuit_tabs)
+                                            for t, c in zip(tab, old)):
+            # straight from the rows the circuit takes 1.55 ms in place of 0.40 + 0.87: its loads
+            # of one word pair per row do not fit L2 for this many rows
+            with torch.cuda.device(words.device):
+                x = torch.empty((cols, in_rows), dtype=torch.int32, device=words.device)
+                timing.timed(f"cl_packed_rows_to_columns[{in_rows}]", lambda: _capi.call(
+                    "cl_packed_rows_to_columns", words.data_ptr(), x.data_ptr(), in_rows,
+                    row_bytes, in_rows, _dl.stream_of(words)))
+            return self.circuit(x, cols, True, in_rows, n)
         colmaj = torch.empty((cols, in_words), dtype=torch.int32, device=words.device)
         counts = torch.empty((n, self.k), dtype=torch.int32, device=words.device)
         stream = _dl.stream_of(words)

@@ -661,22 +661,23 @@ int cl_packed_network_columns(const void* x, int64_t cols, int64_t in_words, int
 
 /* A pruned packed network on LDS pages (packed_circuit.py builds the tables): step by step, the
  * two-input gates left of a frozen network, then the class counts, 64 samples at a time.
- * cl_packed_circuit_limits (host only): the most LDS words per 32-sample plane (pages of 64), gate
- * slots per thread, count steps and input rows.
+ * cl_packed_circuit_limits (host only): the most LDS pages (of 64 signals, 128 words: a word of 32
+ * samples of each signal, then the second), gate slots per thread, count steps and input pages.
  * cl_packed_circuit: x is [rows, cols] 32-bit words, or column-major [cols, in_words] when
- * columns_major; shape (host int64 [8]) = batches of four slots, bit mask of the batches that
- * begin a step, count groups, inverted count groups, input rows staged, k, LDS words, 1 if the
- * counts read inputs.  ent [slots, 1024]: LDS byte addresses of the operands, a | b << 16, with
- * the gate's values for ab = 01, 10, 11 in bits 0, 1 and 16 (00 gives 0); dst [16, max slots /
- * 2]: a wave's page words, two slots to an entry (0xffff: none); in [rows staged]: input row | LDS
- * word << 16; cnt [groups + inverted groups, k, 64, 2]: LDS byte addresses, two to an entry; ones
- * [k]: added to the counts.  counts int32 [nsamples, k].  Page 0 holds zeros; a step reads pages of earlier steps only. */
-int cl_packed_circuit_limits(int64_t* max_words, int64_t* max_slots, int64_t* max_steps,
-                             int64_t* max_inputs);
+ * columns_major; shape (host int64 [7]) = pairs of slots, bit mask of the pairs that
+ * begin a step, count groups, inverted count groups, input pages, k, pages.  ent [slots, 1024]:
+ * LDS words of the operands, a | b << 16; ops [slots / 8, 1024]: a nibble per slot, the gate's
+ * values for ab = 01, 10, 11 in bits 0 to 2 (00 gives 0); dst [16, max slots / 2]: a wave's page
+ * words, two slots to an entry (0xffff: none); in [input pages, 64]: input rows of the signals of
+ * pages 1, 2, ... (0xffff: none); cnt [groups + inverted groups, k, 64, 2]: LDS words, two to an
+ * entry; ones [k]: added to the counts.  counts int32 [nsamples, k].  Page 0 holds zeros; a step
+ * reads pages of earlier steps only; the counts read no page of input. */
+int cl_packed_circuit_limits(int64_t* max_pages, int64_t* max_slots, int64_t* max_steps,
+                             int64_t* max_input_pages);
 int cl_packed_circuit(const void* x, int64_t cols, int64_t columns_major, int64_t in_words,
                       int64_t nsamples, const int64_t* shape, const uint32_t* ent,
-                      const uint32_t* dst, const uint32_t* in, const uint32_t* cnt,
-                      const int32_t* ones, int32_t* counts, void* stream);
+                      const uint32_t* ops, const uint32_t* dst, const uint16_t* in,
+                      const uint32_t* cnt, const int32_t* ones, int32_t* counts, void* stream);
 
 /* Packed rows to columns: y[c * out_words + r] (32-bit words) = word c of row r of x
  * [rows, row_bytes], out_words >= rows; words past the rows of a column are not written. */

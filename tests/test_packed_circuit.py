@@ -42,31 +42,32 @@ def reference_counts(layers, k, x):
 def table_counts(plan, k, x, rng):
     """The kernel's walk over the tables on one column of 64 samples; every step reads the words
     as they were when it began, and the next column's input is staged before the counts."""
-    batches, start, groups, inverted, in_rows, kk, words, hold = plan["shape"]
+    pairs, start, groups, inverted, in_pages, kk, pages = plan["shape"]
     assert kk == k
-    lds = rng.integers(0, 2**63, words).astype(np.uint64)
+    lds = rng.integers(0, 2**63, 128 * pages).astype(np.uint64)   # a signal at its first word
     lds[:64] = 0
-    rows, at = plan["in"][:in_rows] & 0xFFFF, plan["in"][:in_rows] >> 16
+    rows = plan["in"][:64 * in_pages].astype(np.int64)
+    at = 128 * (1 + np.arange(rows.size) // 64) + np.arange(rows.size) % 64
+    rows, at = rows[rows != 0xFFFF], at[rows != 0xFFFF]
     lds[at] = x[rows]
     dst = np.stack([plan["dst"] & 0xFFFF, plan["dst"] >> 16], 2).reshape(16, -1)
-    for b in range(batches):
+    for b in range(pairs):
         if b == 0 or (start >> b) & 1:
             old = lds.copy()
-        for q in range(4 * b, 4 * b + 4):
+        for q in (2 * b, 2 * b + 1):
             for w in range(16):
-                tag = int(dst[w, q])
-                if tag == 0xFFFF:
+                page = int(dst[w, q])
+                if page == 0xFFFF:
                     continue
                 e = plan["ent"][q, 64 * w:64 * w + 64].astype(np.int64)
-                f01, f10, f11 = e & 1, (e >> 1) & 1, (e >> 16) & 1
-                lds[tag:tag + 64] = words_of(f01 << 2 | f10 << 1 | f11, old[(e & 0xFFFC) // 4],
-                                             old[((e >> 16) & 0xFFFC) // 4])
-    if not hold:
-        lds[at] = rng.integers(0, 2**63, in_rows).astype(np.uint64)
+                o = plan["ops"][q // 8, 64 * w:64 * w + 64].astype(np.int64) >> (4 * (q % 8))
+                gate = (o & 1) << 2 | (o & 2) | (o & 4) >> 2
+                lds[page:page + 64] = words_of(gate, old[e & 0xFFFF], old[e >> 16])
+    lds[at] = rng.integers(0, 2**63, rows.size).astype(np.uint64)
     out = np.tile(plan["ones"].astype(np.int64), (64, 1))
     if groups + inverted:
         cnt = plan["cnt"]
-        at = np.stack([cnt & 0xFFFF, cnt >> 16], 4).reshape(groups + inverted, k, 64, 4) // 4
+        at = np.stack([cnt & 0xFFFF, cnt >> 16], 4).reshape(groups + inverted, k, 64, 4)
         v = lds[at]
         v[groups:] = ~v[groups:]
         bits = (v[..., None] >> np.arange(64, dtype=np.uint64)) & np.uint64(1)
@@ -82,7 +83,11 @@ CASES = [
     ([(6, 10)], 2, (0, 15), False),                          # constants only
     ([(50, 700), (700, 640)], 1, (1, 6, 8, 9), False),       # one class, whole pages of a kind
     ([(300, 6000), (6000, 5000)], 20, range(16), False),
-    ([(64, 8000), (8000, 10000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # steps split
+    ([(64, 11000), (11000, 12000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # steps split
+    ([(1500, 2000), (2000, 900)], 3, range(16), False),      # two input pages per wave
+    ([(9000, 12000), (12000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # input rounds
+    ([(6000, 4000), (4000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),    # eight pages
+    ([(3000, 3000), (3000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),    # four pages
 ]
 
 
@@ -98,10 +103,11 @@ def test_tables_give_the_layers_counts(dims, k, gates, strays):
 
 def test_what_does_not_fit_is_refused():
     lim = PC.limits()
-    wide = random_layers([(lim["inputs"], lim["words"] + 64)], 1, (1, 6))
-    assert PC.build(PC.fold(wide, lim["inputs"]), 1) is None                 # LDS words
-    many = random_layers([(lim["inputs"] + 900, 16000)], 2, (1, 6))
-    assert PC.build(PC.fold(many, lim["inputs"] + 900), 1000) is None        # input rows
+    rows = 64 * lim["input_pages"]
+    wide = random_layers([(rows, 64 * lim["pages"])], 1, (1, 6))
+    assert PC.build(PC.fold(wide, rows), 1) is None                          # pages
+    many = random_layers([(2 * rows, 16000)], 2, (1, 6))
+    assert PC.build(PC.fold(many, 2 * rows), 1000) is None                   # input pages
     tall = random_layers([(64, 128 * lim["steps"])], 3, (3, 5))
     assert PC.build(PC.fold(tall, 64), 1) is None                            # entries of a class
 

@@ -409,3 +409,29 @@ def test_tree_front_steps_aside(device):
         model[0].selection[0, 0] = 7 << 8            # row 7 of a 3 x 3 window
     assert net._call_front(x) is None
     assert torch.equal(net(x), model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
+
+
+def test_circuit_follows_the_producer(device):
+    """A circuit of convolutions and tail stands for the tables it was built from: after a change
+    of a convolution's winners the call evaluates the layers as they are."""
+    torch.manual_seed(3)
+    conv = cl.ConvLayer((3, 40, 40), padding=1, c_out=16, ks=3, stride=2)
+    model = torch.nn.Sequential(conv, torch.nn.Flatten(), cl.LogicLayer(conv.out_dim, 3500),
+                                cl.GroupSum(10, 1.0)).to(device)
+    for m in model:
+        if hasattr(m, "freeze"):
+            m.freeze()
+    model.eval()
+    net = cl.PackedNetwork(model)
+    assert net.producer is not None and net.circuit is not None
+    bits = np.random.default_rng(0).integers(0, 2, (200, 4800)).astype(bool)
+    x = cl.PackBitsTensor(torch.as_tensor(bits, device=device), 64)
+
+    def layers():
+        return model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len))
+
+    before = net(x)
+    assert torch.equal(before, layers())
+    conv.w.copy_((conv.w + 1) % conv.num_gates)
+    after = net(x)
+    assert torch.equal(after, layers()) and not torch.equal(before, after)
