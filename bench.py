@@ -617,14 +617,15 @@ def bench_packed_fused(model, in_features: int, log2n: int, passes: int, checksu
     calls = rec.summary()
     fused_call = next((v for k, v in calls.items()
                        if k.startswith(("cl_packed_circuit", "cl_packed_network"))), None)
-    circuit = net.circuit
+    circuit, net_front = net.circuit, getattr(net, "front", None)
     fused_rows = net.rows or []
     prefix = len(net.prefix)
     producer = net.producer is not None and circuit is None
     del xw, counts, net
     torch.cuda.empty_cache()
     out = {"workload": ("the same network and inputs through PackedNetwork: "
-                        + (f"{prefix} modules layer by layer, then " if prefix else "")
+                        + ("the logic-tree blocks on columns, then " if net_front
+                           else f"{prefix} modules layer by layer, then " if prefix else "")
                         + ("the layer before the dense tail written column-major, then "
                            if producer else "")
                         + (f"the {circuit.gates} two-input gates that reach an output of the "
