@@ -14,9 +14,10 @@
 // rows turned to columns 0.40, the circuit 0.87).
 //
 // What bounds it: a workgroup has the CU's LDS to itself, so its phases follow one another.  Of
-// 14000 cycles per column of 64 samples of the first, the gates take 7000 (LDS 80 % busy: 22
-// pages per wave, six words each, 1.07 passes per read), waiting at the levels' barriers 2300,
-// the class counts 4000 (vector work on ten of sixteen waves) and staging 500.
+// 14000 cycles per column of 64 samples of the first, the gates take 7000 (22 pages per wave, six
+// words each, 1.07 passes per read), waiting at the levels' barriers 2300, the class counts 4000
+// (vector work on ten of sixteen waves) and staging 500; over the pass the vector units are 59 %
+// busy and LDS 41 %.
 //
 // A thread holds its gates in registers for the whole launch (slot q: gate lane of the wave's
 // q-th page): the LDS word addresses of both operands, 16 bits each, and the opcode.  A signal is
