@@ -2190,6 +2190,9 @@ extern "C" int cl_dense_backward_rows_any(int dtype, const void* x, const void* 
 // 17 -> 13 us, input and weight gradient 140 + 23 -> 22 us (a launch of 73.7 MB each way of the
 // layer at 3.3 TB/s, bound by the rows in flight as the fp32 kernel), error against 64 bits
 // 3.7e-4 -> 2.2e-4.  Batches of up to 2048 samples, whose rows a wave's registers hold.
+// Rows off 16 bytes (a batch that is no multiple of eight samples, or a buffer that starts
+// between vectors, which the reference-interface kernels take as well) use vectors at any
+// element (vldr).
 namespace {
 using Half = _Float16;
 constexpr int kHalfVec = 8;
@@ -2203,10 +2206,14 @@ int check_half(int64_t batch, int64_t num_gates) {
     return CL_OK;
 }
 
+bool half_tail(int64_t batch, std::initializer_list<const void*> rows) {
+    return batch % kHalfVec != 0 || !all_aligned(rows);
+}
+
 template <typename F>
-void half_units(int64_t batch, F&& f) {
+void half_units(int64_t batch, bool tail, F&& f) {
     auto by_tail = [&](auto uc) {
-        if (batch % kHalfVec) f(uc, std::true_type{});
+        if (tail) f(uc, std::true_type{});
         else f(uc, std::false_type{});
     };
     if (batch <= 64 * kHalfVec) by_tail(std::integral_constant<int, 1>{});
@@ -2228,7 +2235,7 @@ extern "C" int cl_dense_forward_fused_half(const void* x, const float* w, const 
     CL_ARG(x && w && gate_seq && nab && inv_pos && probs && inv_coef && y,
            "null pointer argument");
     CL_ARG(aligned(nab, 16), "nab misaligned");
-    CL_ARG(batch % kHalfVec || all_aligned({x, y}), "x and y must be 16-byte aligned");
+    const bool tail = half_tail(batch, {x, y});
     const Tiling tl = choose_tiling<Half>(batch, out_dim, CL_FWD_LPN, CL_FWD_NPG);
     const unsigned grid = unsigned(tile_grid(tl.map));
     auto launch = [&](auto lc, auto tc) {
@@ -2239,7 +2246,7 @@ extern "C" int cl_dense_forward_fused_half(const void* x, const float* w, const 
             int(num_gates), tl.map, nullptr, 0);
     };
     auto by_tail = [&](auto lc) {
-        if (tl.tail) launch(lc, std::true_type{});
+        if (tail) launch(lc, std::true_type{});
         else launch(lc, std::false_type{});
     };
     if (tl.lpn == 16) by_tail(std::integral_constant<int, 16>{});
@@ -2263,14 +2270,13 @@ extern "C" int cl_dense_backward_rows_half(const void* x, const void* grad_y,
     CL_ARG(!grad_w || (gate_seq && run_ptr && probs), "grad_w needs gate_seq, run_ptr and probs");
     CL_ARG(aligned(slot_rec, 16) && aligned(inv_rec, 16) && aligned(inv_coef, 8),
            "slot_rec / inv_rec must be 16-byte aligned, inv_coef 8-byte aligned");
-    CL_ARG(batch % kHalfVec || all_aligned({x, grad_y, grad_x}),
-           "row buffers must be 16-byte aligned");
+    const bool tail = half_tail(batch, {x, grad_y, grad_x});
     const int64_t avg = 2 * num_runs / in_dim;
     const int S = avg >= CL_BWD_ROWS_S4 ? 4 : avg >= CL_BWD_ROWS_S2 ? 2 : 1;
     const int64_t nblk = ceil_div(ceil_div(in_dim, int64_t(4 / S)), int64_t(kXcds));
     CL_ARG(kXcds * nblk < (int64_t(1) << 31), "too many rows");
     const unsigned grid = unsigned(kXcds * nblk);
-    half_units(batch, [&](auto uc, auto tc) {
+    half_units(batch, tail, [&](auto uc, auto tc) {
         constexpr int U = decltype(uc)::value;
         constexpr bool TAIL = decltype(tc)::value;
         auto launch = [&](auto gwc, auto sc) {
@@ -2308,8 +2314,8 @@ extern "C" int cl_dense_weight_grad_half(const void* x, const void* grad_y,
            "null pointer argument");
     CL_ARG(aligned(run_ab, 8), "run_ab misaligned");
     CL_ARG(in_dim >= 1 && num_runs >= 1, "in_dim and num_runs must be >= 1 when out_dim > 0");
-    CL_ARG(batch % kHalfVec || all_aligned({x, grad_y}), "x and grad_y must be 16-byte aligned");
-    half_units(batch, [&](auto uc, auto tc) {
+    const bool tail = half_tail(batch, {x, grad_y});
+    half_units(batch, tail, [&](auto uc, auto tc) {
         k_wgrad_rows<float, kHalfVec, decltype(uc)::value, true, decltype(tc)::value, Half>
             <<<unsigned(ceil_div(out_dim, int64_t(4))), 256, 0, as_stream(stream)>>>(
                 static_cast<const Half*>(x), static_cast<const Half*>(grad_y), gate_seq, probs,

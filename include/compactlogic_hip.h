@@ -274,8 +274,8 @@ int cl_dense_backward_rows_first_any(int dtype, const void* x, const void* grad_
 
 /* The module path on float16 rows (x, y, grad_y, grad_x) with fp32 logits: the fused forward,
  * the row backward and the weight gradient of single-run neurons of at most 16 slots, batches
- * of 8 to 2048 samples (row buffers 16-byte aligned when batch % 8 == 0).  Sums, softmax and
- * the gradient of the logits are fp32; rows are rounded once on store.  Arguments as for
+ * of 8 to 2048 samples, row buffers at any element (fastest 16-byte aligned with batch % 8 == 0).
+ * Sums, softmax and the gradient of the logits are fp32; rows are rounded once on store.  Arguments as for
  * cl_dense_forward_fused (softmax inside), cl_dense_backward_rows and cl_dense_weight_grad. */
 int cl_dense_forward_fused_half(const void* x, const float* w, const uint8_t* gate_seq,
                                 const int32_t* nab, const int32_t* inv_pos, float* probs,

@@ -591,3 +591,34 @@ def test_half_module_path(device, batch, in_dim, out_dim, g_n):
         np.testing.assert_allclose(np_(got[-1]), ref_gw, **TOL[torch.float32])
         if need_x:
             np.testing.assert_allclose(np_(got[0]).T.astype(np.float64), ref_gx, **small)
+
+
+@pytest.mark.parametrize("off_x,off_gy", [(1, 0), (0, 3), (5, 7)])
+@pytest.mark.parametrize("batch", [8, 64, 1024])
+def test_half_module_path_off_16_bytes(device, batch, off_x, off_gy):
+    """Half rows that start between two 16-byte vectors (views into a flat buffer), at batches
+    that are whole vectors: the results are those of the same rows in buffers of their own, to
+    the one rounding on store (2^-11 relative on either side)."""
+    in_dim, out_dim = 96, 130
+    torch.manual_seed(batch + off_x)
+    layer = cl.LogicLayer(in_dim, out_dim, connections="original").to(device)
+    x = torch.rand((in_dim, batch), device=device).half()
+    gy = torch.randn((out_dim, batch), device=device).half()
+
+    def between(t, off):
+        flat = torch.full((t.numel() + 16,), float("nan"), dtype=t.dtype, device=device)
+        view = flat[off:off + t.numel()].view(t.shape)
+        view.copy_(t)
+        return view
+
+    def passes(x, gy):
+        x = x.t().requires_grad_()
+        y = layer(x)
+        gx, gw = torch.autograd.grad(y, [x, layer.weights], gy.t())
+        return y, gx, gw, torch.autograd.grad(layer(x.detach()), layer.weights, gy.t())[0]
+
+    views = between(x, off_x), between(gy, off_gy)
+    assert [v.data_ptr() % 16 != 0 for v in views] == [off_x > 0, off_gy > 0]
+    for got, ref in zip(passes(*views), passes(x, gy)):
+        np.testing.assert_allclose(np_(got.float()), np_(ref.float()), rtol=2.0 ** -10,
+                                   atol=2.0 ** -24 if got.dtype == torch.float16 else 1e-6)
