@@ -111,6 +111,22 @@ __global__ __launch_bounds__(256) void k_pack_batch(const uint8_t* __restrict__ 
                 for (int k = 0; k < 4; ++k) v[h][4 * c + k] = smp < n ? w[k] : 0u;
             }
         }
+        // a bool byte may hold any non-zero value (a reinterpreted mask): the dot products below
+        // take 0 or 1
+        uint32_t all = 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int k = 0; k < kPackTile / 4; ++k) all |= v[h][k];
+        if (__builtin_expect(__any((all & 0xFEFEFEFEu) != 0u), 0)) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int k = 0; k < kPackTile / 4; ++k) {
+                    const uint32_t b = v[h][k];
+                    v[h][k] = ((((b & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | b) >> 7) & 0x01010101u;
+                }
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
 #pragma unroll

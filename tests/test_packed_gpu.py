@@ -136,3 +136,15 @@ def test_pack_bits_batch(device, bits, n, feats, skew):
     for other in (x.t().contiguous().t(), torch.cat((x, x), 1)[:, :feats]):  # other layouts
         again, pad = dl.packbits_batch(other, bits)
         assert pad == ref_pad and torch.equal(again, packed)
+
+
+@pytest.mark.parametrize("value", [2, 128, 255])
+def test_pack_bits_batch_of_a_reinterpreted_mask(device, value):
+    """A byte mask viewed as bool: every non-zero byte is a set bit, whole 16-byte pieces and the
+    batch's last bytes alike."""
+    rng = np.random.default_rng(value)
+    t = rng.integers(0, 2, (130, 67)).astype(np.uint8)
+    t[:70] *= value                                          # waves of ones and of the value
+    x = torch.as_tensor(t, device=device).view(torch.bool)
+    packed = cl.PackBitsTensor(x, 32).t
+    assert np.array_equal(packed.cpu().numpy().view(np.uint8), P.pack_bits(t.T != 0, 32)[0])
