@@ -210,11 +210,12 @@ def tensor_packbits_cuda(t, bit_count):
 def packbits_batch(t, bit_count):
     """tensor_packbits_cuda(t.T.contiguous(), bit_count) of a bool batch t [n, features],
     reading the batch as it lies (a contiguous batch is not transposed first)."""
-    if t.t().is_contiguous() or not t.is_contiguous():
-        return tensor_packbits_cuda(t.t().contiguous(), bit_count)
-    _check(t, "t")
     n, features = t.shape
-    return _packbits("cl_pack_bits_batch", t, features, n, bit_count)
+    entry = "cl_pack_bits_batch"
+    if n == 1 or features == 1 or not t.is_contiguous():   # a transpose that moves nothing, or must
+        t, entry = t.t().contiguous(), "cl_pack_bits"
+    _check(t, "t")
+    return _packbits(entry, t, features, n, bit_count)
 
 
 def groupbitsum(b, pad_len, k):
