@@ -492,8 +492,11 @@ class LogicLayer(torch.nn.Module):
         self.num_weights = out_dim
         self.is_frozen = False
 
+    _half_refused = None   # the wiring that _half_plan last refused
+
     # caches keyed by weak references, which do not pickle; they rebuild on the next call
-    _weak_caches = ("_argmax_cache", "_plan_key", "_plan", "_packed_key", "_packed_tables")
+    _weak_caches = ("_argmax_cache", "_plan_key", "_plan", "_half_refused", "_packed_key",
+                    "_packed_tables")
 
     def __getstate__(self):
         state = super().__getstate__()
@@ -521,8 +524,8 @@ class LogicLayer(torch.nn.Module):
             if (self.weights.dtype == torch.float32 and self.num_gates <= 16
                     and x.device.type == "cuda"
                     and _HALF_BATCH[0] <= x.shape[1] <= _HALF_BATCH[1]):
-                plan = self.run_plan()
-                if plan.single_run:
+                plan = self._half_plan()
+                if plan is not None:
                     return LogicLayerHalfFunction.apply(x, self.weights, self.gate_sequence,
                                                         plan).transpose(0, 1)
             # other half layers: the reference-interface kernels (half storage, fp32 sums) with
@@ -740,8 +743,7 @@ class LogicLayer(torch.nn.Module):
         trip; the rest of the plan is rebuilt from the new wiring."""
         ind = self.indices
         hit = self._plan_key
-        if (self._plan is None or hit is None or hit[0]() is not ind
-                or hit[1] != (ind._version, ind.device)):
+        if self._plan is None or not self._wiring_is(hit):
             old, order, stale = self._plan, None, 0
             if (old is not None and hit is not None and hit[0]() is ind
                     and old.src_indices is not None and old.src_indices.shape == ind.shape
@@ -753,6 +755,27 @@ class LogicLayer(torch.nn.Module):
             self._plan.stale = stale
             self._plan_key = (weakref.ref(ind), (ind._version, ind.device))
         return self._plan
+
+    def _wiring_is(self, key) -> bool:
+        """Whether key, a weak reference to an indices tensor and its version, names the wiring as
+        it is."""
+        ind = self.indices
+        return key is not None and key[0]() is ind and key[1] == (ind._version, ind.device)
+
+    def _half_plan(self) -> RunPlan | None:
+        """run_plan where the half kernels take the layer, else None: not neurons of several runs
+        or rows out of range (looked for before a plan is laid out that nothing would use, once
+        per wiring), nor under graph capture before the plan is there, which reads back from the
+        device."""
+        ind = self.indices
+        if self._plan is None or not self._wiring_is(self._plan_key):
+            if self._wiring_is(self._half_refused) or torch.cuda.is_current_stream_capturing():
+                return None
+            if not bool(((ind == ind[:, :, :1]) & (ind >= 0) & (ind < self.in_dim)).all()):
+                self._half_refused = (weakref.ref(ind), (ind._version, ind.device))
+                return None
+        plan = self.run_plan()
+        return plan if plan.single_run else None
 
     # -- rewiring, entropy, freezing ----------------------------------------------------------------------------------
 

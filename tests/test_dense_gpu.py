@@ -622,3 +622,51 @@ def test_half_module_path_off_16_bytes(device, batch, off_x, off_gy):
     for got, ref in zip(passes(*views), passes(x, gy)):
         np.testing.assert_allclose(np_(got.float()), np_(ref.float()), rtol=2.0 ** -10,
                                    atol=2.0 ** -24 if got.dtype == torch.float16 else 1e-6)
+
+
+def test_half_layer_plan(device):
+    """A half layer lays no plan out under graph capture (the reference-interface kernels run),
+    for neurons of several runs, or for rows out of range (a NaN row, as those kernels give)."""
+    torch.manual_seed(1)
+    x = torch.rand((96, 64), device=device).half()
+    gy = torch.randn((130, 64), device=device).half()
+
+    def step(layer):
+        xg = x.t().requires_grad_()
+        y = layer(xg)
+        return [y, *torch.autograd.grad(y, [xg, layer.weights], gy.t())]
+
+    eager = cl.LogicLayer(96, 130, connections="original").to(device)
+    ref = step(eager)
+    assert eager._plan is not None
+    fresh = cl.LogicLayer(96, 130, connections="original").to(device)
+    fresh.load_state_dict(eager.state_dict())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):                # loads the kernels
+        step(cl.LogicLayer(96, 130, connections="random").to(device))
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(fresh)
+    assert fresh._plan is None
+    for _ in range(2):
+        for t in got:
+            t.detach().zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        # the softmax rounded to half, and the sixteen products of a logit: 2^-11 each
+        for g, r in zip(got, ref):
+            scale = float(r.detach().abs().max())
+            np.testing.assert_allclose(np_(g.float()), np_(r.float()), rtol=2.0 ** -8,
+                                       atol=2.0 ** -8 * scale)
+    several = cl.LogicLayer(96, 130, connections="random").to(device)
+    step(several)
+    assert several._plan is None
+    with torch.no_grad():
+        eager.indices[0, 5] = 96
+        y = eager(x.t())
+    assert torch.isnan(y[:, 5]).all() and int(torch.isnan(y).any(0).sum()) == 1
+    with torch.no_grad():
+        eager.indices[0, 5] = 95
+        assert not torch.isnan(eager(x.t())).any()
