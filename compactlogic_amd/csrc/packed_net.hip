@@ -121,8 +121,8 @@ __global__ __launch_bounds__(kNetThreads) void k_packed_net(const uint32_t* __re
     __syncthreads();
     const int pairs = 32 * net.k;
     const int P = std::max(1, kNetThreads / pairs);  // threads per (sample, class) pair
-    if (tid < pairs * P) {
-        const int i = tid % pairs, p = tid / pairs;
+    for (int q = tid; q < pairs * P; q += kNetThreads) {  // more than once round past 32 classes
+        const int i = q % pairs, p = q / pairs;
         const int smp = i / net.k, c = i % net.k;
         int32_t n = 0;
         for (int j = p; j < S; j += P) {

@@ -435,3 +435,15 @@ def test_circuit_follows_the_producer(device):
     conv.w.copy_((conv.w + 1) % conv.num_gates)
     after = net(x)
     assert torch.equal(after, layers()) and not torch.equal(before, after)
+
+
+@pytest.mark.parametrize("out_dim,k", [(8500, 50), (17000, 200)])
+def test_counts_of_more_than_32_classes_past_the_register_tables(device, out_dim, k):
+    """A network wider than the register-table kernel takes (a column per workgroup): more
+    (sample, class) pairs than threads."""
+    model = frozen_net([(64, 17000), (17000, out_dim)], k, 4, k, device)
+    rng = np.random.default_rng(k)
+    x = cl.PackBitsTensor(torch.as_tensor(rng.integers(0, 2, (130, 64)).astype(bool),
+                                          device=device), 64)
+    counts = cl.PackedNetwork(model, bank_aware=False)(x)
+    assert np.array_equal(np_(counts), oracle_counts(model, np_(x.t).view(np.uint64), 130))
