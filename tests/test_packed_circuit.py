@@ -91,6 +91,9 @@ CASES = [
 ]
 
 
+TWO = (1, 2, 4, 6, 7, 8, 9, 11, 13, 14)     # opcodes of both operands
+
+
 @pytest.mark.parametrize("dims,k,gates,strays", CASES)
 def test_tables_give_the_layers_counts(dims, k, gates, strays):
     rng = np.random.default_rng(k)
@@ -110,6 +113,20 @@ def test_what_does_not_fit_is_refused():
     assert PC.build(PC.fold(many, 2 * rows), 1000) is None                   # input pages
     tall = random_layers([(64, 128 * lim["steps"])], 3, (3, 5))
     assert PC.build(PC.fold(tall, 64), 1) is None                            # entries of a class
+
+
+def test_what_cannot_fit_is_not_placed(monkeypatch):
+    """A circuit of more gates than slots, or that finds no page at any split, is refused without
+    laying its signals out: the placement takes seconds over all the tries."""
+    def placed(*args):
+        raise AssertionError("a circuit that cannot fit was placed")
+
+    monkeypatch.setattr(PC, "_Banks", placed)
+    for dims in ([784] + [12000] * 6,             # 61000 gates, 49152 slots
+                 [784, 16000, 16000],             # pages: only a schedule shows it
+                 [30000, 20000, 20000]):          # more input pages than the kernel stages
+        layers = random_layers(list(zip(dims[:-1], dims[1:])), 1, TWO)
+        assert PC.build(PC.fold(layers, dims[0]), 10) is None
 
 
 @pytest.mark.gpu
