@@ -243,10 +243,11 @@ class PackedNetwork:
     (packed_circuit).  The gate tables are built once here;
     rebuild after changing the model.  With `bank_aware` (default), each fused layer's rows
     are laid out in LDS by bank_aware_positions, so that the row reads of the kernel's
-    half-waves hit distinct LDS banks; the counts do not depend on the layout.
+    half-waves hit distinct LDS banks; the counts do not depend on the layout.  With `prune`
+    False every row of every layer is evaluated, as where no circuit fits.
     """
 
-    def __init__(self, model, bank_aware: bool = True):
+    def __init__(self, model, bank_aware: bool = True, prune: bool = True):
         mods = list(model)
         if not mods or not isinstance(mods[-1], GroupSum):
             raise ValueError("the network must end with a GroupSum")
@@ -322,11 +323,12 @@ class PackedNetwork:
             # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.33 ms for 1 M, 0.57
             self.circuit = self.circuit_tabs = None
             tail = [w[:3] for w in wiring]
-            if bank_aware and self.producer is None and self.k <= 1024:
+            prune = prune and bank_aware and self.k <= 1024
+            if prune and self.producer is None:
                 self.circuit = _Circuit.of(tail, self.rows[0], self.k, self.device)
                 if self.circuit is not None:
                     return
-            if bank_aware and self.producer is not None and not self.prefix and self.k <= 1024:
+            if prune and self.producer is not None and not self.prefix:
                 # the layers that write the tail's columns and the tail as one circuit: 29000
                 # two-input gates of the 122600 rows of two convolutions of 9 x 32 x 32 and
                 # 2 x 16000 take 1.27 ms for 1 M samples, producer and tail 2.45.  It stands for

@@ -399,8 +399,7 @@ def test_tree_front_every_gate_and_bad_channel(device):
 
 
 def test_tree_front_steps_aside(device):
-    """Taps outside the kernel window, rows of an odd number of words and a non-square input take
-    the layer-by-layer kernels as before."""
+    """Taps outside the kernel window take the layer-by-layer kernels."""
     model = tree_net([(2, 8, 2, 1, 3)], [(32, 100)], 10, 3, device)
     x = cl.PackBitsTensor(torch.rand((100, 2 * 64), device=device) < 0.5, 64)
     net = cl.PackedNetwork(model)
@@ -447,3 +446,111 @@ def test_counts_of_more_than_32_classes_past_the_register_tables(device, out_dim
                                           device=device), 64)
     counts = cl.PackedNetwork(model, bank_aware=False)(x)
     assert np.array_equal(np_(counts), oracle_counts(model, np_(x.t).view(np.uint64), 130))
+
+
+def ran(net, x):
+    """(counts, entry points that ran) of a call."""
+    from compactlogic_amd import timing
+    with timing.record() as rec:
+        counts = net(x)
+    return counts, {name.split("[")[0] for name in rec.summary()}
+
+
+def packed_bits(device, n, feats, seed, bits=64):
+    rng = np.random.default_rng(seed)
+    return cl.PackBitsTensor(torch.as_tensor(rng.integers(0, 2, (n, feats)).astype(bool),
+                                             device=device), bits)
+
+
+@pytest.mark.parametrize("dims,k,g_n,n", [
+    ([(40, 64), (64, 60)], 6, 4, 64),                        # a slot per layer
+    ([(100, 300), (300, 300), (300, 200)], 10, 16, 1000),
+    ([(12, 20)] + [(20, 20)] * 14 + [(20, 30)], 3, 8, 130),  # sixteen layers
+    ([(64, 2000), (2000, 1000)], 8, 16, 4096),               # two slots
+    ([(100, 4000), (4000, 3000)], 40, 4, 500),               # four; more classes than waves
+    ([(3000, 5000), (5000, 2600)], 4, 16, 700),              # eight; 4 inputs per thread
+    ([(784, 9000), (9000, 9000)], 3, 4, 200),                # twelve; 47 rows per lane in a count
+    ([(64, 15000), (15000, 16000)], 2, 4, 300),              # sixteen
+    ([(64, 17000), (17000, 8500)], 10, 4, 200),              # wider than the register tables
+    ([(64, 17000), (17000, 8500)], 50, 4, 130),              # there: more than 32 classes
+    ([(64, 13000)] + [(13000, 13000)] * 5, 100, 4, 70),      # more layers than registers
+])
+@pytest.mark.parametrize("bank_aware", [True, False])
+def test_row_tables_match_oracle_and_layerwise(device, dims, k, g_n, n, bank_aware):
+    """Every row of every layer, in bank-aware places and in row order: the way of the networks
+    that no circuit takes."""
+    model = frozen_net(dims, k, g_n, sum(d[1] for d in dims), device)
+    x = packed_bits(device, n, dims[0][0], n)
+    counts, entries = ran(cl.PackedNetwork(model, bank_aware=bank_aware, prune=False), x)
+    assert entries == {"cl_packed_network"}
+    assert np.array_equal(np_(counts), oracle_counts(model, np_(x.t).view(np.uint64), n))
+    assert torch.equal(counts, model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
+
+
+@pytest.mark.parametrize("in_shape,c_out,convs,widths,k,n,bits", [
+    ((4, 16, 16), 32, 1, [4200, 2100], 10, 1000, 64),    # 8 slots, second layer over the input
+    ((2, 12, 12), 40, 1, [12000, 10000], 10, 333, 64),   # 16 slots, nothing held
+    ((5, 15, 15), 40, 1, [12000, 10000], 20, 100, 32),   # 9000 rows: held slots; odd words
+    ((3, 16, 16), 24, 1, [5000, 4000, 2100], 3, 4096, 64),  # three layers
+    ((3, 16, 16), 32, 2, [4200, 2100], 100, 1000, 64),   # two convs composed; many classes
+    ((4, 16, 16), 24, 3, [3100, 1550], 5, 333, 64),      # conv layer by layer, then a pair
+])
+@pytest.mark.parametrize("bank_aware", [True, False])
+def test_row_tables_on_columns(device, in_shape, c_out, convs, widths, k, n, bits, bank_aware):
+    """The producer written column-major and the tail's rows on those columns."""
+    model = small_conv_net(device, in_shape, c_out, widths, k, seed=n, convs=convs)
+    x = packed_bits(device, n, int(np.prod(in_shape)), n, bits)
+    net = cl.PackedNetwork(model, bank_aware=bank_aware, prune=False)
+    counts, entries = ran(net, x)
+    pair = "cl_eval_packed_indexed" + ("_pair" if convs > 1 else "") + "_columns"
+    assert {pair, "cl_packed_network_columns"} <= entries and "cl_packed_circuit" not in entries
+    words = np_(x.t)
+    if words.dtype != np.int64:                  # 32-bit words: pad to whole 64-bit words
+        words = np.concatenate([words, np.zeros((words.shape[0], words.shape[1] % 2),
+                                                words.dtype)], 1)
+    ref = conv_oracle_counts(model, np.ascontiguousarray(words).view(np.uint64), n)
+    assert np.array_equal(np_(counts), ref)
+
+
+def test_row_tables_of_cfg5(device):
+    cfg = configs.CONV_CONFIGS["cfg5"]
+    model = configs.conv_network(cfg, device=device)
+    configs.freeze_argmax(model)
+    xw = configs.packed_input_words(int(np.prod(cfg.in_shape)), 64, device=device)
+    counts, entries = ran(cl.PackedNetwork(model, prune=False), xw)
+    assert entries == {"cl_eval_packed_indexed_pair_columns", "cl_packed_network_columns"}
+    assert np.array_equal(np_(counts), conv_oracle_counts(model, np_(xw).view(np.uint64), 1 << 12))
+
+
+@pytest.mark.parametrize("side,blocks,dense,k,n", [
+    (32, [(3, 40, 2, 1, 3), (40, 32, 2, 1, 3)], [(128, 300), (300, 200)], 10, 1000),
+    (16, [(2, 17, 1, 1, 3)], [(1088, 1000), (1000, 990)], 90, 333),
+    (32, [(9, 16, 2, 1, 3)], [(1024, 16000), (16000, 16000)], 10, 200),   # held slots
+])
+def test_row_tables_after_the_tree_front(device, side, blocks, dense, k, n):
+    """The tail's rows in the places of the column-major input that the blocks write."""
+    model = tree_net(blocks, dense, k, n, device)
+    x = packed_bits(device, n, blocks[0][0] * side * side, n)
+    counts, entries = ran(cl.PackedNetwork(model, prune=False), x)
+    assert entries == {"cl_packed_rows_to_columns", "cl_tree_columns",
+                       "cl_packed_network_columns"}
+    assert torch.equal(counts, model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
+
+
+def test_tree_front_needs_whole_words_and_a_square(device):
+    """Rows of an odd number of 32-bit words, and a feature count that is no channels * side^2,
+    are left to the layer-by-layer kernels, which refuse them."""
+    from compactlogic_amd.packed_net import tree_columns_layout
+    model = tree_net([(2, 8, 2, 1, 3)], [(32, 100)], 10, 3, device)
+    net = cl.PackedNetwork(model)
+    for n in (96, 65):                           # three words of 32
+        x = packed_bits(device, n, 2 * 64, n, 32)
+        assert x.t.shape[1] == 3 and net._call_front(x) is None
+        with pytest.raises(RuntimeError, match="multiple of 8"):
+            net(x)
+    assert net._call_front(packed_bits(device, 128, 2 * 64, 1, 32)) is not None
+    assert tree_columns_layout(net.front, 2 * 64) is not None
+    assert tree_columns_layout(net.front, 2 * 60) is None and \
+        tree_columns_layout(net.front, 129) is None
+    with pytest.raises(ValueError, match="non-square"):
+        net(packed_bits(device, 64, 2 * 60, 1))
