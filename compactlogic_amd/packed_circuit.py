@@ -162,19 +162,38 @@ def _by_bank(w: np.ndarray) -> np.ndarray:
     return w[np.lexsort((w % 32, rank))]
 
 
-def build(c: dict, k: int) -> dict | None:
-    """Tables for fold's result c with k classes, or None when the circuit does not fit.  A layer
-    split into more steps frees its sources' pages earlier and costs barriers and slots: a layer
-    whose gates find no page is split once more.  Where pages are short they are handed out
-    without the bank placement first, which takes most of the time and changes a page's last reader
-    only where gates of several death steps share a group: what does not fit is found in a tenth of
-    the time (61000 gates of 784 -> 6 x 12000 at once, in place of 1.4 s; 29700 of 784 -> 2 x 16000
-    in 0.11 s, 2.3 s)."""
+def pays(gates: int, groups: int, k: int, row_slots: int) -> bool:
+    """Whether a circuit of this many gates and count groups (of both kinds) is the faster one
+    where evaluating every row takes `row_slots` slots of 1024 gates.  A slot costs either pass
+    the same, so the circuit gains the slots it saves.  It loses in the counts: a wave per class,
+    sixteen classes at a time, adds at least one group of each kind and gathers the bits.
+    Measured for 64 to 1 M samples, circuit / every row, saved slots in brackets: 32 classes of
+    3 x 2400 (4) 0.91 to 1.07 (the last for 64 samples, 0.5 us of the host's); 48 of 4 x 4800
+    (24) 0.77 to 1.01, (13) 0.88 to 1.14, of 2 x 6000 (9) 1.00 to 1.10; 80 of 5 x 12000 (39)
+    0.74 to 0.84, of 4 x 4800 (24) 0.84 to 1.18; 1000 of 2 x 2000 (1) 1.4 to 2.8.  Few classes
+    leave waves idle while one adds many groups: one class of 5 x 12000 (39 slots saved, 28
+    groups) 0.57 to 0.71, of 2 x 12000 (11, 38) 0.86 to 1.10, of 2 x 6000 (4, 24) 0.99 to 1.17;
+    two of 2 x 12000 (11, 20) 0.72 to 0.93, (0, 24) 0.93 to 1.14."""
+    saved, rounds = row_slots - gates // _THREADS, -(-k // _WAVES)
+    return (rounds <= 2 or 10 * rounds - 12 <= saved) and groups * rounds <= 14 + saved
+
+
+def build(c: dict, k: int, row_slots: int | None = None) -> dict | None:
+    """Tables for fold's result c with k classes, or None when the circuit does not fit or (with
+    row_slots) does not pay.  A layer split into more steps frees its sources' pages earlier and
+    costs barriers and slots: a layer whose gates find no page is split once more.  Where pages
+    are short they are handed out without the bank placement first, which takes most of the time
+    and changes a page's last reader only where gates of several death steps share a group: what
+    does not fit is found in a tenth of the time (61000 gates of 784 -> 6 x 12000 at once, in
+    place of 1.1 s; 29700 of 784 -> 2 x 16000 in 0.07 s, 2.2 s)."""
     lim = limits()
     c = _copied_outputs(c)
     groups = _count_groups(c, k)
     least = _least_pages(c, lim)
     if 4 * sum(groups) > lim["steps"] or least > lim["pages"]:
+        return None
+    gates = int(c["live"][c["in_rows"]:].sum())
+    if row_slots is not None and not pays(gates, sum(groups), k, row_slots):
         return None
     for smallest in _MIN_GROUPS:
         for align in _ALIGN:

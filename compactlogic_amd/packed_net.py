@@ -198,9 +198,10 @@ class _Circuit:
     """A tail's pruned circuit (packed_circuit.build) on the device."""
 
     @classmethod
-    def of(cls, layers: list, in_rows: int, k: int, device):
-        """The circuit of layers [(a, b, opcode), ...], or None where it does not fit."""
-        plan = _pc.build(_pc.fold(layers, in_rows), k)
+    def of(cls, layers: list, in_rows: int, k: int, device, row_slots: int | None = None):
+        """The circuit of layers [(a, b, opcode), ...], or None where it does not fit or pay
+        (packed_circuit.build)."""
+        plan = _pc.build(_pc.fold(layers, in_rows), k, row_slots)
         return None if plan is None else cls(plan, in_rows, device)
 
     def __init__(self, plan: dict, in_rows: int, device):
@@ -325,7 +326,8 @@ class PackedNetwork:
             tail = [w[:3] for w in wiring]
             prune = prune and bank_aware and self.k <= 1024
             if prune and self.producer is None:
-                self.circuit = _Circuit.of(tail, self.rows[0], self.k, self.device)
+                self.circuit = _Circuit.of(tail, self.rows[0], self.k, self.device,
+                                           self._row_slots([]))
                 if self.circuit is not None:
                     return
             if prune and self.producer is not None and not self.prefix:
@@ -334,9 +336,9 @@ class PackedNetwork:
                 # 2 x 16000 take 1.27 ms for 1 M samples, producer and tail 2.45.  It stands for
                 # these tables of the layers: with others the call takes the way below
                 tabs = self._producer_tables()
-                self.circuit = _Circuit.of(
-                    [tuple(t.cpu().numpy().astype(np.int64) for t in tab) for tab in tabs] + tail,
-                    self._producer_rows(), self.k, self.device)
+                head = [tuple(t.cpu().numpy().astype(np.int64) for t in tab) for tab in tabs]
+                self.circuit = _Circuit.of(head + tail, self._producer_rows(), self.k, self.device,
+                                           self._row_slots(head))
                 self.circuit_tabs = tabs
             prev_pos = np.arange(self.rows[0], dtype=np.int64)   # input rows stay in place
             lay = self.layout
@@ -379,6 +381,13 @@ class PackedNetwork:
         self.tables = torch.cat(entries).contiguous()
         self.front_tables = torch.cat(front_entries).contiguous() if front_entries else None
         self._rows_host = (ctypes.c_int64 * len(self.rows))(*self.rows)
+
+    def _row_slots(self, head: list) -> int:
+        """Gate slots per thread in which the row tables are evaluated: the kernels give every
+        layer of the tail the slots of its widest (their variants), a producer a row per slot."""
+        widest = -(-max(self.rows[1:]) // 1024)
+        per_layer = next((j for j in (1, 2, 4, 8, 12, 16) if widest <= j), widest)
+        return per_layer * (len(self.rows) - 1) + sum(t[0].size for t in head) // 1024
 
     def _producer_tables(self) -> list:
         """(ia, ib, gate) of the producer's layers as they are now."""

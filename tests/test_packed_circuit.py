@@ -129,6 +129,20 @@ def test_what_cannot_fit_is_not_placed(monkeypatch):
         assert PC.build(PC.fold(layers, dims[0]), 10) is None
 
 
+def test_where_a_circuit_pays():
+    """Few gates saved and many classes, or one class of many rows, take the row tables without
+    a placement; what `pays` allows is laid out."""
+    def built(dims, k, gates, row_slots):
+        layers = random_layers(list(zip(dims[:-1], dims[1:])), k, gates)
+        return PC.build(PC.fold(layers, dims[0]), k, row_slots) is not None
+
+    narrow = [784, 2000, 2000]                    # two slots per layer
+    assert built(narrow, 10, TWO, 4) and not built(narrow, 200, TWO, 4)
+    assert not built(narrow, 50, range(16), 4) and built(narrow, 50, range(16), None)
+    wide = [784, 12000, 12000]
+    assert built(wide, 2, range(16), 24) and not built(wide, 1, range(16), 24)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dims,k,gates,strays", CASES)
 @pytest.mark.parametrize("n", [40000, 33])

@@ -487,6 +487,16 @@ def test_row_tables_match_oracle_and_layerwise(device, dims, k, g_n, n, bank_awa
     assert torch.equal(counts, model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
 
 
+def test_circuit_is_the_default_where_it_pays(device):
+    """Few classes: the circuit; as many as there are rows: every row."""
+    for k, entry in ((10, "cl_packed_circuit"), (1000, "cl_packed_network")):
+        model = frozen_net([(100, 2000), (2000, 2000)], k, 16, k, device)
+        x = packed_bits(device, 500, 100, k)
+        counts, entries = ran(cl.PackedNetwork(model), x)
+        assert entries == {entry}
+        assert np.array_equal(np_(counts), oracle_counts(model, np_(x.t).view(np.uint64), 500))
+
+
 @pytest.mark.parametrize("in_shape,c_out,convs,widths,k,n,bits", [
     ((4, 16, 16), 32, 1, [4200, 2100], 10, 1000, 64),    # 8 slots, second layer over the input
     ((2, 12, 12), 40, 1, [12000, 10000], 10, 333, 64),   # 16 slots, nothing held
