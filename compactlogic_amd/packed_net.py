@@ -322,7 +322,7 @@ class PackedNetwork:
             # the pruned circuit of the tail, where it fits, in place of the row tables: 22800
             # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.51 ms for 4 M samples, all
             # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.33 ms for 1 M, 0.57
-            self.circuit = self.circuit_tabs = None
+            self.circuit = self.circuit_tabs = self._other_tabs = None
             tail = [w[:3] for w in wiring]
             prune = prune and bank_aware and self.k <= 1024
             if prune and self.producer is None:
@@ -388,6 +388,27 @@ class PackedNetwork:
         widest = -(-max(self.rows[1:]) // 1024)
         per_layer = next((j for j in (1, 2, 4, 8, 12, 16) if widest <= j), widest)
         return per_layer * (len(self.rows) - 1) + sum(t[0].size for t in head) // 1024
+
+    def _circuit_holds(self, tabs: list) -> bool:
+        """Whether the circuit stands for these tables of the producer.  Other table tensors than
+        the last ones are compared by content, once (a synchronisation); under graph capture
+        they count as other tables."""
+        def same(old):
+            return old is not None and all(t is c for tab, o in zip(tabs, old)
+                                           for t, c in zip(tab, o))
+
+        if self.circuit is None or same(self._other_tabs):
+            return False
+        if same(self.circuit_tabs):
+            return True
+        if tabs[0][0].is_cuda and torch.cuda.is_current_stream_capturing():
+            return False
+        if all(torch.equal(t, c) for tab, old in zip(tabs, self.circuit_tabs)
+               for t, c in zip(tab, old)):
+            self.circuit_tabs = tabs
+            return True
+        self._other_tabs = tabs
+        return False
 
     def _producer_tables(self) -> list:
         """(ia, ib, gate) of the producer's layers as they are now."""
@@ -467,8 +488,7 @@ class PackedNetwork:
         if row_bytes % 4:
             raise RuntimeError("packed rows must be a multiple of 4 bytes")
         cols, in_words = row_bytes // 4, self.layout["in_words"]
-        if self.circuit is not None and all(t is c for tab, old in zip(tabs, self.circuit_tabs)
-                                            for t, c in zip(tab, old)):
+        if self._circuit_holds(tabs):
             # straight from the rows the circuit takes 1.55 ms in place of 0.40 + 0.87: its loads
             # of one word pair per row do not fit L2 for this many rows
             with torch.cuda.device(words.device):

@@ -564,3 +564,36 @@ def test_tree_front_needs_whole_words_and_a_square(device):
         tree_columns_layout(net.front, 129) is None
     with pytest.raises(ValueError, match="non-square"):
         net(packed_bits(device, 64, 2 * 60, 1))
+
+
+def producer_net(device):
+    torch.manual_seed(3)
+    conv = cl.ConvLayer((3, 40, 40), padding=1, c_out=16, ks=3, stride=2)
+    model = torch.nn.Sequential(conv, torch.nn.Flatten(), cl.LogicLayer(conv.out_dim, 3500),
+                                cl.GroupSum(10, 1.0)).to(device)
+    return model, conv
+
+
+def test_circuit_of_a_producer_goes_by_its_winners(device):
+    """New table tensors of the same winners (a layer frozen again, winners that change and come
+    back) keep the circuit."""
+    model, conv = producer_net(device)
+    for m in (conv, model[2]):
+        m.freeze()
+    model.eval()
+    net = cl.PackedNetwork(model)
+    x = packed_bits(device, 200, 4800, 0)
+
+    def check(entry):
+        counts, entries = ran(net, x)
+        assert entry in entries and len(entries) == 2
+        assert torch.equal(counts, model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
+
+    check("cl_packed_circuit")
+    conv.freeze()                                # a new winner tensor
+    check("cl_packed_circuit")
+    conv.w.copy_((conv.w + 1) % conv.num_gates)
+    check("cl_packed_network_columns")
+    check("cl_packed_network_columns")
+    conv.freeze()
+    check("cl_packed_circuit")
