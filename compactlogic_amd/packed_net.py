@@ -17,6 +17,7 @@ import torch
 
 from . import _capi
 from . import timing
+from . import convlogic_hip as _cl
 from . import difflogic_hip as _dl
 from . import packed_circuit as _pc
 from .layers import ConvLayer, GroupSum, LogicLayer, PackBitsTensor
@@ -194,6 +195,10 @@ def _column_words(layout: dict, layer: int, pos: np.ndarray) -> np.ndarray:
     return layout["base"][layer] + pos
 
 
+def _on_host(tabs: list) -> list:
+    return [tuple(t.cpu().numpy().astype(np.int64) for t in tab) for tab in tabs]
+
+
 class _Circuit:
     """A tail's pruned circuit (packed_circuit.build) on the device."""
 
@@ -303,9 +308,8 @@ class PackedNetwork:
             self.front_layout = columns_layout(self.rows) if self.front else None
             if self.front_layout is None:
                 self.front = None
-        entries, front_entries = [], []
+        wiring = []
         with torch.no_grad():
-            wiring = []
             for m in layers:
                 w = getattr(m, "w", None)
                 if w is None:
@@ -317,70 +321,44 @@ class PackedNetwork:
                 if int(a.min()) < 0 or int(a.max()) >= m.in_dim or int(b.min()) < 0 or \
                         int(b.max()) >= m.in_dim:
                     raise IndexError("connection indices out of range")
-                wiring.append((a.cpu().numpy(), b.cpu().numpy(), g.cpu().numpy(), a.device))
-            self.device = layers[0].weights.device
-            # the pruned circuit of the tail, where it fits, in place of the row tables: 22800
-            # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.51 ms for 4 M samples, all
-            # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.33 ms for 1 M, 0.57
-            self.circuit = self.circuit_tabs = self._other_tabs = None
-            tail = [w[:3] for w in wiring]
-            prune = prune and bank_aware and self.k <= 1024
-            if prune and self.producer is None:
-                self.circuit = _Circuit.of(tail, self.rows[0], self.k, self.device,
-                                           self._row_slots([]))
-                if self.circuit is not None:
-                    return
-            if prune and self.producer is not None and not self.prefix:
-                # the layers that write the tail's columns and the tail as one circuit: 29000
-                # two-input gates of the 122600 rows of two convolutions of 9 x 32 x 32 and
-                # 2 x 16000 take 1.27 ms for 1 M samples, producer and tail 2.45.  It stands for
-                # these tables of the layers: with others the call takes the way below
-                tabs = self._producer_tables()
-                head = [tuple(t.cpu().numpy().astype(np.int64) for t in tab) for tab in tabs]
-                self.circuit = _Circuit.of(head + tail, self._producer_rows(), self.k, self.device,
-                                           self._row_slots(head))
-                self.circuit_tabs = tabs
-            prev_pos = np.arange(self.rows[0], dtype=np.int64)   # input rows stay in place
-            lay = self.layout
-            self.col_order = None
-            if self.producer is not None:
-                # the producer writes its rows in producer_order; input row r of the tail is
-                # then at position inv[r] of a column
-                tabs = [tuple(t.cpu().numpy().astype(np.int64) for t in tab[:2])
-                        for tab in self._producer_tables()]
-                in_rows = self._producer_rows()
-                order = producer_order(tabs, in_rows)
-                prev_pos = np.empty(self.rows[0], dtype=np.int64)
-                prev_pos[order] = np.arange(self.rows[0], dtype=np.int64)
-                self.col_order = torch.as_tensor(order, device=layers[0].weights.device)
-            front_word = np.arange(self.rows[0], dtype=np.int64)  # LDS words in the columns
-            for i, (m, (a, b, g, dev)) in enumerate(zip(layers, wiring)):
-                pa, pb = prev_pos[a], prev_pos[b]
-                if not bank_aware:
-                    pos = np.arange(m.out_dim, dtype=np.int64)
-                elif i + 1 < len(layers):
-                    na, nb = wiring[i + 1][:2]
-                    pos = bank_aware_positions(pa, pb, m.out_dim,
-                                               np.bincount(na, minlength=m.out_dim),
-                                               np.bincount(nb, minlength=m.out_dim))
-                else:  # class groups stay contiguous
-                    pos = bank_aware_positions_grouped(pa, pb, m.out_dim, m.out_dim // self.k)
-                ent = np.empty(m.out_dim, dtype=np.int64)
-                if lay is None:
-                    ent[pos] = (pa * 4) | ((pb * 4) << 20) | (g << 40)   # LDS byte offsets
-                    prev_pos = pos
-                else:
-                    ent[pos] = pa | (pb << 16) | (g << 32)               # LDS words
-                    prev_pos = _column_words(lay, i, pos)
-                entries.append(torch.as_tensor(ent, device=dev))
-                if self.front is not None:   # the same positions for the column-major input
-                    ent = np.empty(m.out_dim, dtype=np.int64)
-                    ent[pos] = front_word[a] | (front_word[b] << 16) | (g << 32)
-                    front_word = _column_words(self.front_layout, i, pos)
-                    front_entries.append(torch.as_tensor(ent, device=dev))
-        self.tables = torch.cat(entries).contiguous()
-        self.front_tables = torch.cat(front_entries).contiguous() if front_entries else None
+                wiring.append((a.cpu().numpy(), b.cpu().numpy(), g.cpu().numpy()))
+        self.device = layers[0].weights.device
         self._rows_host = (ctypes.c_int64 * len(self.rows))(*self.rows)
+        self._wiring, self._bank_aware = wiring, bank_aware
+        self._columns = None          # the producer's tables the row tables are laid out for
+        self.tables = self.front_tables = self.col_order = None
+        # the pruned circuit of the tail, where it fits, in place of the row tables: 22800
+        # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.51 ms for 4 M samples, all
+        # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.33 ms for 1 M, 0.57
+        self.circuit = self.circuit_tabs = self._other_tabs = None
+        if prune and bank_aware and self.k <= 1024 and not (self.producer and self.prefix):
+            # with a producer, the layers that write the tail's columns and the tail as one
+            # circuit: 29000 two-input gates of the 122600 rows of two convolutions of
+            # 9 x 32 x 32 and 2 x 16000 take 1.27 ms for 1 M samples, producer and tail 2.45.
+            # It stands for these tables of the layers: with others the call takes the row tables
+            head = []
+            if self.producer is not None:
+                self.circuit_tabs = self._producer_tables()
+                head = self._columns = _on_host(self.circuit_tabs)
+            self.circuit = _Circuit.of(head + wiring,
+                                       self._producer_rows() if head else self.rows[0], self.k,
+                                       self.device, self._row_slots(head))
+        if self.producer is not None and self._columns is None:
+            self._columns = _on_host(self._producer_tables())
+        if self.circuit is None:
+            self._lay_out_rows()
+        elif self.producer is None:
+            self._wiring = None        # the tail does not change: its circuit is all it needs
+        elif any(getattr(m, "w", None) is None for m in self.producer):
+            # layers that may still train: under graph capture their winners are never known to
+            # be the circuit's, and the row tables cannot be laid out there
+            self._lay_out_rows()
+        else:
+            # the row tables, which take as long to lay out as the circuit, wait for the first
+            # call with other tables; should that be under capture, the layers run one by one
+            self._tail = [tuple(torch.as_tensor(t, dtype=d, device=self.device)
+                                for t, d in zip(w, (torch.int32, torch.int32, torch.uint8)))
+                          for w in wiring]
 
     def _row_slots(self, head: list) -> int:
         """Gate slots per thread in which the row tables are evaluated: the kernels give every
@@ -388,6 +366,49 @@ class PackedNetwork:
         widest = -(-max(self.rows[1:]) // 1024)
         per_layer = next((j for j in (1, 2, 4, 8, 12, 16) if widest <= j), widest)
         return per_layer * (len(self.rows) - 1) + sum(t[0].size for t in head) // 1024
+
+    def _lay_out_rows(self) -> None:
+        """The row tables: `tables` of the tail's layers (`front_tables`: for the column-major
+        input that logic-tree blocks write) and `col_order`, the producer's row order."""
+        prev_pos = np.arange(self.rows[0], dtype=np.int64)   # input rows stay in place
+        lay, col_order = self.layout, None
+        if self.producer is not None:
+            # the producer writes its rows in producer_order; input row r of the tail is
+            # then at position inv[r] of a column
+            order = producer_order([t[:2] for t in self._columns], self._producer_rows())
+            prev_pos = np.empty(self.rows[0], dtype=np.int64)
+            prev_pos[order] = np.arange(self.rows[0], dtype=np.int64)
+            col_order = torch.as_tensor(order, device=self.device)
+        front_word = np.arange(self.rows[0], dtype=np.int64)  # LDS words in the columns
+        entries, front_entries = [], []
+        for i, (a, b, g) in enumerate(self._wiring):
+            pa, pb = prev_pos[a], prev_pos[b]
+            if not self._bank_aware:
+                pos = np.arange(a.size, dtype=np.int64)
+            elif i + 1 < len(self._wiring):
+                na, nb = self._wiring[i + 1][:2]
+                pos = bank_aware_positions(pa, pb, a.size, np.bincount(na, minlength=a.size),
+                                           np.bincount(nb, minlength=a.size))
+            else:  # class groups stay contiguous
+                pos = bank_aware_positions_grouped(pa, pb, a.size, a.size // self.k)
+            ent = np.empty(a.size, dtype=np.int64)
+            if lay is None:
+                ent[pos] = (pa * 4) | ((pb * 4) << 20) | (g << 40)   # LDS byte offsets
+                prev_pos = pos
+            else:
+                ent[pos] = pa | (pb << 16) | (g << 32)               # LDS words
+                prev_pos = _column_words(lay, i, pos)
+            entries.append(ent)
+            if self.front is not None:   # the same positions for the column-major input
+                ent = np.empty(a.size, dtype=np.int64)
+                ent[pos] = front_word[a] | (front_word[b] << 16) | (g << 32)
+                front_word = _column_words(self.front_layout, i, pos)
+                front_entries.append(ent)
+        if front_entries:
+            self.front_tables = torch.as_tensor(np.concatenate(front_entries), device=self.device)
+        self.col_order = col_order
+        # last: a call in another thread that finds it has the others
+        self.tables = torch.as_tensor(np.concatenate(entries), device=self.device)
 
     def _circuit_holds(self, tabs: list) -> bool:
         """Whether the circuit stands for these tables of the producer.  Other table tensors than
@@ -409,6 +430,14 @@ class PackedNetwork:
             return True
         self._other_tabs = tabs
         return False
+
+    def _layer_by_layer(self, words, tabs: list, n: int) -> torch.Tensor:
+        """The producer and the tail one layer at a time (under graph capture, where the row
+        tables cannot be laid out)."""
+        for ia, ib, gate in [*tabs, *self._tail]:
+            words = _cl.eval_packed_indexed(words, ia, ib, gate)
+        pad = words.shape[1] * words.element_size() * 8 - n
+        return _dl.groupbitsum(words, pad, self.k)
 
     def _producer_tables(self) -> list:
         """(ia, ib, gate) of the producer's layers as they are now."""
@@ -497,6 +526,10 @@ class PackedNetwork:
                     "cl_packed_rows_to_columns", words.data_ptr(), x.data_ptr(), in_rows,
                     row_bytes, in_rows, _dl.stream_of(words)))
             return self.circuit(x, cols, True, in_rows, n)
+        if self.tables is None:
+            if torch.cuda.is_current_stream_capturing():
+                return self._layer_by_layer(words, tabs, n)
+            self._lay_out_rows()
         colmaj = torch.empty((cols, in_words), dtype=torch.int32, device=words.device)
         counts = torch.empty((n, self.k), dtype=torch.int32, device=words.device)
         stream = _dl.stream_of(words)

@@ -576,7 +576,7 @@ def producer_net(device):
 
 def test_circuit_of_a_producer_goes_by_its_winners(device):
     """New table tensors of the same winners (a layer frozen again, winners that change and come
-    back) keep the circuit."""
+    back) keep the circuit; the row tables are laid out for the first winners that differ."""
     model, conv = producer_net(device)
     for m in (conv, model[2]):
         m.freeze()
@@ -592,8 +592,42 @@ def test_circuit_of_a_producer_goes_by_its_winners(device):
     check("cl_packed_circuit")
     conv.freeze()                                # a new winner tensor
     check("cl_packed_circuit")
+    assert net.tables is None
     conv.w.copy_((conv.w + 1) % conv.num_gates)
     check("cl_packed_network_columns")
     check("cl_packed_network_columns")
     conv.freeze()
     check("cl_packed_circuit")
+
+
+@pytest.mark.parametrize("frozen", [True, False])
+def test_changed_producer_under_capture(device, frozen):
+    """A graph captured right after a convolution's winners changed, with no call before it,
+    counts with the new winners; layers that may still train are read at each replay."""
+    model, conv = producer_net(device)
+    model[2].freeze()
+    if frozen:
+        conv.freeze()
+    model.eval()
+    net = cl.PackedNetwork(model)
+    assert net.circuit is not None and (net.tables is None) == frozen
+    x = packed_bits(device, 200, 4800, 1)
+    warm = cl.PackedNetwork(model, prune=False)(x)         # loads the kernels
+    with torch.no_grad():
+        if frozen:
+            conv.w.copy_((conv.w + 1) % conv.num_gates)
+        else:
+            conv.weights.copy_(conv.weights.roll(1, 1))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        counts = net(x)
+    for _ in range(2):
+        counts.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len))
+        assert torch.equal(counts, ref) and not torch.equal(counts, warm)
+        if not frozen:
+            with torch.no_grad():
+                conv.weights.copy_(conv.weights.roll(1, 1))
