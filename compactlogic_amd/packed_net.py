@@ -210,21 +210,30 @@ class _Circuit:
         return None if plan is None else cls(plan, in_rows, device)
 
     def __init__(self, plan: dict, in_rows: int, device):
-        def dev(name):
-            a = plan[name]
-            return torch.as_tensor(a.view(np.int16 if a.itemsize == 2 else np.int32), device=device)
-
         self.in_rows, self.k = in_rows, plan["shape"][5]
         self.shape = (ctypes.c_int64 * 7)(*plan["shape"])
-        self.tabs = [dev(name) for name in ("ent", "ops", "dst", "in", "cnt", "ones")]
+        # one buffer, its tables at 16-byte offsets; their addresses are computed when it moves
+        # (a copy of this object has a buffer of its own), not per call
+        parts, self.offsets, end = [], [], 0
+        self.base, self.at = None, ()
+        for name in ("ent", "ops", "dst", "in", "cnt", "ones"):
+            raw = plan[name].reshape(-1).view(np.uint8)
+            parts.append(np.pad(raw, (0, -raw.size % 16)))
+            self.offsets.append(end)
+            end += parts[-1].size
+        self.tables = torch.as_tensor(np.concatenate(parts).view(np.int32), device=device)
         self.gates = plan["gates"]
 
     def __call__(self, words, cols: int, columns_major: bool, in_words: int, n: int):
         counts = torch.empty((n, self.k), dtype=torch.int32, device=words.device)
+        base = self.tables.data_ptr()
+        if base != self.base:
+            self.at, self.base = tuple(base + o for o in self.offsets), base
+        at = self.at
         with torch.cuda.device(words.device):
             timing.timed(f"cl_packed_circuit[{self.in_rows}]", lambda: _capi.call(
                 "cl_packed_circuit", words.data_ptr(), cols, int(columns_major), in_words, n,
-                self.shape, *[t.data_ptr() for t in self.tabs], counts.data_ptr(),
+                self.shape, *at, counts.data_ptr(),
                 _dl.stream_of(words)))
         return counts
 

@@ -631,3 +631,15 @@ def test_changed_producer_under_capture(device, frozen):
         if not frozen:
             with torch.no_grad():
                 conv.weights.copy_(conv.weights.roll(1, 1))
+
+
+def test_copied_network_has_tables_of_its_own(device):
+    import copy
+    model = frozen_net([(64, 400), (400, 300)], 10, 8, 2, device)
+    x = packed_bits(device, 300, 64, 2)
+    net = cl.PackedNetwork(model)
+    ref = net(x)
+    other = copy.deepcopy(net)
+    net.circuit.tables.zero_()
+    assert other.circuit.tables.data_ptr() != net.circuit.tables.data_ptr()
+    assert torch.equal(other(x), ref)
