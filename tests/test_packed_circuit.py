@@ -84,14 +84,47 @@ CASES = [
     ([(50, 700), (700, 640)], 1, (1, 6, 8, 9), False),       # one class, whole pages of a kind
     ([(300, 6000), (6000, 5000)], 20, range(16), False),
     ([(64, 11000), (11000, 12000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # steps split
-    ([(1500, 2000), (2000, 900)], 3, range(16), False),      # two input pages per wave
-    ([(9000, 12000), (12000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # input rounds
+    ([(1500, 2000), (2000, 900)], 3, range(16), False),      # an input page per wave
+    ([(9000, 12000), (12000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),  # eight pages
     ([(6000, 4000), (4000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),    # eight pages
     ([(3000, 3000), (3000, 3000)], 10, (1, 2, 4, 6, 7, 8, 9, 11, 13, 14), False),    # four pages
 ]
 
 
 TWO = (1, 2, 4, 6, 7, 8, 9, 11, 13, 14)     # opcodes of both operands
+
+
+def chain(first, width, layers):
+    return [(first, width)] + [(width, width)] * (layers - 1)
+
+
+# The kernel's variants: the gate slots and count planes it is compiled for, input pages per wave
+# (16: two rounds of eight), and whether a step begins inside a block of four slots.
+VARIANTS = [
+    (chain(100, 2000, 19), 10, range(16), 40, 5, 1, True),
+    (chain(100, 1100, 21), 10, TWO, 48, 5, 1, True),
+    (chain(64, 3500, 10), 1, TWO, 40, 9, 1, False),
+    ([(9200, 12000)] + chain(12000, 6000, 5), 2, TWO, 48, 9, 8, False),
+    ([(1800, 3000), (3000, 2000)], 10, TWO, 32, 5, 2, False),
+    ([(9400, 11000)], 1, TWO, 32, 9, 16, False),
+    ([(9400, 11000)], 100, TWO, 32, 5, 16, False),
+    (chain(8400, 4500, 8), 10, TWO, 40, 5, 8, False),
+    (chain(600, 6500, 6), 50, TWO, 48, 5, 1, False),
+]
+
+
+@pytest.mark.parametrize("dims,k,gates,slots,planes,inputs,inside", VARIANTS)
+def test_tables_of_every_kernel_variant(dims, k, gates, slots, planes, inputs, inside):
+    rng = np.random.default_rng(k)
+    layers = random_layers(dims, k, gates)
+    plan = PC.build(PC.fold(layers, dims[0][0]), k)
+    pairs, start, groups, inverted, in_pages = plan["shape"][:5]
+    assert next(v for v in (32, 40, 48) if 2 * pairs <= v) == slots
+    assert (5 if 4 * (groups + inverted) < 32 else 9) == planes
+    assert next(v for v in (1, 2, 4, 8, 16) if in_pages <= 16 * v) == inputs
+    assert any((start >> b) & 1 for b in range(1, pairs, 2)) == inside
+    x = rng.integers(0, 2**63, dims[0][0]).astype(np.uint64)
+    assert np.array_equal(table_counts(plan, k, x, rng), reference_counts(layers, k, x))
 
 
 @pytest.mark.parametrize("dims,k,gates,strays", CASES)
@@ -144,7 +177,8 @@ def test_where_a_circuit_pays():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dims,k,gates,strays", CASES)
+@pytest.mark.parametrize("dims,k,gates,strays",
+                         CASES + [(*v[:3], False) for v in VARIANTS])
 @pytest.mark.parametrize("n", [40000, 33])
 def test_circuit_kernel(device, dims, k, gates, strays, n):
     """Several columns per workgroup (256 workgroups take 16384 samples at a time), row-major and
