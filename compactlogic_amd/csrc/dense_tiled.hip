@@ -1830,7 +1830,12 @@ extern "C" int cl_dense_weight_grad(int dtype, const void* x, const void* grad_y
         auto* ab = reinterpret_cast<const int2*>(run_ab);
         auto* gw = static_cast<T*>(grad_w);
         const bool wide = batch >= W;
-        if (wide && num_gates <= 64 && batch <= 64 * W * 8) {
+        // A small batch off the vector leaves a wave per neuron few lanes to work with; 16 lanes
+        // are enough for it where there are neurons for them (8000 neurons of 16 runs, rows /
+        // full: fp64 66 / 54 us at 7 samples, 77 / 69 at 33, 106 / 112 at 95, fp32 47 / 43 at 5;
+        // 800 neurons: 37 / 45 at 7).
+        const bool few = !v && batch < 64 && out_dim >= 4096;
+        if (wide && !few && num_gates <= 64 && batch <= 64 * W * 8) {
             const unsigned wgrid = unsigned(ceil_div(out_dim, int64_t(4)));
             auto launch = [&](auto uc, auto tc) {
                 constexpr int U = decltype(uc)::value;

@@ -247,9 +247,15 @@ _ROWS_SHARED_FROM = 6
 
 
 def _row_backward_fits(plan: RunPlan, x: torch.Tensor) -> bool:
-    """Whether cl_dense_backward_rows takes this layer at this batch (x: [in_dim, batch])."""
+    """Whether cl_dense_backward_rows takes this layer at this batch (x: [in_dim, batch]).  A
+    batch below 64 samples that is no multiple of the 16-byte vector takes the tiled kernels
+    unless its inputs have many uses: a wave per row then has few of its lanes at work (forward
+    and backward of 12011 neurons on 10007 inputs, 2.4 uses each, rows / tiled: 21 / 16.5 us at
+    5 samples, 22 / 20 at 47, 25 / 26 at 95; of 8000 on 784, 20 uses, 19 / 24 at 5)."""
     wide = 16 // x.element_size()
     batch = x.shape[1]
+    if batch % wide and batch < 64 and plan.num_runs < 4 * plan.in_dim:
+        return False
     return plan.single_run and plan.num_gates <= 64 and wide <= batch <= 64 * wide * 8
 
 
