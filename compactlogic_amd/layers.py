@@ -459,6 +459,11 @@ class GroupSumFunction(torch.autograd.Function):
 _PACKED_CHAIN_MAX_DEGREE = 8
 
 
+def _wiring_is(key, ind: torch.Tensor) -> bool:
+    """Whether key, a weak reference to an indices tensor and its version, names ind as it is."""
+    return key is not None and key[0]() is ind and key[1] == (ind._version, ind.device)
+
+
 class LogicLayer(torch.nn.Module):
     """Differentiable logic-gate layer (compactlogic/compactlogic.py:10-130).
 
@@ -527,13 +532,10 @@ class LogicLayer(torch.nn.Module):
         x = to_rows(x)
         assert x.shape[0] == self.in_dim, (x.shape, self.in_dim)
         if x.dtype == torch.float16:
-            if (self.weights.dtype == torch.float32 and self.num_gates <= 16
-                    and x.device.type == "cuda"
-                    and _HALF_BATCH[0] <= x.shape[1] <= _HALF_BATCH[1]):
-                plan = self._half_plan()
-                if plan is not None:
-                    return LogicLayerHalfFunction.apply(x, self.weights, self.gate_sequence,
-                                                        plan).transpose(0, 1)
+            plan = self._half_plan(x)
+            if plan is not None:
+                return LogicLayerHalfFunction.apply(x, self.weights, self.gate_sequence,
+                                                    plan).transpose(0, 1)
             # other half layers: the reference-interface kernels (half storage, fp32 sums) with
             # the reference's own argument list and inverse index
             w = torch.nn.functional.softmax(self.weights, dim=-1).to(x.dtype)
@@ -626,7 +628,7 @@ class LogicLayer(torch.nn.Module):
         on it stay cached across eval calls (one device comparison, which synchronises; under
         graph capture the fresh winners are returned as they are)."""
         src = self.weights
-        w = self._fresh_slots()
+        w = src.argmax(-1).to(dtype=torch.uint8)
         if src.device.type == "cuda" and torch.cuda.is_current_stream_capturing():
             return w
         prev = getattr(self, "_argmax_cache", None)
@@ -749,7 +751,7 @@ class LogicLayer(torch.nn.Module):
         trip; the rest of the plan is rebuilt from the new wiring."""
         ind = self.indices
         hit = self._plan_key
-        if self._plan is None or not self._wiring_is(hit):
+        if self._plan is None or not _wiring_is(hit, ind):
             old, order, stale = self._plan, None, 0
             if (old is not None and hit is not None and hit[0]() is ind
                     and old.src_indices is not None and old.src_indices.shape == ind.shape
@@ -762,25 +764,25 @@ class LogicLayer(torch.nn.Module):
             self._plan_key = (weakref.ref(ind), (ind._version, ind.device))
         return self._plan
 
-    def _wiring_is(self, key) -> bool:
-        """Whether key, a weak reference to an indices tensor and its version, names the wiring as
-        it is."""
+    def _half_plan(self, x: torch.Tensor) -> RunPlan | None:
+        """run_plan where the half kernels take the layer at x's batch, else None: not neurons of
+        several runs or rows out of range (looked for before a plan is laid out that nothing
+        would use, once per wiring), nor under graph capture before the plan is there, which reads
+        back from the device."""
         ind = self.indices
-        return key is not None and key[0]() is ind and key[1] == (ind._version, ind.device)
-
-    def _half_plan(self) -> RunPlan | None:
-        """run_plan where the half kernels take the layer, else None: not neurons of several runs
-        or rows out of range (looked for before a plan is laid out that nothing would use, once
-        per wiring), nor under graph capture before the plan is there, which reads back from the
-        device."""
-        ind = self.indices
-        if self._plan is None or not self._wiring_is(self._plan_key):
-            if self._wiring_is(self._half_refused) or torch.cuda.is_current_stream_capturing():
+        if _wiring_is(self._half_refused, ind):
+            return None
+        if not (self.weights.dtype == torch.float32 and self.num_gates <= 16
+                and x.device.type == "cuda" and _HALF_BATCH[0] <= x.shape[1] <= _HALF_BATCH[1]):
+            return None
+        plan = self._plan
+        if plan is None or not _wiring_is(self._plan_key, ind):
+            if torch.cuda.is_current_stream_capturing():
                 return None
             if not bool(((ind == ind[:, :, :1]) & (ind >= 0) & (ind < self.in_dim)).all()):
                 self._half_refused = (weakref.ref(ind), (ind._version, ind.device))
                 return None
-        plan = self.run_plan()
+            plan = self.run_plan()
         return plan if plan.single_run else None
 
     # -- rewiring, entropy, freezing ----------------------------------------------------------------------------------
