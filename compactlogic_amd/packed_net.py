@@ -174,6 +174,30 @@ def tree_columns_layout(blocks: list, rows: int) -> tuple | None:
     return (arr, out[2].value, out[3].value) if out[0].value else None
 
 
+def tree_columns_from(blocks: list, rows: int) -> float:
+    """Number of 32-sample columns from which cl_tree_columns is faster than the blocks one by one
+    on a square input of `rows` features (inf: never).  The column pass turns every input row to
+    columns and gives a wave a channel of 64 positions (`whole` rows, channels rounded up to the
+    sixteen waves; `others`: a lane per position); the row kernels read the rows that are tapped
+    and cost a launch per block.  Measured, columns / rows, for 64 K and 1 M samples: 9 x 32 x 32
+    -> 256 -> 512 channels 0.75, 0.59; -> 64 -> 128 1.37, 0.86; -> 16 2.2, 1.09; 2 x 16 x 16 -> 64
+    0.94, 0.54, -> 17 1.29, 1.11; 64 x 16 x 16 -> 64 2.6, 1.36; 3 x 12 x 12 -> 10 -> 12 (36 and 9
+    positions) 1.08, 1.97."""
+    h = w = math.isqrt(rows // blocks[0].in_channels)
+    whole = waves = others = 0
+    for m in blocks:
+        (sh, sw), (ph, pw), (kh, kw) = m.stride, m.padding, m.kernel
+        h, w = ((h + 2 * ph - kh) // sh + 1) // 2, ((w + 2 * pw - kw) // sw + 1) // 2
+        if h * w % 64:
+            others += m.out_channels * h * w
+        else:
+            whole += m.out_channels * h * w
+            waves += -(-m.out_channels // 16) * 16 * h * w
+    if 5 * whole < 2 * waves + others + rows + 1200:
+        return math.inf
+    return 2 ** 24 / whole
+
+
 def _table_layer_before(body: list, j: int):
     """Index of the module before body[j] (Flatten modules pass a PackBitsTensor through
     unchanged) when it is a packed layer from index tables (ConvLayer or LogicLayer); else
@@ -311,7 +335,7 @@ class PackedNetwork:
             raise ValueError(f"in_dim ({self.rows[-1]}) has to be divisible by k ({self.k}) "
                              "but it is not")
         # complete logic-tree blocks before the tail: they can hand it columns
-        self.front = self.front_layout = None
+        self.front = self.front_layout = self._front_from = None
         if self.producer is None:
             self.front = _tree_front(self.prefix)
             self.front_layout = columns_layout(self.rows) if self.front else None
@@ -464,7 +488,8 @@ class PackedNetwork:
         if self.producer is not None:
             return self._call_columns(x)
         if self.prefix:
-            counts = self._call_front(x) if self.rows is not None and self.front else None
+            counts = (self._call_front(x) if self.rows is not None and self.front
+                      and self._front_pays(x) else None)
             if counts is not None:
                 return counts
             if isinstance(x, PackBitsTensor):
@@ -562,6 +587,13 @@ class PackedNetwork:
                 self.tables.data_ptr(), self._rows_host, len(self.rows) - 1, self.k,
                 counts.data_ptr(), stream))
         return counts
+
+    def _front_pays(self, x) -> bool:
+        words = x.t if isinstance(x, PackBitsTensor) else x
+        rows = words.shape[0]
+        if self._front_from is None or self._front_from[0] != rows:
+            self._front_from = (rows, tree_columns_from(self.front, rows))
+        return words.shape[-1] * words.element_size() >= 4 * self._front_from[1]
 
     def _call_front(self, x):
         """The logic-tree blocks and the tail on columns: the packed rows turned to columns, all

@@ -11,6 +11,14 @@ from oracle import packed as P
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def columns_at_every_size(request, monkeypatch):
+    """The column pass of logic-tree blocks at any size and shape, for the tests of its kernels."""
+    if "tree_front" in request.node.name:
+        from compactlogic_amd import packed_net
+        monkeypatch.setattr(packed_net, "tree_columns_from", lambda blocks, rows: 0)
+
+
 def np_(t):
     return t.detach().cpu().numpy()
 
@@ -643,3 +651,24 @@ def test_copied_network_has_tables_of_its_own(device):
     net.circuit.tables.zero_()
     assert other.circuit.tables.data_ptr() != net.circuit.tables.data_ptr()
     assert torch.equal(other(x), ref)
+
+
+def test_tree_blocks_take_columns_where_they_pay(device):
+    """The rule of the column pass: from 32 K samples for many channels of 64 positions, never for
+    channels that leave waves idle, positions off 64 or an input of far more rows than outputs;
+    both ways count alike on either side of it."""
+    from compactlogic_amd.packed_net import tree_columns_from
+    wide = tree_net([(9, 256, 2, 1, 3), (256, 512, 2, 1, 3)], [(2048, 2000)], 10, 1, device)
+    blocks = [wide[0], wide[1]]
+    assert tree_columns_from(blocks, 9 * 1024) == 1024
+    for block, rows in (((2, 17, 1, 1, 3), 512), ((3, 10, 1, 1, 3), 432), ((64, 64, 1, 1, 3), 16384)):
+        layer = cl.ConvLogicLayer(block[0], block[1], stride=1, padding=1, kernel=3, complete=True,
+                                  num_chn=0)
+        assert tree_columns_from([layer], rows) == float("inf")
+    net = cl.PackedNetwork(wide)
+    for n, columns in ((32768 - 64, False), (32768, True)):
+        gen = torch.Generator(device=device).manual_seed(n)
+        words = torch.randint(-2**62, 2**62, (9 * 1024, n // 64), generator=gen, device=device)
+        counts, entries = ran(net, words)
+        assert ("cl_tree_columns" in entries) == columns
+        assert torch.equal(counts, wide(cl.PackBitsTensor.from_packed(words)))
