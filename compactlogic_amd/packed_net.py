@@ -223,6 +223,14 @@ def _on_host(tabs: list) -> list:
     return [tuple(t.cpu().numpy().astype(np.int64) for t in tab) for tab in tabs]
 
 
+# Bytes of a producer's packed input up to which its circuit reads the rows as they lie, a word
+# pair per row: they stay in the Infinity Cache then, and a launch is saved (two convolutions of
+# 9 x 32 x 32 and 2 x 16000, rows / columns: 23 / 32 us for 64 samples, 120 / 133 for 128 K, 274 /
+# 284 for 256 K (302 MB), 974 / 875 for 768 K; one of 3 x 40 x 40 and 3500 194 / 219 for 512 K
+# (315 MB), 376 / 345 for 768 K).
+_ROWS_IN_CACHE = 256 << 20
+
+
 class _Circuit:
     """A tail's pruned circuit (packed_circuit.build) on the device."""
 
@@ -254,7 +262,7 @@ class _Circuit:
         if base != self.base:
             self.at, self.base = tuple(base + o for o in self.offsets), base
         at = self.at
-        with torch.cuda.device(words.device):
+        with _dl.on_device_of(words):
             timing.timed(f"cl_packed_circuit[{self.in_rows}]", lambda: _capi.call(
                 "cl_packed_circuit", words.data_ptr(), cols, int(columns_major), in_words, n,
                 self.shape, *at, counts.data_ptr(),
@@ -451,7 +459,7 @@ class PackedNetwork:
             return old is not None and all(t is c for tab, o in zip(tabs, old)
                                            for t, c in zip(tab, o))
 
-        if self.circuit is None or same(self._other_tabs):
+        if same(self._other_tabs):
             return False
         if same(self.circuit_tabs):
             return True
@@ -551,10 +559,10 @@ class PackedNetwork:
         if row_bytes % 4:
             raise RuntimeError("packed rows must be a multiple of 4 bytes")
         cols, in_words = row_bytes // 4, self.layout["in_words"]
-        if self._circuit_holds(tabs):
-            # straight from the rows the circuit takes 1.55 ms in place of 0.40 + 0.87: its loads
-            # of one word pair per row do not fit L2 for this many rows
-            with torch.cuda.device(words.device):
+        if self.circuit is not None and self._circuit_holds(tabs):
+            if row_bytes * in_rows <= _ROWS_IN_CACHE:
+                return self.circuit(words, cols, False, 0, n)
+            with _dl.on_device_of(words):
                 x = torch.empty((cols, in_rows), dtype=torch.int32, device=words.device)
                 timing.timed(f"cl_packed_rows_to_columns[{in_rows}]", lambda: _capi.call(
                     "cl_packed_rows_to_columns", words.data_ptr(), x.data_ptr(), in_rows,
@@ -619,7 +627,7 @@ class PackedNetwork:
         def ints(*shape):
             return torch.empty(shape, dtype=torch.int32, device=dev)
 
-        with torch.no_grad(), torch.cuda.device(dev):
+        with torch.no_grad(), _dl.on_device_of(words):
             gates = [m.weights.argmax(-1).to(torch.uint8).contiguous() for m in blocks]
             taps = [m.selection.to(torch.int32).contiguous() for m in blocks]
             ptrs = [(ctypes.c_void_p * len(blocks))(*[t.data_ptr() for t in ts])

@@ -582,9 +582,10 @@ def producer_net(device):
     return model, conv
 
 
-def test_circuit_of_a_producer_goes_by_its_winners(device):
+def test_circuit_of_a_producer_goes_by_its_winners(device, monkeypatch):
     """New table tensors of the same winners (a layer frozen again, winners that change and come
     back) keep the circuit; the row tables are laid out for the first winners that differ."""
+    from compactlogic_amd import packed_net
     model, conv = producer_net(device)
     for m in (conv, model[2]):
         m.freeze()
@@ -592,18 +593,21 @@ def test_circuit_of_a_producer_goes_by_its_winners(device):
     net = cl.PackedNetwork(model)
     x = packed_bits(device, 200, 4800, 0)
 
-    def check(entry):
+    def check(entry, calls=1):
         counts, entries = ran(net, x)
-        assert entry in entries and len(entries) == 2
+        assert entry in entries and len(entries) == calls
         assert torch.equal(counts, model(cl.PackBitsTensor.from_packed(x.t.clone(), x.pad_len)))
 
+    monkeypatch.setattr(packed_net, "_ROWS_IN_CACHE", 0)   # rows turned to columns first
+    check("cl_packed_circuit", 2)
+    monkeypatch.undo()
     check("cl_packed_circuit")
     conv.freeze()                                # a new winner tensor
     check("cl_packed_circuit")
     assert net.tables is None
     conv.w.copy_((conv.w + 1) % conv.num_gates)
-    check("cl_packed_network_columns")
-    check("cl_packed_network_columns")
+    check("cl_packed_network_columns", 2)
+    check("cl_packed_network_columns", 2)
     conv.freeze()
     check("cl_packed_circuit")
 
