@@ -7,7 +7,7 @@
 // the 8 XCDs of an MI355X, so workgroup w runs on XCD w % 8, and chunk c is given only to
 // workgroups w with w % 8 == c % 8.  The chunk's band of the activation matrix (rows x CS
 // samples, 1.5-3 MB at 12000 rows) then stays in that XCD's 4 MB L2 and the second gather of
-// a row hits L2.  Outputs use ordinary write-back stores (see vst_stream).
+// a row hits L2.  Outputs use ordinary write-back stores (see vstr).
 //
 // Per layer and training step:
 //   k_prep        logits -> softmax probabilities and the collapsed coefficients K of every
@@ -61,6 +61,9 @@ __device__ __forceinline__ V vldr(const T* p) {
     }
 }
 
+// Store of an output row segment.  Regular (write-back) stores measure faster inside a
+// training step than non-temporal ones: the next kernel reads these rows right away and then
+// finds them in the Infinity Cache.
 template <bool TAIL, typename T, typename V>
 __device__ __forceinline__ void vstr(T* p, V v) {
     if constexpr (TAIL) {
@@ -131,13 +134,6 @@ constexpr int kFwdRunBatch = 4;
 // Inverse-index entries the tiled backward gathers together (connections='random': 0.367 ->
 // 0.314 ms per 12000 -> 12000 layer against one at a time; two 0.342, eight 0.339 ms).
 constexpr int kBwdEntryBatch = 4;
-// Store of an output row segment.  Regular (write-back) stores measure faster inside a
-// training step than non-temporal ones: the next kernel reads these rows right away and then
-// finds them in the Infinity Cache.
-template <typename V>
-__device__ __forceinline__ void vst_stream(void* p, V v) {
-    *reinterpret_cast<V*>(p) = v;
-}
 
 template <typename T, int N>
 __device__ __forceinline__ T hsum(typename VT<T, N>::type v) {

@@ -10,8 +10,9 @@
 // 64 gates and reused once the last level that reads one of them is done: a whole network of two
 // convolutions of 9 x 32 x 32 and 2 x 16000 (122600 rows, 28000 to 31000 gates left) fits.
 // Against all rows: 784 -> 6 x 12000 for 4 M samples 1.51 ms (3.96), the tail 2 x 16000 of a
-// logic-tree network for 1 M 0.33 (0.57), the convolutions and their tail for 1 M 1.27 (2.45:
-// rows turned to columns 0.40, the circuit 0.87).
+// logic-tree network for 1 M 0.38 (0.66), the convolutions and their tail for 1 M 1.29 (2.47):
+// rows turned to columns 0.48, the circuit 0.80.  Where it is not the faster one:
+// packed_circuit.pays.
 //
 // What bounds it: a workgroup has the CU's LDS to itself, so its phases follow one another.  Of
 // 14000 cycles per column of 64 samples of the first, the gates take 7000 (22 pages per wave, six

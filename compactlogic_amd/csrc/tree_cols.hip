@@ -10,7 +10,8 @@
 // address arithmetic nor the gate choice costs vector instructions per word.  Between the
 // blocks nothing leaves LDS.  9x32x32 -> 256 -> 512 channels at 2^20 samples: 1.75 ms and 0.48 ms
 // for the rows turned to columns, where the row-major blocks took 3.30 + 0.60 ms and 0.40 ms for
-// widening their input rows.  Bound by the instructions a SIMD issues, vector and scalar ones
+// widening their input rows (shapes and sizes where they stay the faster ones: tree_columns_from
+// in packed_net.py).  Bound by the instructions a SIMD issues, vector and scalar ones
 // together (a column takes 32000 cycles: 22000 in the first block, 6500 in the second, the
 // rest staging and barriers): every tap and gate evaluated 2.72 ms, only live ones with a
 // branch per tap 2.13, a branch per subtree and unshared table words 1.75.

@@ -285,10 +285,10 @@ class PackedNetwork:
     (cl_packed_network_columns).  When no tail qualifies every module runs layer by
     layer and the counts come from the group popcount.  A fused tail whose prefix is complete
     ConvLogicLayers alone takes its input column-major from them (cl_tree_columns: all blocks on
-    one column in LDS).  Where it fits, a fused tail, or the whole network when the layers that
-    write its columns come first, is reduced to the two-input gates that reach an output
-    (packed_circuit).  The gate tables are built once here;
-    rebuild after changing the model.  With `bank_aware` (default), each fused layer's rows
+    one column in LDS) where that is the faster way (tree_columns_from).  Where it fits and pays
+    (packed_circuit.build), a fused tail, or the whole network when the layers that
+    write its columns come first, is reduced to the two-input gates that reach an output.
+    The gate tables are built once here; rebuild after changing the model.  With `bank_aware` (default), each fused layer's rows
     are laid out in LDS by bank_aware_positions, so that the row reads of the kernel's
     half-waves hit distinct LDS banks; the counts do not depend on the layout.  With `prune`
     False every row of every layer is evaluated, as where no circuit fits.
@@ -370,12 +370,12 @@ class PackedNetwork:
         self.tables = self.front_tables = self.col_order = None
         # the pruned circuit of the tail, where it fits, in place of the row tables: 22800
         # two-input gates of the 72000 of 784 -> 6 x 12000 take 1.51 ms for 4 M samples, all
-        # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.33 ms for 1 M, 0.57
+        # rows 3.96; the 2 x 16000 tail of a logic-tree network 0.38 ms for 1 M, 0.66
         self.circuit = self.circuit_tabs = self._other_tabs = None
         if prune and bank_aware and self.k <= 1024 and not (self.producer and self.prefix):
             # with a producer, the layers that write the tail's columns and the tail as one
             # circuit: 29000 two-input gates of the 122600 rows of two convolutions of
-            # 9 x 32 x 32 and 2 x 16000 take 1.27 ms for 1 M samples, producer and tail 2.45.
+            # 9 x 32 x 32 and 2 x 16000 take 1.29 ms for 1 M samples, producer and tail 2.47.
             # It stands for these tables of the layers: with others the call takes the row tables
             head = []
             if self.producer is not None:
