@@ -599,9 +599,10 @@ class PackedNetwork:
     def _front_pays(self, x) -> bool:
         words = x.t if isinstance(x, PackBitsTensor) else x
         rows = words.shape[0]
-        if self._front_from is None or self._front_from[0] != rows:
-            self._front_from = (rows, tree_columns_from(self.front, rows))
-        return words.shape[-1] * words.element_size() >= 4 * self._front_from[1]
+        known = self._front_from
+        if known is None or known[0] != rows:
+            known = self._front_from = (rows, tree_columns_from(self.front, rows))
+        return words.shape[-1] * words.element_size() >= 4 * known[1]
 
     def _call_front(self, x):
         """The logic-tree blocks and the tail on columns: the packed rows turned to columns, all
