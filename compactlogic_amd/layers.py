@@ -196,7 +196,8 @@ class LogicLayerRunsFunction(torch.autograd.Function):
         stream = _dl.stream_of(x)
         batch = x.shape[1]
         with torch.cuda.device(x.device):
-            if need_x and LogicLayerRunsFunction.row_backward and _row_backward_fits(plan, x):
+            if (need_x and LogicLayerRunsFunction.row_backward and _row_backward_fits(plan, x)
+                    and _row_backward_pays(plan, x)):
                 timing.timed(f"cl_dense_backward_rows[{plan.in_dim}->{plan.out_dim}]", lambda: _capi.call(
                     _rows_entry("cl_dense_backward_rows", x), code, x.data_ptr(), grad_y.data_ptr(),
                     plan.slot_rec.data_ptr(), plan.inv_rec.data_ptr(), inv_coef.data_ptr(),
@@ -247,16 +248,23 @@ _ROWS_SHARED_FROM = 6
 
 
 def _row_backward_fits(plan: RunPlan, x: torch.Tensor) -> bool:
-    """Whether cl_dense_backward_rows takes this layer at this batch (x: [in_dim, batch]).  A
-    batch below 64 samples that is no multiple of the 16-byte vector takes the tiled kernels
-    unless its inputs have many uses: a wave per row then has few of its lanes at work (forward
-    and backward of 12011 neurons on 10007 inputs, 2.4 uses each, rows / tiled: 21 / 16.5 us at
-    5 samples, 22 / 20 at 47, 25 / 26 at 95; of 8000 on 784, 20 uses, 19 / 24 at 5)."""
+    """Whether cl_dense_backward_rows takes this layer at this batch (x: [in_dim, batch])."""
     wide = 16 // x.element_size()
     batch = x.shape[1]
-    if batch % wide and batch < 64 and plan.num_runs < 4 * plan.in_dim:
-        return False
     return plan.single_run and plan.num_gates <= 64 and wide <= batch <= 64 * wide * 8
+
+
+def _row_backward_pays(plan: RunPlan, x: torch.Tensor) -> bool:
+    """Where the row backward fits, whether it is the faster one for a layer alone.  A batch
+    below 64 samples that is no multiple of the 16-byte vector takes the tiled kernels for many
+    inputs of few uses: a wave per row then has few of its lanes at work (forward and backward of
+    12011 neurons on 10007 inputs, 2.4 uses each, rows / tiled: 21 / 16.5 us at 5 samples, 22 / 20
+    at 47, 25 / 26 at 95; of 5000 on 3000 18 / 18; of 8000 on 784, 20 uses, 19 / 24).  A step that
+    also finishes the first layer (LogicLayerFirstPairFunction) saves two launches and stays with
+    the rows: 216 / 222 us for 784 -> 3 x 12000 at 5 samples, 429 / 439 at 33."""
+    batch = x.shape[1]
+    few = batch < 64 and batch % (16 // x.element_size()) != 0
+    return not (few and plan.in_dim >= 4096 and plan.num_runs < 4 * plan.in_dim)
 
 
 def _rows_entry(name: str, x: torch.Tensor) -> str:
@@ -587,7 +595,8 @@ class LogicLayer(torch.nn.Module):
                 or first.weights.dtype != x.dtype or x.data_ptr() != x_in.data_ptr()
                 or plan1.out_dim != plan.in_dim or not _row_backward_fits(plan, x)):
             return None
-        # bitwise equal to the unpaired steps only where those take one wave per input row
+        # bitwise equal to the unpaired steps only where those take one wave per input row (a few
+        # samples off the vector width: to rounding, see _row_backward_pays)
         if 2 * plan.num_runs // max(plan.in_dim, 1) >= _ROWS_SHARED_FROM:
             return None
         return LogicLayerFirstPairFunction.apply(
