@@ -521,8 +521,8 @@ class PackedNetwork:
             raise RuntimeError(f"x must be [{self.rows[0]}, words], got {tuple(words.shape)}")
         row_bytes = words.shape[1] * words.element_size()
         if self.circuit is not None:
-            if row_bytes % 4:
-                raise RuntimeError("packed rows must be a multiple of 4 bytes")
+            if row_bytes % 4:     # as cl_packed_network does
+                raise _capi.CompactLogicError("packed rows must be a multiple of 4 bytes")
             return self.circuit(words, row_bytes // 4, False, 0, n)
         counts = torch.empty((n, self.k), dtype=torch.int32, device=words.device)
         with torch.cuda.device(words.device):

@@ -676,3 +676,13 @@ def test_tree_blocks_take_columns_where_they_pay(device):
         counts, entries = ran(net, words)
         assert ("cl_tree_columns" in entries) == columns
         assert torch.equal(counts, wide(cl.PackBitsTensor.from_packed(words)))
+
+
+@pytest.mark.parametrize("prune", [True, False])
+def test_rows_off_four_bytes_are_refused_alike(device, prune):
+    """Rows that are no whole 32-bit words raise the library's error on either way."""
+    from compactlogic_amd._capi import CompactLogicError
+    net = cl.PackedNetwork(frozen_net([(64, 400), (400, 300)], 10, 8, 4, device), prune=prune)
+    for bits in (8, 16):
+        with pytest.raises(CompactLogicError, match="multiple of 4 bytes"):
+            net(packed_bits(device, 9, 64, bits, bits))
